@@ -1395,10 +1395,12 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
             const int px0 = f2i_sat(floorf(xo)) - R - 2, py0 = f2i_sat(floorf(yo)) - R - 2;
             const int px0a = px0 & ~3, poff = px0 - px0a;
             unsigned tmax = 0u, tmin = 255u;
-            if (px0 >= 0 && py0 >= 0 && px0 + pside <= G.w && py0 + pside <= G.h) {
-                // interior: aligned words [px0a, round_up(px0 + pside, 4)) of each row,
-                // which end within the row's pitch
-                const int nw = (poff + pside + 3) >> 2;  // <= kPS / 4
+            const int nw = (poff + pside + 3) >> 2;  // aligned words of a row, <= kPS / 4
+            if (px0 >= 0 && py0 >= 0 && px0a + 4 * nw <= G.w && py0 + pside <= G.h) {
+                // interior: the words [px0a, round_up(px0 + pside, 4)) of each row lie
+                // within the image. (Ending within the row's pitch is not enough: the
+                // bytes past the width are whatever the memory held, and the texel
+                // range below would take them in.)
                 const int tot = nw * pside;              // <= 18 * 68 < 5 * 256
                 const float inv_nw = 1.0f / (float)nw;
                 const uint8_t* rowp = G.g + (size_t)py0 * G.pitch + px0a;
