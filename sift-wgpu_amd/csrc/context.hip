@@ -629,16 +629,12 @@ int Context::run(const Batch& B, RunOutputs* outs) {
             in_pitch[i] = (int)(im.stride ? im.stride : im.width);
         } else {
             in_pitch[i] = (int)round_up(im.width, 64);
-            in_off[i] = C.take((size_t)in_pitch[i] * im.height);
+            // a grey host input goes with the staged inputs below
+            if (fmt != SIFT_PIXEL_GRAY8) in_off[i] = C.take((size_t)in_pitch[i] * im.height);
         }
         if (fmt != SIFT_PIXEL_GRAY8) {
-            const int bpp = pixel_bytes(fmt);
-            if (B.device_input) {
-                color_pitch[i] = (int)(im.stride ? im.stride : (size_t)im.width * bpp);
-            } else {
-                color_pitch[i] = (int)round_up((size_t)im.width * bpp, 64);
-                color_off[i] = C.take((size_t)color_pitch[i] * im.height);
-            }
+            const size_t row = (size_t)im.width * pixel_bytes(fmt);
+            color_pitch[i] = (int)(!B.device_input ? host_pitch(row) : im.stride ? im.stride : row);
         }
         lev_off[i].resize(shapes[i].size());
         dog_off[i].resize(shapes[i].size());
@@ -729,6 +725,18 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     const size_t wide_off = C.take((size_t)cap * 4);  // keypoints for the wide-window descriptor
     const size_t mid_off = C.take((size_t)cap * 4);   // keypoints for the R <= 31 descriptor
     const size_t descu8_off = B.desc_u8 ? C.take((size_t)kcap * 128) : 0;
+    // The host inputs lie next to the job blob, which follows them: the pinned
+    // staging holds the same bytes in the same places, rows at the device pitch,
+    // so any run of them is one linear copy. (A 2D copy between unequal pitches
+    // that are not multiples of 4 bytes goes row by row, about 8 us each: 12.4 ms
+    // of a 14.1 ms call on two 1023 x 767 images, 0.5 of 0.7 ms on one of 97 x 61.)
+    const size_t in_base = round_up(C.off, 256);
+    if (!B.device_input)
+        for (int i = 0; i < n; i++) {
+            const bool grey = B.format(i) == SIFT_PIXEL_GRAY8;
+            const size_t pitch = (size_t)(grey ? in_pitch[i] : color_pitch[i]);
+            (grey ? in_off : color_off)[i] = C.take(pitch * B.images[i].height);
+        }
 
     // --- job blob (host), uploaded to the end of the arena ---
     std::vector<char> blob;
@@ -1061,41 +1069,43 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         HIP_TRY(hipMemcpyAsync(A + blob_dev_off, ext_pinned + tb, blob.size(), hipMemcpyHostToDevice, st));
     }
     // staging: inputs + blob in pinned memory (inputs that are pinned already
-    // are copied from where they are)
-    size_t in_bytes = 0;
-    if (!B.device_input && !B.host_pinned)
-        for (int i = 0; i < n; i++)
-            in_bytes += (size_t)B.images[i].width * B.images[i].height * pixel_bytes(B.format(i));
+    // are copied from where they are), and the summary on its way back
+    unsigned* h_summary = nullptr;
     if (!B.ext) {
-        rc = ensure_pinned(round_up(blob.size(), 256) + in_bytes + 256);
+        const bool staged = !B.device_input && !B.host_pinned;
+        const size_t blob_at = staged ? blob_dev_off - in_base : 0;
+        const size_t summary_at = round_up(blob_at + blob.size(), 256);
+        rc = ensure_pinned(summary_at + (size_t)(n + 3) * sizeof(unsigned));
         if (rc) return rc;
+        h_summary = (unsigned*)(pinned + summary_at);
         HIP_TRY(hipStreamSynchronize(stream));  // pinned staging is reused across calls
-        memcpy(pinned, blob.data(), blob.size());
-        HIP_TRY(hipMemcpyAsync(A + blob_dev_off, pinned, blob.size(), hipMemcpyHostToDevice, st));
-    }
-    if (!B.device_input) {
-        size_t po = round_up(blob.size(), 256);
-        for (int i = 0; i < n; i++) {
+        char* const dst = A + (blob_dev_off - blob_at);
+        size_t sent = 0;  // bytes of the staging whose copy is queued
+        for (int i = 0; i < n && !B.device_input; i++) {
             const sift_image_t& im = B.images[i];
-            const uint32_t fmt = B.format(i);
-            const size_t row = (size_t)im.width * pixel_bytes(fmt);
+            const bool grey = B.format(i) == SIFT_PIXEL_GRAY8;
+            const size_t row = (size_t)im.width * pixel_bytes(B.format(i));
             const size_t stride = im.stride ? im.stride : row;
-            const uint8_t* src = im.data;
-            size_t spitch = stride;
-            if (!B.host_pinned) {
-                for (uint32_t y = 0; y < im.height; y++)
-                    memcpy(pinned + po + (size_t)y * row, im.data + (size_t)y * stride, row);
-                src = (const uint8_t*)pinned + po;
-                spitch = row;
-                po += row * im.height;
+            const size_t pitch = (size_t)(grey ? in_pitch[i] : color_pitch[i]);
+            const size_t off = grey ? in_off[i] : color_off[i];
+            if (!staged) {
+                if (stride != pitch) return fail(SIFT_ERR_DEVICE, "internal: pinned rows not at the device pitch");
+                HIP_TRY(hipMemcpyAsync(A + off, im.data, pitch * im.height, hipMemcpyHostToDevice, st));
+                continue;
             }
-            if (fmt == SIFT_PIXEL_GRAY8)
-                HIP_TRY(hipMemcpy2DAsync(A + in_off[i], in_pitch[i], src, spitch, row, im.height,
-                                         hipMemcpyHostToDevice, st));
-            else
-                HIP_TRY(hipMemcpy2DAsync(A + color_off[i], color_pitch[i], src, spitch, row,
-                                         im.height, hipMemcpyHostToDevice, st));
+            char* const to = pinned + (off - in_base);
+            for (uint32_t y = 0; y < im.height; y++) {
+                memcpy(to + y * pitch, im.data + y * stride, row);
+                // long inputs go in pieces, each on its way while the next is staged
+                const size_t end = off - in_base + (y + 1) * pitch;
+                if (end - sent >= kStageChunk) {
+                    HIP_TRY(hipMemcpyAsync(dst + sent, pinned + sent, end - sent, hipMemcpyHostToDevice, st));
+                    sent = end;
+                }
+            }
         }
+        memcpy(pinned + blob_at, blob.data(), blob.size());
+        HIP_TRY(hipMemcpyAsync(dst + sent, pinned + sent, blob_at + blob.size() - sent, hipMemcpyHostToDevice, st));
     }
     char* D = A + blob_dev_off;
     const OctaveDesc* d_oct = (const OctaveDesc*)(D + oct_blob);
@@ -1290,6 +1300,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         outs->d_desc = d_desc;
         outs->d_desc_u8 = B.desc_u8 ? (uint8_t*)AP(descu8_off) : nullptr;
         outs->d_summary = d_sum;
+        outs->h_summary = h_summary;
         outs->d_cand = d_cand;
         outs->d_cand_resp = (float*)AP(candresp_off);
         outs->d_ref = d_ref;
@@ -1444,31 +1455,31 @@ int check_color_image(const sift_color_image_t* im) {
     return SIFT_OK;
 }
 
-// Copies the results out: f32 descriptors into `out`, or (when out8 is set)
-// the u8 descriptors into `out8`, with the keypoint convention kp_conv.
-// The f32 results of a finished run (summary `sum` read): each image's
-// keypoints and descriptors in one pinned pool block, [keypoints | pad |
-// descriptors], filled by two DMAs from the device; images the pool cannot
-// serve get malloc'd buffers, filled through the context's pinned staging.
-int collect_pinned(sh::Context* C, int n, sh::RunOutputs& R, const std::vector<unsigned>& sum,
-                   sift_result_t* out) {
-    constexpr size_t kDesc = 128 * sizeof(float);
+// The results of a finished run (summary `sum` read), f32 or u8 descriptors by
+// the type of `out`: each image's keypoints and descriptors in one pinned pool
+// block, [keypoints | pad | descriptors], filled by two DMAs from the device;
+// images the pool cannot serve get malloc'd buffers, filled through the
+// context's pinned staging.
+template <typename Result, typename Desc>
+int collect_pinned(sh::Context* C, int n, sh::RunOutputs& R, const unsigned* sum, const Desc* d_desc,
+                   Result* out) {
+    constexpr size_t kDesc = 128 * sizeof(Desc);
     std::vector<char> pooled(n, 0);
     size_t staged = 0;  // keypoints of the images that go through the staging
     for (int i = 0; i < n; i++) {
         const size_t c = sum[3 + i] - sum[2 + i];
-        out[i] = sift_result_t{nullptr, nullptr, c};
+        out[i] = Result{nullptr, nullptr, c};
         if (!c) continue;
         const size_t kb = (c * sizeof(sift_keypoint_t) + 255) / 256 * 256;
         char* blk = (char*)sh::pinned_alloc(kb + c * kDesc);
         if (blk) {
             out[i].keypoints = (sift_keypoint_t*)blk;
-            out[i].descriptors = (float*)(blk + kb);
+            out[i].descriptors = (Desc*)(blk + kb);
             pooled[i] = 1;
             continue;
         }
         out[i].keypoints = (sift_keypoint_t*)malloc(c * sizeof(sift_keypoint_t));
-        out[i].descriptors = (float*)malloc(c * kDesc);
+        out[i].descriptors = (Desc*)malloc(c * kDesc);
         if (!out[i].keypoints || !out[i].descriptors) return fail(SIFT_ERR_NOMEM, "host allocation failed");
         staged += c;
     }
@@ -1490,7 +1501,7 @@ int collect_pinned(sh::Context* C, int n, sh::RunOutputs& R, const std::vector<u
         void* dd = pooled[i] ? (void*)out[i].descriptors : (void*)(sdesc + so * kDesc);
         hipError_t e = hipMemcpyAsync(kd, R.d_kps + b, c * sizeof(sh::Keypoint), hipMemcpyDeviceToHost, C->stream);
         if (e == hipSuccess)
-            e = hipMemcpyAsync(dd, R.d_desc + b * 128, c * kDesc, hipMemcpyDeviceToHost, C->stream);
+            e = hipMemcpyAsync(dd, d_desc + b * 128, c * kDesc, hipMemcpyDeviceToHost, C->stream);
         if (e != hipSuccess) {
             // copies already queued must land before the caller frees (and the
             // pool reuses) the blocks they write
@@ -1511,10 +1522,12 @@ int collect_pinned(sh::Context* C, int n, sh::RunOutputs& R, const std::vector<u
     return SIFT_OK;
 }
 
+// Copies the results out: f32 descriptors into `out`, or (when out8 is set)
+// the u8 descriptors into `out8`, with the keypoint convention kp_conv.
 int collect(sh::Context* C, int n, sh::RunOutputs& R, sift_result_t* out, bool* retry,
             sift_result_u8_t* out8 = nullptr, uint32_t kp_conv = SIFT_KEYPOINTS_CPU) {
-    std::vector<unsigned> sum(n + 3);
-    HIP_TRY(hipMemcpyAsync(sum.data(), R.d_summary, (n + 3) * 4, hipMemcpyDeviceToHost, C->stream));
+    const unsigned* const sum = R.h_summary;
+    HIP_TRY(hipMemcpyAsync(R.h_summary, R.d_summary, (n + 3) * 4, hipMemcpyDeviceToHost, C->stream));
     HIP_TRY(hipStreamSynchronize(C->stream));
     const size_t ncand = sum[0], nkp = sum[1];
     *retry = false;
@@ -1524,56 +1537,20 @@ int collect(sh::Context* C, int n, sh::RunOutputs& R, sift_result_t* out, bool* 
         *retry = true;
         return SIFT_OK;
     }
-    if (!out && !out8) return SIFT_OK;
-    if (!out8) return collect_pinned(C, n, R, sum, out);
-    const size_t dsz = out8 ? 128 : 128 * 4;
-    const size_t kbytes = nkp * sizeof(sh::Keypoint), dbytes = nkp * dsz;
-    int rc = C->ensure_pinned_out(kbytes + dbytes + 256);
-    if (rc) return rc;
-    sh::Keypoint* kps = (sh::Keypoint*)C->pinned_out;
-    char* desc = C->pinned_out + ((kbytes + 255) / 256) * 256;
-    if (nkp) {
-        HIP_TRY(hipMemcpyAsync((void*)kps, R.d_kps, kbytes, hipMemcpyDeviceToHost, C->stream));
-        HIP_TRY(hipMemcpyAsync((void*)desc, out8 ? (const void*)R.d_desc_u8 : (const void*)R.d_desc,
-                               dbytes, hipMemcpyDeviceToHost, C->stream));
-        HIP_TRY(hipStreamSynchronize(C->stream));
-    }
-    if (kp_conv == SIFT_KEYPOINTS_WGPU_V2)
-        for (size_t k = 0; k < nkp; k++) {
-            kps[k].size = kps[k].size * 2.0f;
-            kps[k].response = 0.0f;
-            kps[k].octave = 0;
-            kps[k].layer = 0;
-        }
     if (out8) {
-        for (int i = 0; i < n; i++) {
-            size_t b = sum[2 + i], c = sum[3 + i] - b;
-            out8[i] = sift_result_u8_t{nullptr, nullptr, c};
-            if (c) {
-                out8[i].keypoints = (sift_keypoint_t*)malloc(c * sizeof(sift_keypoint_t));
-                out8[i].descriptors = (uint8_t*)malloc(c * 128);
-                if (!out8[i].keypoints || !out8[i].descriptors) return fail(SIFT_ERR_NOMEM, "host allocation failed");
-                memcpy(out8[i].keypoints, kps + b, c * sizeof(sift_keypoint_t));
-                memcpy(out8[i].descriptors, desc + b * 128, c * 128);
+        int rc = collect_pinned(C, n, R, sum, R.d_desc_u8, out8);
+        if (rc || kp_conv != SIFT_KEYPOINTS_WGPU_V2) return rc;
+        for (int i = 0; i < n; i++)
+            for (size_t k = 0; k < out8[i].count; k++) {
+                sift_keypoint_t& kp = out8[i].keypoints[k];
+                kp.size = kp.size * 2.0f;
+                kp.response = 0.0f;
+                kp.octave = 0;
+                kp.layer = 0;
             }
-        }
         return SIFT_OK;
     }
-    for (int i = 0; i < n; i++) {
-        size_t b = sum[2 + i], e = sum[3 + i];
-        size_t c = e - b;
-        out[i].count = c;
-        out[i].keypoints = nullptr;
-        out[i].descriptors = nullptr;
-        if (c) {
-            out[i].keypoints = (sift_keypoint_t*)malloc(c * sizeof(sift_keypoint_t));
-            out[i].descriptors = (float*)malloc(c * 128 * sizeof(float));
-            if (!out[i].keypoints || !out[i].descriptors) return fail(SIFT_ERR_NOMEM, "host allocation failed");
-            memcpy(out[i].keypoints, kps + b, c * sizeof(sift_keypoint_t));
-            memcpy(out[i].descriptors, desc + b * 128 * 4, c * 128 * sizeof(float));
-        }
-    }
-    return SIFT_OK;
+    return out ? collect_pinned(C, n, R, sum, R.d_desc, out) : SIFT_OK;
 }
 
 }  // namespace
@@ -1749,8 +1726,10 @@ int sift_hip_detect_batch_u8(sift_hip_ctx* ctx, const sift_color_image_t* images
 
 void sift_result_u8_free(sift_result_u8_t* r) {
     if (!r) return;
-    free(r->keypoints);
-    free(r->descriptors);
+    if (!sh::pinned_release(r->keypoints)) {
+        free(r->keypoints);
+        free(r->descriptors);
+    }
     r->keypoints = nullptr;
     r->descriptors = nullptr;
     r->count = 0;
@@ -1766,14 +1745,14 @@ int sift_hip_to_luma8(sift_hip_ctx* ctx, const sift_color_image_t* image, uint8_
     const uint32_t w = image->width, h = image->height;
     const size_t row = (size_t)w * sh::pixel_bytes(image->format);
     const size_t stride = image->stride ? image->stride : row;
-    const size_t cpitch = round_up(row, 64), gpitch = round_up(w, 64);
+    const size_t cpitch = sh::host_pitch(row), gpitch = round_up(w, 64);
     sh::Carver L;
     const size_t job_off = L.take(sizeof(sh::LumaJob));
     const size_t color_off = L.take(cpitch * h);
     const size_t gray_off = L.take(gpitch * h);
     if ((rc = C->ensure_arena(L.off))) return rc;
-    if ((rc = C->ensure_pinned(256 + row * h))) return rc;
-    if ((rc = C->ensure_pinned_out((size_t)w * h))) return rc;
+    if ((rc = C->ensure_pinned(256 + cpitch * h))) return rc;
+    if ((rc = C->ensure_pinned_out(gpitch * h))) return rc;
     HIP_TRY(hipStreamSynchronize(C->stream));  // pinned staging is reused across calls
     sh::LumaJob J{};
     J.src = (const uint8_t*)C->arena + color_off;
@@ -1787,16 +1766,15 @@ int sift_hip_to_luma8(sift_hip_ctx* ctx, const sift_color_image_t* image, uint8_
     J.tiles = J.tiles_x * J.h;
     J.tile_begin = 0;
     memcpy(C->pinned, &J, sizeof(J));
-    for (uint32_t y = 0; y < h; y++) memcpy(C->pinned + 256 + y * row, image->data + y * stride, row);
+    // rows at the device pitch on both ways, so the copies are linear
+    for (uint32_t y = 0; y < h; y++) memcpy(C->pinned + 256 + y * cpitch, image->data + y * stride, row);
     HIP_TRY(hipMemcpyAsync(C->arena + job_off, C->pinned, sizeof(J), hipMemcpyHostToDevice, C->stream));
-    HIP_TRY(hipMemcpy2DAsync(C->arena + color_off, cpitch, C->pinned + 256, row, row, h,
-                             hipMemcpyHostToDevice, C->stream));
+    HIP_TRY(hipMemcpyAsync(C->arena + color_off, C->pinned + 256, cpitch * h, hipMemcpyHostToDevice, C->stream));
     sh::launch_luma((const sh::LumaJob*)(C->arena + job_off), 1, J.tiles, C->stream);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpy2DAsync(C->pinned_out, w, C->arena + gray_off, gpitch, w, h, hipMemcpyDeviceToHost,
-                             C->stream));
+    HIP_TRY(hipMemcpyAsync(C->pinned_out, C->arena + gray_off, gpitch * h, hipMemcpyDeviceToHost, C->stream));
     HIP_TRY(hipStreamSynchronize(C->stream));
-    memcpy(out, C->pinned_out, (size_t)w * h);
+    for (uint32_t y = 0; y < h; y++) memcpy(out + (size_t)y * w, C->pinned_out + y * gpitch, w);
     return SIFT_OK;
 }
 
@@ -1822,8 +1800,8 @@ int sift_hip_detect_batch_device(sift_hip_ctx* ctx, const sift_image_t* images,
         sh::RunOutputs R;
         int rc = C->run(B, &R);
         if (rc) return rc;
-        std::vector<unsigned> sum(n + 3);
-        HIP_TRY(hipMemcpyAsync(sum.data(), R.d_summary, (n + 3) * 4, hipMemcpyDeviceToHost, C->stream));
+        const unsigned* const sum = R.h_summary;
+        HIP_TRY(hipMemcpyAsync(R.h_summary, R.d_summary, (n + 3) * 4, hipMemcpyDeviceToHost, C->stream));
         HIP_TRY(hipStreamSynchronize(C->stream));
         if (sum[0] > (unsigned)R.cap || sum[1] > (unsigned)R.kcap) {
             C->cand_cap = std::max(C->cand_cap, (size_t)sum[0] + sum[0] / 4 + 1024);

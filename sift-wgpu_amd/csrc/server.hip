@@ -87,8 +87,9 @@ struct Request {
     uint32_t w, h;
     uint32_t format;  // SIFT_PIXEL_*
     sift_params_t params;
-    // the frame's rows, packed: a pinned pool block (copied to the device without
-    // staging), or, when the pool has none to give, plain host memory
+    // the frame's rows at the device pitch (host_pitch): a pinned pool block
+    // (copied to the device as it is, without staging), or, when the pool has
+    // none to give, plain host memory
     struct Pixels {
         uint8_t* p = nullptr;
         bool pinned = false;
@@ -151,9 +152,10 @@ void run_batch(Context* lane, const std::vector<Request>& batch, std::vector<sif
         Batch B;
         B.host_pinned = true;
         for (size_t i = i0; i < i1; i++) {
-            const uint32_t row = batch[i].w * (uint32_t)pixel_bytes(batch[i].format);
+            const uint32_t pitch =
+                (uint32_t)host_pitch((size_t)batch[i].w * pixel_bytes(batch[i].format));
             B.host_pinned = B.host_pinned && batch[i].pixels.pinned;
-            B.images.push_back(sift_image_t{batch[i].pixels.p, batch[i].w, batch[i].h, row});
+            B.images.push_back(sift_image_t{batch[i].pixels.p, batch[i].w, batch[i].h, pitch});
             B.formats.push_back(batch[i].format);
             B.params.push_back(batch[i].params);
         }
@@ -277,14 +279,14 @@ int submit_frame(sift_hip_ctx* ctx, const sift_color_image_t* image, const sift_
     if (r.bytes > S->lane_share) {
         rc = set_error(SIFT_ERR_NOMEM, "frame needs more device memory than a lane's share of the HBM budget");
     } else {
-        const size_t row = (size_t)r.w * bpp;
-        const bool ok = r.pixels.alloc(row * r.h);
+        const size_t row = (size_t)r.w * bpp, pitch = host_pitch(row);
+        const bool ok = r.pixels.alloc(pitch * r.h);
         const size_t stride = image->stride ? image->stride : row;
-        if (ok && stride == row) {
+        if (ok && stride == pitch && row == pitch) {
             memcpy(r.pixels.p, image->data, row * r.h);
         } else if (ok) {
             for (uint32_t y = 0; y < r.h; y++)
-                memcpy(r.pixels.p + (size_t)y * row, image->data + (size_t)y * stride, row);
+                memcpy(r.pixels.p + (size_t)y * pitch, image->data + (size_t)y * stride, row);
         }
         r.submit_ms = t_submit;
         std::lock_guard<std::mutex> lk(S->mu);

@@ -91,6 +91,13 @@ struct ExternalMem {
     unsigned* offsets = nullptr;  // the caller's n + 1 per-image keypoint offsets
 };
 
+// Bytes between the rows of a host image on its way to the device, which are
+// the device's: a row of `row` bytes starts on a 64-byte boundary.
+constexpr size_t host_pitch(size_t row) { return (row + 63) / 64 * 64; }
+// The staging of a batch's host inputs is copied to the device in pieces of at
+// least this many bytes, so the host's copy of the next piece runs beside it.
+constexpr size_t kStageChunk = (size_t)1 << 20;
+
 struct Batch {
     const ExternalMem* ext = nullptr;  // set: no allocation, no graphs, no timing
     std::vector<sift_image_t> images;
@@ -98,7 +105,9 @@ struct Batch {
     std::vector<sift_params_t> params;
     bool desc_u8 = false;           // also produce the u8 descriptors (RunOutputs::d_desc_u8)
     bool device_input = false;
-    bool host_pinned = false;  // host inputs are pinned (pinned_alloc): copied without staging
+    // host inputs are pinned (pinned_alloc), their rows host_pitch apart: copied
+    // without staging
+    bool host_pinned = false;
     bool pyramid_only = false;
     bool want_dog = false;
     bool want_stages = false;
@@ -110,6 +119,7 @@ struct RunOutputs {
     float* d_desc = nullptr;
     uint8_t* d_desc_u8 = nullptr;
     unsigned* d_summary = nullptr;
+    unsigned* h_summary = nullptr;  // pinned, n + 3 words, for the summary's way back (not in external memory)
     Cand* d_cand = nullptr;
     float* d_cand_resp = nullptr;
     Keypoint* d_ref = nullptr;
