@@ -368,7 +368,7 @@ enum KernelId {
     K_BLUR_H = 0, K_BLUR_V, K_COPY, K_BLUR_H_GENERIC, K_RESIZE_V, K_RESIZE_H, K_EXTREMA, K_SCAN,
     K_COMPACT, K_REFINE, K_ORIENT, K_DESCRIPTOR, K_FINALIZE, K_BLUR_V_NARROW, K_BLUR_V_GENERIC,
     K_BLUR_H2, K_BLUR_H_SMALL, K_BLUR_V_SMALL, K_LUMA, K_DESC_U8, K_RESIZE_FUSED, K_BLUR_V_SMALL8,
-    K_BLUR_H16, K_BLUR_V8, K_COUNT
+    K_BLUR_H16, K_BLUR_V8, K_BLUR_HV, K_BLUR_HV_LONG, K_BLUR_HV_SMALL, K_COUNT
 };
 // Names as rocprofv3 reports the kernels (template arguments included).
 const char* const kKernelNames[K_COUNT] = {
@@ -376,7 +376,9 @@ const char* const kKernelNames[K_COUNT] = {
     "k_extrema_tile", "k_scan", "k_compact", "k_refine", "k_orient", "k_descriptor",
     "k_finalize", "k_blur_v_narrow", "k_blur_v_generic", "k_blur_h<2>", "k_blur_h_small",
     "k_blur_v_small", "k_luma", "k_desc_u8", "k_resize_fused", "k_blur_v_small8", "k_blur_h<16>",
-    "k_blur_v<8>"};
+    "k_blur_v<8>", "k_blur_hv<false>", "k_blur_hv<true>", "k_blur_hv_small"};
+
+bool is_blur_hv(int kind) { return kind == K_BLUR_HV || kind == K_BLUR_HV_LONG || kind == K_BLUR_HV_SMALL; }
 
 
 double blur_job_bytes(const BlurJob& j, int kind) {
@@ -391,7 +393,7 @@ double blur_job_bytes(const BlurJob& j, int kind) {
 // the reference's f32 arithmetic, which the kernels keep without contraction.
 double blur_job_ops(const BlurJob& j, int kind) {
     if (kind == K_COPY) return 0.0;
-    return 2.0 * (double)j.w * j.h * j.ntaps;
+    return (is_blur_hv(kind) ? 4.0 : 2.0) * (double)j.w * j.h * j.ntaps;
 }
 double resize_job_ops(const ResizeJob& j, int kind) {
     const double v = 2.0 * (double)j.in_w * j.out_h * (kind == K_RESIZE_FUSED ? j.vmaxtaps : j.maxtaps);
@@ -483,6 +485,29 @@ std::pair<int, int> blur_heuristic(int w, int h, int ntaps, int npad) {
     else if (blur_v_valid(BV_NARROW, w, h, ntaps)) vf = BV_NARROW;
     else vf = BV_GENERIC;
     return {hf, vf};
+}
+
+// Whether both passes of a blur go in one kernel (k_blur_hv / k_blur_hv_small).
+bool blur_hv_valid(const uint8_t* src, int src_pitch, int ntaps) {
+    return ntaps >= kHvMinTaps && ntaps <= kHvMaxTaps && (((uintptr_t)src | (uintptr_t)src_pitch) & 3) == 0;
+}
+// The fused blur's tiles for a job of a step whose fused jobs hold step_px pixels.
+// The large tiles need 6 Mpixel to fill the GPU (16 levels of 640 x 480, 7 taps:
+// 14.1 us against 12.7 us with the small ones; 8 of 1280 x 720: 14.6 against
+// 16.5 us), and per pixel of their tiles cost 1/1.25 of the small ones (1/1.5 for
+// the long tap counts), which a level that fills them badly loses (64 levels of
+// 320 x 240, 7 taps: 14.5 against 12.6 us).
+bool blur_hv_large(const BlurJob& J, double step_px) {
+    if (step_px < 6e6) return false;
+    auto fill = [&](int tw, int th) {
+        return (double)J.w * J.h / ((double)round_up(J.w, tw) * round_up(J.h, th));
+    };
+    return fill(kHvTileW, kHvTileH) * (J.ntaps > kHvShortTaps ? 1.5 : 1.25) >= fill(kHvSmallW, kHvSmallH);
+}
+void blur_hv_tiles(BlurJob& J, bool large) {
+    const int tw = large ? kHvTileW : kHvSmallW, th = large ? kHvTileH : kHvSmallH;
+    J.tiles_x = (J.w + tw - 1) / tw;
+    J.tiles = J.tiles_x * ((J.h + th - 1) / th);
 }
 
 // Tile counts of a job in a form.
@@ -751,9 +776,11 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         maxO = std::max(maxO, (int)shapes[i].size());
         Lmax = std::max(Lmax, (int)B.params[i].num_intervals + 3);
     }
-    // per blur step up to 12 blur launches (five H forms, six V forms, the copy)
-    // and 3 Lanczos3 launches; at most 1 + maxO * Lmax steps
-    const size_t max_launches = (size_t)(1 + maxO * Lmax) * 15 + (size_t)maxO * 3 + 8;
+    // per blur step up to 15 blur launches (three fused, five H forms, six V forms,
+    // the copy) and 3 Lanczos3 launches; at most 1 + maxO * Lmax steps. One image
+    // has at most three octaves in a step, with two launches each (the server's
+    // frame_device_bytes counts 15 per frame).
+    const size_t max_launches = (size_t)(1 + maxO * Lmax) * (n == 1 ? 15 : 18) + (size_t)maxO * 3 + 8;
     const size_t max_jobs = (size_t)n * ((1 + (size_t)maxO * Lmax) * 2 + (size_t)maxO * 2);
     const size_t blob_bound = max_launches * 256 + max_jobs * std::max(sizeof(BlurJob), sizeof(ResizeJob)) +
                               octs.size() * sizeof(OctaveDesc) + (size_t)n * sizeof(ImageParams) +
@@ -779,7 +806,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     char* T = B.ext ? B.ext->base : tables.dev;
     auto AP = [&](size_t off) { return A + off; };
 
-    std::vector<BlurJob> hj, hj2, hj16, hgj, hsj, vj, v8j, vnj, vgj, vsj, vs8j, cj;
+    std::vector<BlurJob> hj, hj2, hj16, hgj, hsj, vj, v8j, vnj, vgj, vsj, vs8j, cj, hvj;
     const std::pair<int, int> forced = blur_forced();
     int vn_rows = 0, hs_taps4 = 0, vs_taps4 = 0, vs_rows = 0, vs8_taps4 = 0, vs8_rows = 0;
 
@@ -833,6 +860,14 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         J.taps = (const float*)(T + R.off);
         J.ntaps = R.ntaps;
         J.ntaps_pad = R.npad;
+        if (!dog && forced.first < 0 && forced.second < 0 && blur_hv_valid(src, src_pitch, R.ntaps)) {
+            J.src = src;
+            J.src_pitch = src_pitch;
+            J.dst = dst;
+            J.dst_pitch = dst_pitch;
+            hvj.push_back(J);  // its tiles: flush_blur
+            return;
+        }
         const std::pair<int, int> form = blur_choice(w, h, R.ntaps, R.npad, n >= kTuneManyJobs, forced);
         const int n4 = (R.ntaps + 3) & ~3, r = R.ntaps / 2;
         BlurJob H = J;
@@ -886,6 +921,17 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         for (auto& j : hj) maxpad = std::max(maxpad, j.ntaps_pad);
         for (auto& j : hj2) maxpad2 = std::max(maxpad2, j.ntaps_pad);
         for (auto& j : hj16) maxpad16 = std::max(maxpad16, j.ntaps_pad);
+        std::vector<BlurJob> hv[3];  // large tiles with short and long tap counts, small tiles
+        double step_px = 0.0;
+        for (const BlurJob& j : hvj) step_px += (double)j.w * j.h;
+        for (BlurJob& j : hvj) {
+            const bool large = blur_hv_large(j, step_px);
+            blur_hv_tiles(j, large);
+            hv[large ? j.ntaps > kHvShortTaps : 2].push_back(j);
+        }
+        push_launch(K_BLUR_HV, hv[0], 0, 0);
+        push_launch(K_BLUR_HV_LONG, hv[1], 0, 0);
+        push_launch(K_BLUR_HV_SMALL, hv[2], 0, 0);
         push_launch(K_BLUR_H16, hj16, maxpad16, 16);
         push_launch(K_BLUR_H, hj, maxpad, 8);
         push_launch(K_BLUR_H2, hj2, maxpad2, 2);
@@ -903,6 +949,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         hj16.clear();
         v8j.clear();
         cj.clear();
+        hvj.clear();
         vn_rows = hs_taps4 = vs_taps4 = vs_rows = vs8_taps4 = vs8_rows = 0;
     };
 
@@ -1139,6 +1186,13 @@ int Context::run(const Batch& B, RunOutputs* outs) {
                     break;
                 case K_BLUR_V: launch_blur_v((const BlurJob*)(D + L.job_off), L.njobs, L.tiles, 0, st); break;
                 case K_BLUR_V8: launch_blur_v8((const BlurJob*)(D + L.job_off), L.njobs, L.tiles, st); break;
+                case K_BLUR_HV:
+                case K_BLUR_HV_LONG:
+                    launch_blur_hv((const BlurJob*)(D + L.job_off), L.njobs, L.tiles, L.kind == K_BLUR_HV_LONG, st);
+                    break;
+                case K_BLUR_HV_SMALL:
+                    launch_blur_hv_small((const BlurJob*)(D + L.job_off), L.njobs, L.tiles, st);
+                    break;
                 case K_BLUR_V_NARROW:
                     launch_blur_v((const BlurJob*)(D + L.job_off), L.njobs, L.tiles, L.variant, st);
                     break;

@@ -57,6 +57,41 @@ __device__ __forceinline__ float mul_add_exact(float acc, float a, float b) {
     return __fadd_rn(acc, __fmul_rn(a, b));
 }
 
+// From here on v_cvt_pk_u8_f32 truncates: the wave's f32 rounding mode is set to
+// round toward zero. Every sum of `a` is complete before the switch and is read
+// only after it (volatile asm statements keep their order). No other f32
+// arithmetic may follow, but for round_even().
+template <int N>
+__device__ __forceinline__ void pin(float (&a)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; i++) asm volatile("" : "+v"(a[i]));
+}
+template <int N>
+__device__ __forceinline__ void truncating(float (&a)[N]) {
+    pin(a);
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\ts_nop 1");
+    pin(a);
+}
+// Back to round to nearest even, once the conversions packed into v are done.
+template <int N>
+__device__ __forceinline__ void round_even(unsigned (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; i++) asm volatile("" : "+v"(v[i]));
+    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\ts_nop 1");
+#pragma unroll
+    for (int i = 0; i < N; i++) asm volatile("" : "+v"(v[i]));
+}
+// Four non-negative sums as bytes, after truncating(): v_cvt_pk_u8_f32 under
+// round toward zero equals min((unsigned)x, 255) for every f32 x >= 0 (checked for
+// all of them up to 2^33) and places the byte, one instruction where the
+// conversion, the bound and the packing took three.
+__device__ __forceinline__ unsigned pack_u8(float a, float b, float c, float d) {
+    unsigned v = __builtin_amdgcn_cvt_pk_u8_f32(a, 0u, 0u);
+    v = __builtin_amdgcn_cvt_pk_u8_f32(b, 1u, v);
+    v = __builtin_amdgcn_cvt_pk_u8_f32(c, 2u, v);
+    return __builtin_amdgcn_cvt_pk_u8_f32(d, 3u, v);
+}
+
 __device__ __forceinline__ float q255(unsigned v) { return __fdiv_rn((float)v, 255.0f); }
 
 // The tap tables are written by host copies before any launch and only read
@@ -243,32 +278,24 @@ __global__ __launch_bounds__(kThreads) void k_blur_h(const BlurJob* __restrict__
     const int x = x0 + base;
     if (x >= w) return;
     uint8_t* dst = J.dst + (size_t)y * J.dst_pitch + x;
-    unsigned res[PX];
+    truncating(acc);
+    if constexpr (PX >= 8) {
+        unsigned v[PX / 4];
 #pragma unroll
-    for (int q = 0; q < PX; q++) res[q] = u8_trunc(acc[q]);
-    if constexpr (PX == 8) {
-        if (x + 8 <= w) {
-            uint2 v;
-            v.x = res[0] | (res[1] << 8) | (res[2] << 16) | (res[3] << 24);
-            v.y = res[4] | (res[5] << 8) | (res[6] << 16) | (res[7] << 24);
-            *(uint2*)dst = v;
+        for (int k = 0; k < PX / 4; k++) v[k] = pack_u8(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]);
+        if (x + PX <= w) {
+            if constexpr (PX == 8) *(uint2*)dst = make_uint2(v[0], v[1]);
+            else *(uint4*)dst = make_uint4(v[0], v[1], v[2], v[3]);
             return;
         }
-    }
-    if constexpr (PX == 16) {
-        if (x + 16 <= w) {
-            uint4 v;
-            v.x = res[0] | (res[1] << 8) | (res[2] << 16) | (res[3] << 24);
-            v.y = res[4] | (res[5] << 8) | (res[6] << 16) | (res[7] << 24);
-            v.z = res[8] | (res[9] << 8) | (res[10] << 16) | (res[11] << 24);
-            v.w = res[12] | (res[13] << 8) | (res[14] << 16) | (res[15] << 24);
-            *(uint4*)dst = v;
-            return;
-        }
-    }
 #pragma unroll
-    for (int q = 0; q < PX; q++)
-        if (x + q < w) dst[q] = (uint8_t)res[q];
+        for (int q = 0; q < PX; q++)
+            if (x + q < w) dst[q] = (uint8_t)(v[q / 4] >> (8 * (q & 3)));
+    } else {
+#pragma unroll
+        for (int q = 0; q < PX; q++)
+            if (x + q < w) dst[q] = (uint8_t)__builtin_amdgcn_cvt_pk_u8_f32(acc[q], 0u, 0u);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -286,26 +313,38 @@ __device__ __forceinline__ void cvt4(unsigned v, float* o) {
     o[3] = (float)(v >> 24);
 }
 
-__device__ __forceinline__ void store_row4(const BlurJob& J, int y, int x, const float* acc) {
-    unsigned res[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) res[c] = u8_trunc(acc[c]);
+// v: four pixels of row y from column x, packed.
+__device__ __forceinline__ void store_row4(const BlurJob& J, int y, int x, unsigned v) {
     uint8_t* dst = J.dst + (size_t)y * J.dst_pitch + x;
     const int w = J.w;
     if (x + 4 <= w) {
-        *(unsigned*)dst = res[0] | (res[1] << 8) | (res[2] << 16) | (res[3] << 24);
+        *(unsigned*)dst = v;
     } else {
 #pragma unroll
         for (int c = 0; c < 4; c++)
-            if (x + c < w) dst[c] = (uint8_t)res[c];
+            if (x + c < w) dst[c] = (uint8_t)(v >> (8 * c));
     }
     if (J.dog) {
         const uint8_t* prev = J.prev + (size_t)y * J.dst_pitch + x;
         float* dg = J.dog + (size_t)y * J.dog_pitch + x;
 #pragma unroll
         for (int c = 0; c < 4; c++)
-            if (x + c < w) dg[c] = q255(res[c]) - q255(prev[c]);
+            if (x + c < w) dg[c] = q255((v >> (8 * c)) & 0xff) - q255(prev[c]);
     }
+}
+
+// RV rows of four sums as packed bytes; the rounding mode is as before after it
+// (the DoG epilogue divides).
+template <int RV>
+__device__ __forceinline__ void trunc_rows(float (&acc)[RV][4], unsigned (&res)[RV]) {
+#pragma unroll
+    for (int q = 0; q < RV; q++) pin(acc[q]);
+    truncating(acc[0]);
+#pragma unroll
+    for (int q = 1; q < RV; q++) pin(acc[q]);
+#pragma unroll
+    for (int q = 0; q < RV; q++) res[q] = pack_u8(acc[q][0], acc[q][1], acc[q][2], acc[q][3]);
+    round_even(res);
 }
 
 // Any tap count: a register window of RV input rows x 4 columns slides over the
@@ -426,11 +465,211 @@ __global__ __launch_bounds__(kThreads) void k_blur_v(const BlurJob* __restrict__
     if constexpr (RV == kVRows) {
         if (!fixed) vconv_blocks<RV>(J.src + x, pitch, yb - r, h, n, taps, acc);
     }
+    unsigned res[RV];
+    trunc_rows(acc, res);
 #pragma unroll
     for (int q = 0; q < RV; q++) {
         const int y = yb + q;
         if (y >= h) break;
-        store_row4(J, y, x, acc[q]);
+        store_row4(J, y, x, res[q]);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Both passes of one blur in one kernel, for kernels of 5 to kHvMaxTaps taps. A
+// work-group makes a tile of TW columns x TH rows: the horizontal pass of the
+// tile's TH + 2r input rows (clamped to the image) goes to LDS as bytes, and the
+// vertical pass reads them there, so the level between the passes, its write and
+// its read, never leave the CU, and a level takes one launch.
+// Horizontal: TW / PX lanes per row, PX outputs per lane, straight from global
+// memory: a lane loads the aligned words of its PX + 2 kHalo window bytes (its
+// neighbours' loads hit L1) and needs no LDS or exchange. In tiles at the left or
+// right edge the word addresses are clamped and the bytes past the edge replaced
+// by one v_perm per word (a word past the image is never read: the last one read
+// holds the row's last pixel).
+// Vertical: RV rows x 4 columns (256-column tiles) or x 1 column (64) per lane,
+// each staged row read and converted once, as in k_blur_v.
+// Bound: the exact multiply and add of every tap; the staged rows' 2r / TH extra
+// horizontal work pays for the saved level. 64 levels of 1920 x 1080, 7 / 15 / 21
+// taps: 114 / 201 / 289 us against 149 / 232 / 338 us of the best two-pass forms;
+// one level of 640 x 480, 9 / 33 taps (of which about 6 us are the launch and its
+// event): 6.2 / 8.4 against 12.4 us; 33 taps at 480 x 270 are the worst case met
+// (48.5 against 42.7 us at 64 levels, for the tiles that do not fit the level).
+// ---------------------------------------------------------------------------
+template <int NT, int TW, int PX, int RV, int TH>
+__device__ __forceinline__ void blur_hv_tile(const BlurJob& J, int x0, int y0, uint8_t* rows) {
+    constexpr int R = NT / 2, kHalo = R <= 8 ? 8 : 16, NW = (PX + 2 * kHalo) / 4;
+    constexpr int kLanes = TW / PX;               // lanes per row
+    constexpr int kPassRows = kThreads / kLanes;  // rows of one pass of the work-group
+    const int w = J.w, h = J.h, pitch = J.src_pitch;
+    const ctap_t* taps = as_const_taps(J.taps);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int xl = (tid % kLanes) * PX;  // the lane's first column in the tile
+    const bool inside = x0 >= kHalo && x0 + TW + kHalo <= w;
+    const int wl = (w - 1) & ~3, last = (w - 1) & 3;  // the row's last word and its last pixel's byte
+    const unsigned sel_end = last == 3 ? 0x03020100u : last == 2 ? 0x02020100u : last == 1 ? 0x01010100u : 0u;
+    const unsigned sel_past = (unsigned)last * 0x01010101u;
+    float wk[NT];
+#pragma unroll
+    for (int k = 0; k < NT; k++) wk[k] = taps[k];
+#pragma unroll 1
+    for (int r0 = 0; r0 < TH + 2 * R; r0 += kPassRows) {
+        const int row = r0 + tid / kLanes;
+        if (row >= TH + 2 * R) break;
+        const int yy = min(max(y0 - R + row, 0), h - 1);
+        gbyte_t* src = (gbyte_t*)J.src + (size_t)yy * pitch;
+        const int xb = x0 + xl - kHalo;
+        unsigned u[NW];
+        if (inside) {
+#pragma unroll
+            for (int k = 0; k < NW; k++) u[k] = *(__attribute__((address_space(1))) const unsigned*)(src + xb + 4 * k);
+        } else {
+#pragma unroll
+            for (int k = 0; k < NW; k++)
+                u[k] = *(__attribute__((address_space(1))) const unsigned*)(src + min(max(xb + 4 * k, 0), wl));
+#pragma unroll
+            for (int k = 0; k < NW; k++) {
+                const int xw = xb + 4 * k;
+                const unsigned sel = xw < 0 ? 0u : xw < wl ? 0x03020100u : xw == wl ? sel_end : sel_past;
+                u[k] = __builtin_amdgcn_perm(u[k], u[k], sel);
+            }
+        }
+        float win[PX + NT - 1];
+#pragma unroll
+        for (int k = 0; k < PX + NT - 1; k++) {
+            constexpr int o = kHalo - R;
+            win[k] = (float)((u[(o + k) / 4] >> (8 * ((o + k) & 3))) & 0xff);
+        }
+        float acc[PX];
+#pragma unroll
+        for (int q = 0; q < PX; q++) acc[q] = __fmul_rn(win[q], wk[0]);
+#pragma unroll
+        for (int k = 1; k < NT; k++)
+#pragma unroll
+            for (int q = 0; q < PX; q++) acc[q] = mul_add_exact(acc[q], win[q + k], wk[k]);
+        truncating(acc);
+        unsigned v[PX / 4];
+#pragma unroll
+        for (int k = 0; k < PX / 4; k++) v[k] = pack_u8(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]);
+        round_even(v);
+        uint8_t* to = rows + row * TW + xl;
+        if constexpr (PX == 16) *(uint4*)to = make_uint4(v[0], v[1], v[2], v[3]);
+        else if constexpr (PX == 8) *(uint2*)to = make_uint2(v[0], v[1]);
+        else *(unsigned*)to = v[0];
+    }
+    __syncthreads();
+    if constexpr (TW == 64) {
+        static_assert(TH == RV * kThreads / 64, "one group of rows per wave");
+        const int x = x0 + lane, yb = y0 + wave * RV;
+        if (x >= w || yb >= h) return;
+        const uint8_t* col = rows + wave * RV * TW + lane;
+        float acc[RV];
+#pragma unroll
+        for (int i = 0; i < RV + NT - 1; i++) {
+            const float p = (float)col[i * TW];
+#pragma unroll
+            for (int q = 0; q < RV; q++) {
+                const int k = i - q;
+                if (k < 0 || k >= NT) continue;
+                acc[q] = k == 0 ? __fmul_rn(p, wk[0]) : mul_add_exact(acc[q], p, wk[k]);
+            }
+        }
+        truncating(acc);
+#pragma unroll
+        for (int q = 0; q < RV; q++)
+            if (yb + q < h)
+                J.dst[(size_t)(yb + q) * J.dst_pitch + x] = (uint8_t)__builtin_amdgcn_cvt_pk_u8_f32(acc[q], 0u, 0u);
+        return;
+    }
+    const int x = x0 + 4 * lane;
+    for (int g = wave; g < TH / RV; g += kThreads / 64) {
+        const int yb = y0 + g * RV;
+        if (yb >= h) break;
+        const unsigned* col = (const unsigned*)rows + (g * RV) * (kVTileW / 4) + lane;
+        float acc[RV][4];
+#pragma unroll
+        for (int i = 0; i < RV + NT - 1; i++) {
+            float p[4];
+            cvt4(col[i * (kVTileW / 4)], p);
+#pragma unroll
+            for (int q = 0; q < RV; q++) {
+                const int k = i - q;
+                if (k < 0 || k >= NT) continue;
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    acc[q][c] = k == 0 ? __fmul_rn(p[c], wk[0]) : mul_add_exact(acc[q][c], p[c], wk[k]);
+            }
+        }
+        unsigned res[RV];
+        trunc_rows(acc, res);
+#pragma unroll
+        for (int q = 0; q < RV; q++)
+            if (yb + q < h && x < w) store_row4(J, yb + q, x, res[q]);
+    }
+}
+
+// Large launches: 256 x 64 tiles, the short and the long tap counts apart (77 and
+// 85 VGPRs).
+template <bool kLong>
+__global__ __launch_bounds__(kThreads) void k_blur_hv(const BlurJob* __restrict__ jobs, int njobs) {
+    constexpr int TW = kHvTileW, TH = kHvTileH;
+    __shared__ __align__(16) uint8_t rows[(TH + (kLong ? kHvMaxTaps : kHvShortTaps) - 1) * TW];
+    const int tile = xcd_remap(blockIdx.x, gridDim.x);
+    const BlurJob& J = jobs[find_job(jobs, njobs, tile)];
+    const int t = tile - J.tile_begin;
+    const int x0 = (t % J.tiles_x) * TW, y0 = (t / J.tiles_x) * TH;
+    if constexpr (!kLong) {
+        switch (J.ntaps) {
+            case 5: blur_hv_tile<5, TW, 16, 8, TH>(J, x0, y0, rows); break;
+            case 7: blur_hv_tile<7, TW, 16, 8, TH>(J, x0, y0, rows); break;
+            case 9: blur_hv_tile<9, TW, 16, 8, TH>(J, x0, y0, rows); break;
+            case 11: blur_hv_tile<11, TW, 16, 8, TH>(J, x0, y0, rows); break;
+            case 13: blur_hv_tile<13, TW, 16, 8, TH>(J, x0, y0, rows); break;
+            default: blur_hv_tile<15, TW, 16, 8, TH>(J, x0, y0, rows); break;
+        }
+    } else {
+        switch (J.ntaps) {
+            case 17: blur_hv_tile<17, TW, 8, 8, TH>(J, x0, y0, rows); break;
+            case 19: blur_hv_tile<19, TW, 8, 8, TH>(J, x0, y0, rows); break;
+            case 21: blur_hv_tile<21, TW, 8, 8, TH>(J, x0, y0, rows); break;
+            case 23: blur_hv_tile<23, TW, 8, 8, TH>(J, x0, y0, rows); break;
+            case 25: blur_hv_tile<25, TW, 8, 8, TH>(J, x0, y0, rows); break;
+            case 27: blur_hv_tile<27, TW, 8, 8, TH>(J, x0, y0, rows); break;
+            case 29: blur_hv_tile<29, TW, 8, 8, TH>(J, x0, y0, rows); break;
+            case 31: blur_hv_tile<31, TW, 8, 8, TH>(J, x0, y0, rows); break;
+            default: blur_hv_tile<33, TW, 8, 8, TH>(J, x0, y0, rows); break;
+        }
+    }
+}
+
+// Small launches (single frames, small batches, deep octaves): 64 x 16 tiles of
+// any of the tap counts. What counts there is the number of instructions of one
+// wave (a wave alone on its SIMD issues one every 8 cycles), so a lane makes few
+// outputs.
+__global__ __launch_bounds__(kThreads) void k_blur_hv_small(const BlurJob* __restrict__ jobs, int njobs) {
+    constexpr int TW = kHvSmallW, TH = kHvSmallH;
+    __shared__ __align__(16) uint8_t rows[(TH + kHvMaxTaps - 1) * TW];
+    const int tile = xcd_remap(blockIdx.x, gridDim.x);
+    const BlurJob& J = jobs[find_job(jobs, njobs, tile)];
+    const int t = tile - J.tile_begin;
+    const int x0 = (t % J.tiles_x) * TW, y0 = (t / J.tiles_x) * TH;
+    switch (J.ntaps) {
+        case 5: blur_hv_tile<5, TW, 8, 4, TH>(J, x0, y0, rows); break;
+        case 7: blur_hv_tile<7, TW, 8, 4, TH>(J, x0, y0, rows); break;
+        case 9: blur_hv_tile<9, TW, 8, 4, TH>(J, x0, y0, rows); break;
+        case 11: blur_hv_tile<11, TW, 8, 4, TH>(J, x0, y0, rows); break;
+        case 13: blur_hv_tile<13, TW, 8, 4, TH>(J, x0, y0, rows); break;
+        case 15: blur_hv_tile<15, TW, 8, 4, TH>(J, x0, y0, rows); break;
+        case 17: blur_hv_tile<17, TW, 4, 4, TH>(J, x0, y0, rows); break;
+        case 19: blur_hv_tile<19, TW, 4, 4, TH>(J, x0, y0, rows); break;
+        case 21: blur_hv_tile<21, TW, 4, 4, TH>(J, x0, y0, rows); break;
+        case 23: blur_hv_tile<23, TW, 4, 4, TH>(J, x0, y0, rows); break;
+        case 25: blur_hv_tile<25, TW, 4, 4, TH>(J, x0, y0, rows); break;
+        case 27: blur_hv_tile<27, TW, 4, 4, TH>(J, x0, y0, rows); break;
+        case 29: blur_hv_tile<29, TW, 4, 4, TH>(J, x0, y0, rows); break;
+        case 31: blur_hv_tile<31, TW, 4, 4, TH>(J, x0, y0, rows); break;
+        default: blur_hv_tile<33, TW, 4, 4, TH>(J, x0, y0, rows); break;
     }
 }
 
@@ -935,6 +1174,18 @@ void launch_blur_v(const BlurJob* d_jobs, int njobs, int total_tiles, int narrow
 void launch_blur_v8(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s) {
     if (total_tiles <= 0) return;
     hipLaunchKernelGGL(k_blur_v<8>, dim3(total_tiles), dim3(kThreads), 0, s, d_jobs, njobs);
+}
+
+void launch_blur_hv(const BlurJob* d_jobs, int njobs, int total_tiles, bool longer, hipStream_t s) {
+    if (total_tiles <= 0) return;
+    const dim3 g(total_tiles), b(kThreads);
+    if (longer) hipLaunchKernelGGL(k_blur_hv<true>, g, b, 0, s, d_jobs, njobs);
+    else hipLaunchKernelGGL(k_blur_hv<false>, g, b, 0, s, d_jobs, njobs);
+}
+
+void launch_blur_hv_small(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s) {
+    if (total_tiles <= 0) return;
+    hipLaunchKernelGGL(k_blur_hv_small, dim3(total_tiles), dim3(kThreads), 0, s, d_jobs, njobs);
 }
 
 void launch_blur_h_small(const BlurJob* d_jobs, int njobs, int total_tiles, int max_taps4,

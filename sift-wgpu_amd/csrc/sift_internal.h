@@ -120,6 +120,12 @@ void launch_blur_v(const BlurJob* d_jobs, int njobs, int total_tiles, int narrow
                    hipStream_t s);
 // 8 rows per lane (256 x 32 tiles); only for 7, 9, 11, 13 or 15 taps.
 void launch_blur_v8(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
+// Both passes in one kernel, without the DoG epilogue (BlurJob src -> dst): odd
+// tap counts from 5 to kHvMaxTaps, the source and its pitch aligned to 4 bytes.
+// kHvTileW x kHvTileH tiles, tap counts up to kHvShortTaps or (longer) above; or
+// kHvSmallW x kHvSmallH tiles of any of them.
+void launch_blur_hv(const BlurJob* d_jobs, int njobs, int total_tiles, bool longer, hipStream_t s);
+void launch_blur_hv_small(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
 void launch_resize_v(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
 // Both Lanczos3 passes in one kernel, the f32 intermediate kept in LDS: for jobs
 // whose every tile of kResizeRows x 256 outputs needs at most kResizeFusedSpan
@@ -180,6 +186,9 @@ void launch_finalize(const unsigned* d_slot_offsets, const int* d_img_slot_begin
 // the first min(*d_count, kcap) descriptors.
 void launch_desc_u8(const float* d_desc, const unsigned* d_count, int kcap, uint8_t* d_out,
                     hipStream_t s);
+// The fused blur: its tap counts and tiles.
+constexpr int kHvMinTaps = 5, kHvShortTaps = 15, kHvMaxTaps = 33;
+constexpr int kHvTileW = 256, kHvTileH = 64, kHvSmallW = 64, kHvSmallH = 16;
 // Max padded tap count handled by the LDS row-tile horizontal pass.
 constexpr int kMaxHPad = 3576;
 // Small-level kernels: taps (rounded up to 4) and staged rows they accept.
