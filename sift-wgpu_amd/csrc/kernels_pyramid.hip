@@ -2,7 +2,7 @@
 //   k_blur_h / k_blur_v : one separable pass of imageproc gaussian_blur_f32 on u8
 //                         (called at src/sift.rs:159,1211), optional DoG epilogue
 //                         (src/sift.rs:92-124,182-204) in the vertical pass.
-//   k_resize_fused      : image resize_exact(.., Lanczos3) (src/sift.rs:83-88), both
+//   k_resize_tall/_small: image resize_exact(.., Lanczos3) (src/sift.rs:83-88), both
 //                         passes in one kernel; k_resize_v/_h: the two-pass form.
 //   k_luma              : colour -> grey (image 0.25.6 to_luma8, the wasm canvas rule).
 //
@@ -1053,95 +1053,198 @@ __global__ __launch_bounds__(kThreads) void k_resize_h(const ResizeJob* __restri
 }
 
 // ---------------------------------------------------------------------------
-// Fused Lanczos3 resize: one work-group computes kResizeRows output rows x 256
-// output columns. The vertical pass for those rows over the input columns the
-// tile's horizontal windows need, [lo4, hi) with lo4 = left[ox0] rounded down to
-// a multiple of 4, goes to LDS as f32 (the same t += p * w in window order as
-// k_resize_v: wave w takes output rows w and w + 4, so its weights are
-// wave-uniform, and lane l the column quads l, l + 64, ...); the horizontal pass
-// then reads it from LDS as k_resize_h does. The f32 intermediate never goes to
-// HBM. The host takes this kernel only when every tile's span fits
-// kResizeFusedSpan (octave steps, ratio ~2, need about 524 columns).
+// Both passes of the octave step in one kernel: the vertical pass of a tile's
+// rows, over the input columns its horizontal windows need, goes to LDS as f32 (the
+// same t += p * w in window order as k_resize_v) and the horizontal pass reads it
+// there. The rounding is round(clamp(t, 0, 255)) as t + 0.5 and the conversion,
+// both under round toward zero: the sum cannot reach an integer that the exact one
+// does not, and negative sums give 0 (checked for every f32 up to 2^15).
+// k_resize_tall: tiles of kResizeTallW x kResizeTallH outputs, four rows per wave. A
+// wave's lanes hold the tile's input column quads (120 outputs need at most 64) and
+// stream the rows its four windows share once, converting each texel once instead
+// of once per window (the windows of an exact or nearly exact halving lie two, now
+// and then three rows apart; the first and last rows, whose windows are cut, take
+// each on its own). The horizontal weights go through LDS, loaded in order once per
+// tile: per output and lane they were 12 loads of 64 scattered words.
+// 64 levels of 1920 x 1080: 196 -> 135 us against a wave per output row without
+// either (576-column tiles); 960 x 540: 58 -> 42 us; one of 3840 x 2160: 24 -> 15 us.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void k_resize_fused(const ResizeJob* __restrict__ jobs,
-                                                           int njobs) {
-    __shared__ __align__(16) float vt[kResizeRows][kResizeFusedSpan];
+// NT-row windows 2 apart: output row q adds input row base + i as its tap i - 2q.
+template <int NT>
+__device__ __forceinline__ void resize_v_rows(gbyte_t* src, int pitch, int in_h, int base,
+                                              const float (&w)[4][14], float (&s)[4][4]) {
+#pragma unroll
+    for (int i = 0; i < NT + 6; i++) {
+        float p[4];
+        cvt4(*(__attribute__((address_space(1))) const unsigned*)(src + (size_t)min(base + i, in_h - 1) * pitch), p);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int k = i - 2 * q;
+            if (k < 0 || k >= NT) continue;
+#pragma unroll
+            for (int c = 0; c < 4; c++) s[q][c] = mul_add_exact(s[q][c], p[c], w[q][k]);
+        }
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void k_resize_tall(const ResizeJob* __restrict__ jobs,
+                                                          int njobs) {
+    constexpr int kTaps = kResizeMaxTaps;
+    __shared__ __align__(16) float vt[kThreads / 64][4][kResizeTallSpan];
+    __shared__ float hw[kResizeTallW * kTaps];
     const int tile = xcd_remap(blockIdx.x, gridDim.x);
     const ResizeJob& J = jobs[find_job(jobs, njobs, tile)];
     const int t = tile - J.tile_begin;
-    const int y0 = (t / J.tiles_x) * kResizeRows;
-    const int ox0 = (t % J.tiles_x) * kThreads;
-    const int oxl = min(ox0 + kThreads, J.out_w) - 1;
-    const int nrows = min(kResizeRows, J.out_h - y0);
-    const int lo4 = J.left[ox0] & ~3;
-    const int hi = J.left[oxl] + J.count[oxl];  // exclusive, <= in_w
-    const int nq = (hi - lo4 + 3) >> 2;         // column quads: 4 * nq <= kResizeFusedSpan
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int in_w = J.in_w, pitch = J.src_pitch;
-    for (int r = wave; r < nrows; r += kThreads / 64) {
-        const int oy = y0 + r;
-        const int l = J.vleft[oy], n = J.vcount[oy];
-        const ctap_t* wr = as_const_taps(J.vweights) + (size_t)oy * J.vmaxtaps;
-        for (int q = lane; q < nq; q += 64) {
-            const int x = lo4 + 4 * q;
-            const uint8_t* src = J.src_u8 + (size_t)l * pitch + x;
-            float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (x + 4 <= in_w) {
-                int i = 0;
-                for (; i + 4 <= n; i += 4) {
-                    unsigned u[4];
+    const int ox0 = (t % J.tiles_x) * kResizeTallW, cols = min(kResizeTallW, J.out_w - ox0);
+    const int y0 = (t / J.tiles_x) * kResizeTallH + wave * 4;
+    const int pitch = J.src_pitch, hn = J.maxtaps;
+    for (int i = threadIdx.x; i < cols * hn; i += kThreads) hw[i] = J.weights[(size_t)ox0 * hn + i];
+    const int lo4 = J.left[ox0] & ~3, nq = (J.left[ox0 + cols - 1] + hn - lo4 + 3) >> 2;  // <= 64
+    const int x = lo4 + 4 * lane;
+    float s[4][4] = {};
+    if (lane < nq && x < J.in_w && y0 < J.out_h) {
+        gbyte_t* src = (gbyte_t*)J.src_u8 + x;
+        const int base = J.vleft[y0];
+        const int vm = J.vmaxtaps;
+        int n[4], sh[4];
+        bool step2 = true, taps12 = vm >= 12;  // windows 2 (or once 3) rows apart; all of 12 rows
 #pragma unroll
-                    for (int k = 0; k < 4; k++) u[k] = *(const unsigned*)(src + (size_t)(i + k) * pitch);
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const float wk = wr[i + k];
-                        float p[4];
-                        cvt4(u[k], p);
-#pragma unroll
-                        for (int c = 0; c < 4; c++) s[c] = mul_add_exact(s[c], p[c], wk);
-                    }
-                }
-                for (; i < n; i++) {
-                    const float wk = wr[i];
-                    float p[4];
-                    cvt4(*(const unsigned*)(src + (size_t)i * pitch), p);
-#pragma unroll
-                    for (int c = 0; c < 4; c++) s[c] = mul_add_exact(s[c], p[c], wk);
-                }
-            } else {  // the quad at the right edge: columns >= in_w are never read back
-                for (int i = 0; i < n; i++) {
-                    const float wk = wr[i];
-#pragma unroll
-                    for (int c = 0; c < 4; c++)
-                        if (x + c < in_w) s[c] = mul_add_exact(s[c], (float)src[(size_t)i * pitch + c], wk);
-                }
-            }
-            *(float4*)&vt[r][4 * q] = make_float4(s[0], s[1], s[2], s[3]);
+        for (int q = 0; q < 4; q++) {
+            const int oy = min(y0 + q, J.out_h - 1);
+            n[q] = J.vcount[oy];
+            sh[q] = J.vleft[oy] - base - 2 * q;
+            step2 = step2 && sh[q] >= 0 && sh[q] + n[q] <= 14;
+            taps12 = taps12 && sh[q] == 0 && n[q] <= 12;
         }
-    }
-    __syncthreads();
-    const int ox = ox0 + threadIdx.x;
-    if (ox >= J.out_w) return;
-    const int l = J.left[ox], n = J.count[ox];
-    const float* wr = J.weights + (size_t)ox * J.maxtaps;
-    float wv[16];  // this column's weights, loaded once for all rows
-    if (n <= 16) {
+        const ctap_t* vw = as_const_taps(J.vweights);
+        if (taps12) {  // the rows of weights are zero past their count
+            float w[4][14];
 #pragma unroll
-        for (int i = 0; i < 16; i++) wv[i] = i < n ? wr[i] : 0.0f;
-    }
-    for (int r = 0; r < nrows; r++) {
-        const float* in = &vt[r][l - lo4];
-        float s = 0.0f;
-        if (n <= 16) {
+            for (int q = 0; q < 4; q++)
 #pragma unroll
-            for (int i = 0; i < 16; i++)
-                if (i < n) s = mul_add_exact(s, in[i], wv[i]);
+                for (int k = 0; k < 12; k++) w[q][k] = vw[min(y0 + q, J.out_h - 1) * vm + k];
+            resize_v_rows<12>(src, pitch, J.in_h, base, w, s);
+        } else if (step2) {
+            float w[4][14];
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int k = 0; k < 14; k++) {
+                    const int i = k - sh[q];
+                    const float v = vw[min(y0 + q, J.out_h - 1) * vm + min(max(i, 0), vm - 1)];
+                    w[q][k] = i >= 0 && i < n[q] ? v : 0.0f;
+                }
+            resize_v_rows<14>(src, pitch, J.in_h, base, w, s);
         } else {
-            for (int i = 0; i < n; i++) s = mul_add_exact(s, in[i], wr[i]);
+            for (int q = 0; q < 4; q++) {
+                const int oy = min(y0 + q, J.out_h - 1);
+                const int l = J.vleft[oy], n = J.vcount[oy];
+                const ctap_t* vw = as_const_taps(J.vweights) + (size_t)oy * J.vmaxtaps;
+                float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                for (int i = 0; i < n; i++) {
+                    const float wk = vw[i];
+                    float p[4];
+                    cvt4(*(__attribute__((address_space(1))) const unsigned*)(src + (size_t)(l + i) * pitch), p);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) a[c] = mul_add_exact(a[c], p[c], wk);
+                }
+#pragma unroll
+                for (int c = 0; c < 4; c++) s[q][c] = a[c];
+            }
         }
-        float c = s < 0.0f ? 0.0f : (s > 255.0f ? 255.0f : s);
-        J.dst[(size_t)(y0 + r) * J.dst_pitch + ox] = (uint8_t)roundf(c);
     }
+#pragma unroll
+    for (int q = 0; q < 4; q++) *(float4*)&vt[wave][q][4 * lane] = make_float4(s[q][0], s[q][1], s[q][2], s[q][3]);
+    __syncthreads();
+    for (int c0 = 0; c0 < cols; c0 += 60) {
+        const int c = c0 + lane;
+        if (lane >= 60 || c >= cols) continue;
+        const int at = J.left[ox0 + c] - lo4;
+        float wv[kTaps];
+#pragma unroll
+        for (int i = 0; i < kTaps; i++)
+            if (i < hn) wv[i] = hw[c * hn + i];
+        float h[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < kTaps; i++) {
+            if (i >= hn) break;
+#pragma unroll
+            for (int q = 0; q < 4; q++) h[q] = mul_add_exact(h[q], vt[wave][q][at + i], wv[i]);
+        }
+        truncating(h);
+        unsigned v[1];
+#pragma unroll
+        for (int q = 0; q < 4; q++) h[q] = __fadd_rn(h[q], 0.5f);
+        v[0] = pack_u8(h[0], h[1], h[2], h[3]);
+        round_even(v);
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (y0 + q < J.out_h)
+                J.dst[(size_t)(y0 + q) * J.dst_pitch + ox0 + c] = (uint8_t)(v[0] >> (8 * q));
+    }
+}
+
+// k_resize_small: tiles of 64 output columns x 4 rows for launches that do not fill
+// the GPU, where a tile's own latency is what counts: one output row per wave, all
+// its loads issued before the first product, and only its own row of LDS, so no
+// barrier. One level of 640 x 480: 15.4 -> 7.4 us (of which about 6 are the launch
+// and its event); 64 of 1920 x 1080 take 430 us, for the weights and texels it
+// loads again for every row.
+__global__ __launch_bounds__(kThreads) void k_resize_small(const ResizeJob* __restrict__ jobs,
+                                                           int njobs) {
+    __shared__ __align__(16) float vt[kResizeSmallH][kResizeSmallSpan];
+    const int tile = xcd_remap(blockIdx.x, gridDim.x);
+    const ResizeJob& J = jobs[find_job(jobs, njobs, tile)];
+    const int t = tile - J.tile_begin;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int oy = (t / J.tiles_x) * kResizeSmallH + wave;
+    if (oy >= J.out_h) return;
+    const int ox0 = (t % J.tiles_x) * kResizeSmallW, ox = ox0 + lane;
+    const int oxc = min(ox, J.out_w - 1), oxl = min(ox0 + kResizeSmallW, J.out_w) - 1;
+    const int pitch = J.src_pitch, hn = J.maxtaps;
+    const int l = J.left[oxc];
+    const int lo4 = J.left[ox0] & ~3, nq = (J.left[oxl] + hn - lo4 + 3) >> 2;  // 4 nq <= kResizeSmallSpan
+    const int vl = J.vleft[oy], vn = J.vcount[oy];
+    const ctap_t* vw = as_const_taps(J.vweights) + (size_t)oy * J.vmaxtaps;
+    const int x = lo4 + 4 * lane;
+    unsigned u[kResizeMaxTaps];
+    gbyte_t* src = (gbyte_t*)J.src_u8 + (size_t)vl * pitch + x;
+    const bool in = lane < nq && x < J.in_w;
+#pragma unroll
+    for (int i = 0; i < kResizeMaxTaps; i++)
+        if (i < vn && in) u[i] = *(__attribute__((address_space(1))) const unsigned*)(src + (size_t)i * pitch);
+    const float* wr = J.weights + (size_t)oxc * hn;
+    float wv[kResizeMaxTaps];
+#pragma unroll
+    for (int i = 0; i < kResizeMaxTaps; i++)
+        if (i < hn) wv[i] = wr[i];
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (in) {
+#pragma unroll
+        for (int i = 0; i < kResizeMaxTaps; i++) {
+            if (i < vn) {
+                const float wk = vw[i];
+                float p[4];
+                cvt4(u[i], p);
+#pragma unroll
+                for (int c = 0; c < 4; c++) s[c] = mul_add_exact(s[c], p[c], wk);
+            }
+        }
+    }
+    if (lane < nq) *(float4*)&vt[wave][4 * lane] = make_float4(s[0], s[1], s[2], s[3]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const float* row = &vt[wave][l - lo4];
+    float h[1] = {0.0f};
+#pragma unroll
+    for (int i = 0; i < kResizeMaxTaps; i++)
+        if (i < hn) h[0] = mul_add_exact(h[0], row[i], wv[i]);
+    truncating(h);
+    h[0] = __fadd_rn(h[0], 0.5f);  // truncated, as the conversion is: rounds half up, exactly
+    if (ox < J.out_w)
+        J.dst[(size_t)oy * J.dst_pitch + ox] = (uint8_t)__builtin_amdgcn_cvt_pk_u8_f32(h[0], 0u, 0u);
 }
 
 }  // namespace
@@ -1238,9 +1341,14 @@ void launch_resize_v(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStr
     hipLaunchKernelGGL(k_resize_v, dim3(total_tiles), dim3(kThreads), 0, s, d_jobs, njobs);
 }
 
-void launch_resize_fused(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s) {
+void launch_resize_tall(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s) {
     if (total_tiles <= 0) return;
-    hipLaunchKernelGGL(k_resize_fused, dim3(total_tiles), dim3(kThreads), 0, s, d_jobs, njobs);
+    hipLaunchKernelGGL(k_resize_tall, dim3(total_tiles), dim3(kThreads), 0, s, d_jobs, njobs);
+}
+
+void launch_resize_small(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s) {
+    if (total_tiles <= 0) return;
+    hipLaunchKernelGGL(k_resize_small, dim3(total_tiles), dim3(kThreads), 0, s, d_jobs, njobs);
 }
 
 void launch_resize_h(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s) {

@@ -49,7 +49,7 @@ struct ResizeJob {
     const int* count;
     const float* weights;   // [out][maxtaps]
     int maxtaps;
-    // the vertical table, for the fused kernel (its left/count/weights are horizontal)
+    // the vertical table, for the kernels of both passes (their left/count/weights are horizontal)
     const int* vleft;
     const int* vcount;
     const float* vweights;
@@ -127,10 +127,13 @@ void launch_blur_v8(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream
 void launch_blur_hv(const BlurJob* d_jobs, int njobs, int total_tiles, bool longer, hipStream_t s);
 void launch_blur_hv_small(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
 void launch_resize_v(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
-// Both Lanczos3 passes in one kernel, the f32 intermediate kept in LDS: for jobs
-// whose every tile of kResizeRows x 256 outputs needs at most kResizeFusedSpan
-// input columns (from left[ox0] rounded down to a multiple of 4).
-void launch_resize_fused(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
+// Both Lanczos3 passes in one kernel, the f32 intermediate kept in LDS, in tiles
+// of kResizeTallW x kResizeTallH or kResizeSmallW x kResizeSmallH outputs: at most
+// kResizeMaxTaps weights per output in either pass, and the windows of a tile's
+// outputs (maxtaps columns from every left) within kResizeTallSpan or
+// kResizeSmallSpan columns of the first left rounded down to a multiple of 4.
+void launch_resize_tall(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
+void launch_resize_small(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
 void launch_resize_h(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
 void launch_copy_level(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
 // Small levels: one output per lane (tiles of 64 x 4). max_taps4 = the largest
@@ -202,10 +205,12 @@ constexpr int kScanTileElems = 4096;
 // descriptor's two lists, then the work-queue counters (kNumXcd each) of
 // k_orient and of the two descriptor instantiations.
 constexpr int kCountExtra = 2 + 3 * kNumXcd;
-// Lanczos3 resize tiles: output rows per work-group of the horizontal and fused
-// kernels, and the input columns the fused kernel stages per tile.
+// Lanczos3 resize tiles: output rows per work-group of the horizontal kernel, and
+// the outputs, input columns and taps of the kernels that make both passes.
 constexpr int kResizeRows = 8;
-constexpr int kResizeFusedSpan = 576;
+constexpr int kResizeMaxTaps = 16;
+constexpr int kResizeTallW = 120, kResizeTallH = 16, kResizeTallSpan = 256;
+constexpr int kResizeSmallW = 64, kResizeSmallH = 4, kResizeSmallSpan = 160;
 // Rows of one extremum-test strip (64 columns wide, tested as bands of 16 rows):
 // kExtStripRows when a launch has at least kExtFillBands bands of 16 rows (enough
 // strips to fill the GPU several times over), else one band per strip.
