@@ -366,7 +366,7 @@ struct LaunchRec {
 
 enum KernelId {
     K_BLUR_H = 0, K_BLUR_V, K_COPY, K_BLUR_H_GENERIC, K_RESIZE_V, K_RESIZE_H, K_EXTREMA, K_SCAN,
-    K_COMPACT, K_REFINE, K_ORIENT, K_DESCRIPTOR, K_FINALIZE, K_BLUR_V_NARROW, K_BLUR_V_GENERIC,
+    K_COMPACT, K_REFINE, K_ORIENT, K_DESCRIPTOR, K_BLUR_V_NARROW, K_BLUR_V_GENERIC,
     K_BLUR_H2, K_BLUR_H_SMALL, K_BLUR_V_SMALL, K_LUMA, K_DESC_U8, K_RESIZE_TALL, K_BLUR_V_SMALL8,
     K_BLUR_H16, K_BLUR_V8, K_BLUR_HV, K_BLUR_HV_LONG, K_BLUR_HV_SMALL, K_RESIZE_SMALL,
     K_COUNT
@@ -375,7 +375,7 @@ enum KernelId {
 const char* const kKernelNames[K_COUNT] = {
     "k_blur_h<8>", "k_blur_v<4>", "k_copy_level", "k_blur_h_generic", "k_resize_v", "k_resize_h",
     "k_extrema_tile", "k_scan", "k_compact", "k_refine", "k_orient", "k_descriptor",
-    "k_finalize", "k_blur_v_narrow", "k_blur_v_generic", "k_blur_h<2>", "k_blur_h_small",
+    "k_blur_v_narrow", "k_blur_v_generic", "k_blur_h<2>", "k_blur_h_small",
     "k_blur_v_small", "k_luma", "k_desc_u8", "k_resize_tall", "k_blur_v_small8", "k_blur_h<16>",
     "k_blur_v<8>", "k_blur_hv<false>", "k_blur_hv<true>", "k_blur_hv_small",
     "k_resize_small"};
@@ -752,7 +752,11 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     const int kcap = B.ext ? (int)std::min<size_t>(B.ext->kcap, INT_MAX / 512) : (int)kp_cap;
 
     const size_t bits_off = C.take((size_t)std::max<long long>(nbits, 1) * 8);
-    const size_t counts_off = C.take((size_t)(nslots + kCountExtra) * 4);  // + lists and queue heads
+    // the row-slot counts (+ lists and queue heads): zeros uploaded with the job blob
+    // when there are few, else zeroed by a kernel
+    const size_t counts_bytes = (size_t)(nslots + kCountExtra) * 4;
+    const bool counts_in_blob = !B.ext && nslots <= kCompactScanMax;
+    const size_t counts_off = counts_in_blob ? 0 : C.take(counts_bytes);
     const size_t offs_off = C.take((size_t)(nslots + 2) * 4);
     const size_t scantmp1_off = C.take((size_t)(nslots / kScanTileElems + 4) * 4);
     const size_t cand_off = C.take((size_t)cap * sizeof(Cand));
@@ -803,7 +807,8 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     const size_t max_jobs = (size_t)n * ((1 + (size_t)maxO * Lmax) * 2 + (size_t)maxO * 2);
     const size_t blob_bound = max_launches * 256 + max_jobs * std::max(sizeof(BlurJob), sizeof(ResizeJob)) +
                               octs.size() * sizeof(OctaveDesc) + (size_t)n * sizeof(ImageParams) +
-                              (size_t)(n + 1) * sizeof(int) + 4096;
+                              (size_t)(n + 1) * sizeof(int) + 4096 +
+                              (counts_in_blob ? counts_bytes : 0);
     const size_t blob_dev_off = round_up(C.off, 256);
     if (B.ext && blob_dev_off + blob_bound > B.ext->cap)
         return fail(SIFT_ERR_NOMEM, "batch needs " + std::to_string(blob_dev_off + blob_bound) +
@@ -1117,6 +1122,8 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     const size_t isb_blob = blob_take((n + 1) * sizeof(int));
     memcpy(blob.data() + isb_blob, img_slot_begin.data(), (n + 1) * sizeof(int));
 
+    const size_t counts_blob = counts_in_blob ? blob_take(counts_bytes) : 0;  // zeros
+
     if (blob.size() > blob_bound) return fail(SIFT_ERR_DEVICE, "internal: job blob bound exceeded");
 
     hipStream_t st = stream;
@@ -1175,7 +1182,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     char* D = A + blob_dev_off;
     const OctaveDesc* d_oct = (const OctaveDesc*)(D + oct_blob);
     const ImageParams* d_par = (const ImageParams*)(D + par_blob);
-    unsigned* d_counts = (unsigned*)AP(counts_off);
+    unsigned* d_counts = counts_in_blob ? (unsigned*)(D + counts_blob) : (unsigned*)AP(counts_off);
     unsigned* d_offs = (unsigned*)AP(offs_off);
     Cand* d_cand = (Cand*)AP(cand_off);
     Keypoint* d_ref = (Keypoint*)AP(ref_off);
@@ -1187,6 +1194,10 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     float* d_desc = B.ext ? B.ext->desc : (float*)AP(desc_off);
     unsigned* d_sum = (unsigned*)AP(summary_off);
     unsigned* d_total = d_offs + nslots;
+
+    int max_radius = 0;
+    for (int i = 0; i < n; i++)
+        max_radius = std::max(max_radius, descriptor_max_radius(B.params[i].sigma, (int)B.params[i].num_intervals));
 
     // Every launch of the batch, in order. Kernel arguments are arena addresses
     // and scalars of this layout; the per-call data (images, taps) is read from
@@ -1255,17 +1266,14 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         if (tile_ext)
             launch_extrema_tile(S0, strip_rows, d_oct, noct, total_tiles, d_par,
                                 (unsigned long long*)AP(bits_off),
-                                d_counts, nslots, st);
+                                d_counts, nslots, counts_in_blob, st);
         else
             launch_extrema(d_oct, noct, total_rows, d_par, (unsigned long long*)AP(bits_off), d_counts,
-                           nslots, st);
+                           nslots, counts_in_blob, st);
         prof_end(K_EXTREMA, ext_bytes, ev);
-        prof_begin(K_SCAN, 0.0, &ev);
-        launch_scan_dev(d_counts, nslots, nullptr, d_offs, (unsigned*)AP(scantmp1_off), st);
-        prof_end(K_SCAN, 0.0, ev);
         prof_begin(K_COMPACT, 0.0, &ev);
         launch_compact(d_oct, noct, nslots, (const unsigned long long*)AP(bits_off), d_counts, d_offs,
-                       d_cand, cap, st);
+                       (unsigned*)AP(scantmp1_off), d_cand, cap, st);
         prof_end(K_COMPACT, 0.0, ev);
         prof_begin(K_REFINE, 0.0, &ev);
         launch_refine(d_oct, d_par, d_cand, d_total, cap, d_ref, d_valid,
@@ -1276,17 +1284,14 @@ int Context::run(const Batch& B, RunOutputs* outs) {
                       d_counts + nslots + 2, st);  // kNumXcd queue counters
         prof_end(K_ORIENT, 0.0, ev);
         prof_begin(K_SCAN, 0.0, &ev);
-        launch_scan_dev(d_npk, cap, d_total, d_koff, (unsigned*)AP(scantmp2_off), st);
+        launch_keypoint_offsets(d_npk, cap, d_total, d_koff, (unsigned*)AP(scantmp2_off), d_offs,
+                                (const int*)(D + isb_blob), n, d_sum, B.ext ? B.ext->offsets : nullptr, st);
         prof_end(K_SCAN, 0.0, ev);
         prof_begin(K_DESCRIPTOR, 0.0, &ev);
         launch_descriptor(d_oct, d_par, d_cand, d_total, cap, d_ref, d_npk, d_ang, d_koff, kcap, d_kps,
                           d_desc, d_counts + nslots, (int*)AP(wide_off), d_counts + nslots + 1,
-                          (int*)AP(mid_off), d_counts + nslots + 2 + kNumXcd, st);
+                          (int*)AP(mid_off), d_counts + nslots + 2 + kNumXcd, max_radius, st);
         prof_end(K_DESCRIPTOR, 0.0, ev);
-        prof_begin(K_FINALIZE, 0.0, &ev);
-        launch_finalize(d_offs, (const int*)(D + isb_blob), n, d_koff, d_total, cap, d_sum,
-                        B.ext ? B.ext->offsets : nullptr, st);
-        prof_end(K_FINALIZE, 0.0, ev);
         if (B.desc_u8) {
             prof_begin(K_DESC_U8, 0.0, &ev);
             launch_desc_u8(d_desc, d_sum + 1, kcap, (uint8_t*)AP(descu8_off), st);
@@ -1310,7 +1315,8 @@ int Context::run(const Batch& B, RunOutputs* outs) {
                                      oct_blob, par_blob, isb_blob, bits_off, counts_off, offs_off,
                                      scantmp1_off, cand_off, candresp_off, ref_off, valid_off, npk_off,
                                      ang_off, koff_off, scantmp2_off, kps_off, desc_off, summary_off,
-                                     wide_off, mid_off, (uint64_t)B.desc_u8, descu8_off};
+                                     wide_off, mid_off, (uint64_t)B.desc_u8, descu8_off, counts_blob,
+                                     (uint64_t)max_radius};
         for (const LaunchRec& L : launches) {
             key.push_back((uint64_t)L.kind << 32 | (uint32_t)L.njobs);
             key.push_back(L.job_off);

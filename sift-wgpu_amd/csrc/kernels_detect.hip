@@ -12,6 +12,8 @@
 // formed without it by q255f, or read from an LDS table of it in the row-wise
 // extremum and wide-window kernels), which is bit-identical to the reference's
 // (G_{s+1} as f32 / 255.0) - (G_s as f32 / 255.0) (src/sift.rs:97,120).
+#include <math.h>
+
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -430,6 +432,46 @@ __device__ __forceinline__ int scan_n(int n_static, const unsigned* n_dev) {
     return (int)min(v, (unsigned)n_static);
 }
 
+// The 16 elements of a thread, from base on (a multiple of 16; the arrays start on
+// 256-byte boundaries): four 16-byte accesses where all lie below n. As 16 guarded
+// words every access of a wave touched 64 lines.
+__device__ __forceinline__ void scan_load16(const unsigned* __restrict__ in, int base, int n,
+                                            unsigned (&v)[16]) {
+    if (base + 16 <= n) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint4 u = *reinterpret_cast<const uint4*>(in + base + 4 * i);
+            v[4 * i] = u.x;
+            v[4 * i + 1] = u.y;
+            v[4 * i + 2] = u.z;
+            v[4 * i + 3] = u.w;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = (base + i < n) ? in[base + i] : 0u;
+    }
+}
+// Writes the exclusive prefixes of v, run before them, and returns their end.
+__device__ __forceinline__ unsigned scan_store16(unsigned* __restrict__ out, int base, int n,
+                                                 const unsigned (&v)[16], unsigned run) {
+    unsigned o[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        o[i] = run;
+        run += v[i];
+    }
+    if (base + 16 <= n) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            *reinterpret_cast<uint4*>(out + base + 4 * i) = make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; i++)
+            if (base + i < n) out[base + i] = o[i];
+    }
+    return run;
+}
+
 __global__ __launch_bounds__(kThreads) void k_scan_reduce(const unsigned* __restrict__ in, int n_max,
                                                           const unsigned* n_dev,
                                                           unsigned* __restrict__ tile_sums) {
@@ -468,31 +510,56 @@ __global__ __launch_bounds__(kThreads) void k_scan_down(const unsigned* __restri
     const int base = blockIdx.x * kScanTile + threadIdx.x * 16;
     unsigned v[16];
     unsigned s = 0;
+    scan_load16(in, base, n, v);
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        v[i] = (base + i < n) ? in[base + i] : 0u;
-        s += v[i];
-    }
+    for (int i = 0; i < 16; i++) s += v[i];
     unsigned tot;
     unsigned ex = block_excl_scan(s, sh, tot);
-    unsigned run = tile_prefix[blockIdx.x] + ex;
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        if (base + i < n) out[base + i] = run;
-        run += v[i];
-        if (base + i == n - 1) out[n] = run;
-    }
+    const unsigned end = scan_store16(out, base, n, v, tile_prefix[blockIdx.x] + ex);
+    if (base < n && base + 16 >= n) out[n] = end;
     if (n == 0 && blockIdx.x == 0 && threadIdx.x == 0) out[0] = 0;
 }
 
-// The same scan in one work-group of 1024 threads, for small n_max (single
+// Per-image keypoint ranges: summary[2+i] = koff[first candidate of image i]
+// (and out_offsets[i], when given); summary[0] = total candidates (may exceed
+// cap), summary[1] = total keypoints.
+struct FinalizeArgs {
+    const unsigned* slot_offsets;
+    const int* img_slot_begin;
+    int nimg;
+    const unsigned* koff;
+    const unsigned* total;
+    int cap;
+    unsigned* summary;
+    unsigned* out_offsets;
+};
+__device__ __forceinline__ void finalize_entry(const FinalizeArgs& F, int i) {
+    const unsigned n = min(*F.total, (unsigned)F.cap);
+    const unsigned cb = min(F.slot_offsets[F.img_slot_begin[i]], n);
+    const unsigned k = F.koff[cb];
+    F.summary[2 + i] = k;
+    if (F.out_offsets) F.out_offsets[i] = k;
+    if (i == 0) {
+        F.summary[0] = *F.total;
+        F.summary[1] = F.koff[n];
+    }
+}
+
+__global__ void k_finalize(FinalizeArgs F) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i <= F.nimg) finalize_entry(F, i);
+}
+
+// The same scan in one work-group of 1024 threads, for few elements (single
 // frames, small batches): 16384-element chunks with a running carry, one
-// launch instead of three.
+// launch instead of three. The keypoint offsets' scan (F.summary set) writes the
+// per-image ranges too, which needs every offset and here is one barrier away
+// instead of one launch (4 us on a single frame).
 constexpr int kScanSingleThreads = 1024;
 constexpr int kScanSingleMax = 1 << 16;
 __global__ __launch_bounds__(kScanSingleThreads) void k_scan_single(const unsigned* __restrict__ in,
                                                                    int n_max, const unsigned* n_dev,
-                                                                   unsigned* __restrict__ out) {
+                                                                   unsigned* out, FinalizeArgs F) {
     __shared__ unsigned sh[kScanSingleThreads / 64];
     const int n = scan_n(n_max, n_dev);
     unsigned carry = 0;
@@ -500,21 +567,20 @@ __global__ __launch_bounds__(kScanSingleThreads) void k_scan_single(const unsign
         const int base = b + threadIdx.x * 16;
         unsigned v[16];
         unsigned s = 0;
+        scan_load16(in, base, n, v);
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            v[i] = (base + i < n) ? in[base + i] : 0u;
-            s += v[i];
-        }
+        for (int i = 0; i < 16; i++) s += v[i];
         unsigned tot;
-        unsigned run = carry + block_excl_scan(s, sh, tot);
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            if (base + i < n) out[base + i] = run;
-            run += v[i];
-        }
+        const unsigned ex = block_excl_scan(s, sh, tot);
+        scan_store16(out, base, n, v, carry + ex);
         carry += tot;
     }
     if (threadIdx.x == 0) out[n] = carry;
+    if (F.summary) {
+        __threadfence_block();
+        __syncthreads();  // the offsets just written are read back
+        for (int i = threadIdx.x; i <= F.nimg; i += kScanSingleThreads) finalize_entry(F, i);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -527,6 +593,10 @@ __global__ __launch_bounds__(kScanSingleThreads) void k_scan_single(const unsign
 // their loads overlap. For each slot the set bits are ranked with popcounts and
 // a wave prefix sum and the candidates written at offsets[slot] + rank, i.e. in
 // the reference's order. Rows of more than 64 words take a chunked loop.
+// kScan: the work-group sums the counts of all slots before its own itself and
+// writes its slots' offsets (and the total), which saves the scan its launch: a
+// single frame's few thousand counts lie in L2 (1920 x 1080: 25 KB, 13 KB per
+// work-group on average), where the scan in one work-group took 5 to 10 us.
 // ---------------------------------------------------------------------------
 constexpr int kCompactSlots = 8;
 
@@ -558,18 +628,53 @@ __device__ __forceinline__ void compact_word(unsigned long long m, int wi, int j
     base += tot;
 }
 
+template <bool kScan>
 __global__ __launch_bounds__(kThreads) void k_compact(const OctaveDesc* __restrict__ oct, int noct,
                                                       int nslots,
                                                       const unsigned long long* __restrict__ bits,
                                                       const unsigned* __restrict__ counts,
-                                                      const unsigned* __restrict__ offsets,
+                                                      unsigned* __restrict__ offsets,
                                                       Cand* __restrict__ cand, int cap, int spw) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int s0 = (blockIdx.x * (kThreads / 64) + wave) * spw;
-    if (s0 >= nslots) return;
     const int ns = min(spw, nslots - s0);
-    const unsigned cnt_l = lane < ns ? counts[s0 + lane] : 0u;
-    const unsigned off_l = lane < ns ? offsets[s0 + lane] : 0u;
+    unsigned cnt_l, off_l;
+    if constexpr (kScan) {
+        __shared__ unsigned wsum[kThreads / 64];
+        const int per = (kThreads / 64) * spw, first = blockIdx.x * per;  // slots of the work-group, <= 64
+        unsigned p = 0;
+        for (int i = threadIdx.x * 4; i < first; i += kThreads * 4) {  // first is a multiple of 4
+            const uint4 v = *reinterpret_cast<const uint4*>(counts + i);
+            p += (v.x + v.y) + (v.z + v.w);
+        }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) p += __shfl_xor(p, d, 64);
+        if (lane == 0) wsum[wave] = p;
+        const int slot = first + lane;
+        const bool mine = lane < per && slot < nslots;
+        const unsigned c = mine ? counts[slot] : 0u;
+        unsigned x = c;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned t = __shfl_up(x, d, 64);
+            if (lane >= d) x += t;
+        }
+        __syncthreads();
+        x += (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+        if (wave == 0 && mine) {
+            offsets[slot] = x - c;
+            if (slot == nslots - 1) offsets[nslots] = x;
+        }
+        const int at = wave * spw + lane;
+        cnt_l = __shfl(c, at & 63, 64);
+        off_l = __shfl(x - c, at & 63, 64);
+        if (lane >= ns) cnt_l = 0u;
+        if (s0 >= nslots) return;
+    } else {
+        if (s0 >= nslots) return;
+        cnt_l = lane < ns ? counts[s0 + lane] : 0u;
+        off_l = lane < ns ? offsets[s0 + lane] : 0u;
+    }
     const unsigned long long any = ballot64(cnt_l != 0u);
     if (any == 0ull) return;
     // each slot's octave (the slots are ordered by octave)
@@ -1719,25 +1824,6 @@ __global__ __launch_bounds__(kThreads) void k_descriptor_wide(
     }
 }
 
-// Per-image keypoint ranges: summary[2+i] = koff[first candidate of image i]
-// (and out_offsets[i], when given); summary[0] = total candidates (may exceed
-// cap), summary[1] = total keypoints.
-__global__ void k_finalize(const unsigned* __restrict__ slot_offsets,
-                           const int* __restrict__ img_slot_begin, int nimg,
-                           const unsigned* __restrict__ koff, const unsigned* __restrict__ total,
-                           int cap, unsigned* __restrict__ summary, unsigned* __restrict__ out_offsets) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i > nimg) return;
-    const unsigned n = min(*total, (unsigned)cap);
-    const unsigned cb = min(slot_offsets[img_slot_begin[i]], n);
-    summary[2 + i] = koff[cb];
-    if (out_offsets) out_offsets[i] = koff[cb];
-    if (i == 0) {
-        summary[0] = *total;
-        summary[1] = koff[n];
-    }
-}
-
 // u8 descriptors of the WebGPU backends (src/shaders/descriptor.wgsl:256-262):
 // trunc(clamp(d * 512, 0, 255)) of each value, 4 values per lane.
 __device__ __forceinline__ unsigned desc_u8_of(float d) {
@@ -1759,9 +1845,10 @@ __global__ __launch_bounds__(256) void k_desc_u8(const float4* __restrict__ desc
 }  // namespace
 
 void launch_extrema(const OctaveDesc* d_oct, int noct, int total_rows, const ImageParams* d_params,
-                    unsigned long long* d_bits, unsigned* d_counts, int nslots, hipStream_t s) {
+                    unsigned long long* d_bits, unsigned* d_counts, int nslots, bool zeroed, hipStream_t s) {
     // the counters after the row-slot counts (the descriptor's lists, the work queues)
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, d_counts + nslots, kCountExtra, 0u);
+    if (!zeroed)
+        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, d_counts + nslots, kCountExtra, 0u);
     if (total_rows <= 0) return;
     hipLaunchKernelGGL(k_extrema, dim3(total_rows), dim3(kThreads), 0, s, d_oct, noct, d_params,
                        d_bits, d_counts);
@@ -1771,10 +1858,11 @@ bool extrema_tile_supported(int S) { return S >= 1 && S <= 6; }
 
 void launch_extrema_tile(int S, int strip_rows, const OctaveDesc* d_oct, int noct, int total_tiles,
                          const ImageParams* d_params, unsigned long long* d_bits, unsigned* d_counts,
-                         int nslots, hipStream_t s) {
+                         int nslots, bool zeroed, hipStream_t s) {
     // the row-slot counts and the counters after them (the descriptor's lists, the work queues)
-    hipLaunchKernelGGL(k_fill_u32, dim3((nslots + kCountExtra + 255) / 256), dim3(256), 0, s, d_counts,
-                       nslots + kCountExtra, 0u);
+    if (!zeroed)
+        hipLaunchKernelGGL(k_fill_u32, dim3((nslots + kCountExtra + 255) / 256), dim3(256), 0, s, d_counts,
+                           nslots + kCountExtra, 0u);
     if (total_tiles <= 0) return;
     switch (S) {
 #define SH_EXT(SS) \
@@ -1787,29 +1875,48 @@ void launch_extrema_tile(int S, int strip_rows, const OctaveDesc* d_oct, int noc
 }
 
 // n_dev may be null (then n_max is the count). out needs n_max+1 entries;
-// tmp needs ceil(n_max/4096)+1 entries.
-void launch_scan_dev(const unsigned* d_in, int n_max, const unsigned* n_dev, unsigned* d_out,
-                     unsigned* d_tmp, hipStream_t s) {
+// tmp needs ceil(n_max/4096)+1 entries. Returns whether fin (may be null) was done.
+static bool scan(const unsigned* d_in, int n_max, const unsigned* n_dev, unsigned* d_out,
+                 unsigned* d_tmp, const FinalizeArgs* fin, hipStream_t s) {
     if (n_max <= kScanSingleMax) {
         hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(kScanSingleThreads), 0, s, d_in, n_max, n_dev,
-                           d_out);
-        return;
+                           d_out, fin ? *fin : FinalizeArgs{});
+        return true;
     }
     const int tiles = n_max > 0 ? (n_max + kScanTile - 1) / kScanTile : 1;
     hipLaunchKernelGGL(k_scan_reduce, dim3(tiles), dim3(kThreads), 0, s, d_in, n_max, n_dev, d_tmp);
     hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kThreads), 0, s, d_tmp, tiles);
     hipLaunchKernelGGL(k_scan_down, dim3(tiles), dim3(kThreads), 0, s, d_in, n_max, n_dev, d_tmp,
                        d_out);
+    return false;
 }
 
 void launch_compact(const OctaveDesc* d_oct, int noct, int nslots, const unsigned long long* d_bits,
-                    const unsigned* d_counts, const unsigned* d_offsets, Cand* d_cand, int cap,
+                    const unsigned* d_counts, unsigned* d_offsets, unsigned* d_tmp, Cand* d_cand, int cap,
                     hipStream_t s) {
+    if (nslots > 0 && nslots <= kCompactScanMax) {
+        // slots per wave: enough that the work-groups' reads of the counts before
+        // theirs stay a few MB in all (12756 slots of 3840 x 2160: 10 MB)
+        const int spw = nslots <= 2048 ? 1 : nslots <= 4096 ? 2 : nslots <= 8192 ? 4 : 8;
+        const int per = (kThreads / 64) * spw;
+        hipLaunchKernelGGL(k_compact<true>, dim3((nslots + per - 1) / per), dim3(kThreads), 0, s, d_oct,
+                           noct, nslots, d_bits, d_counts, d_offsets, d_cand, cap, spw);
+        return;
+    }
+    (void)scan(d_counts, nslots, nullptr, d_offsets, d_tmp, nullptr, s);
     if (nslots <= 0) return;
     const int spw = nslots >= 65536 ? kCompactSlots : 1;  // slots per wave
     const int per = (kThreads / 64) * spw;                 // slots per work-group
-    hipLaunchKernelGGL(k_compact, dim3((nslots + per - 1) / per), dim3(kThreads), 0, s, d_oct, noct,
+    hipLaunchKernelGGL(k_compact<false>, dim3((nslots + per - 1) / per), dim3(kThreads), 0, s, d_oct, noct,
                        nslots, d_bits, d_counts, d_offsets, d_cand, cap, spw);
+}
+
+void launch_keypoint_offsets(const unsigned* d_npeaks, int cap, const unsigned* d_total, unsigned* d_koff,
+                             unsigned* d_tmp, const unsigned* d_slot_offsets, const int* d_img_slot_begin,
+                             int nimg, unsigned* d_summary, unsigned* d_out_offsets, hipStream_t s) {
+    const FinalizeArgs F{d_slot_offsets, d_img_slot_begin, nimg, d_koff, d_total, cap, d_summary, d_out_offsets};
+    if (!scan(d_npeaks, cap, d_total, d_koff, d_tmp, &F, s))
+        hipLaunchKernelGGL(k_finalize, dim3((nimg + 1 + 255) / 256), dim3(256), 0, s, F);
 }
 
 static int grid_for(int cap, int per_block, int max_blocks) {
@@ -1873,7 +1980,7 @@ void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, con
                        const unsigned* d_npeaks, const float* d_angles, const unsigned* d_koff,
                        int kcap, Keypoint* d_kps, float* d_desc, unsigned* d_wide_count,
                        int* d_wide_list, unsigned* d_mid_count, int* d_mid_list, unsigned* d_queues,
-                       hipStream_t s) {
+                       int max_radius, hipStream_t s) {
     // as k_orient: a work queue, or few keypoints per work-group. Windows up to
     // kDescSmallR run at 8 work-groups per CU and list the few others for the
     // kDescMaxR instantiation (6 per CU), which lists still wider ones for
@@ -1891,9 +1998,10 @@ void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, con
                            d_params, d_cand, d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap,
                            d_kps, d_desc, nullptr, nullptr, d_wide_count, d_wide_list,
                            q ? d_queues + kNumXcd : nullptr);
-        hipLaunchKernelGGL(k_descriptor_wide, dim3(256), dim3(kThreads), 0, s, d_oct, d_params, d_cand,
-                           d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap, d_kps, d_desc,
-                           d_wide_count, d_wide_list);
+        if (max_radius > kDescMaxR)
+            hipLaunchKernelGGL(k_descriptor_wide, dim3(256), dim3(kThreads), 0, s, d_oct, d_params, d_cand,
+                               d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap, d_kps, d_desc,
+                               d_wide_count, d_wide_list);
         return;
     }
     const void* k28 = (const void*)k_descriptor<kDescSmallR, false>;
@@ -1903,20 +2011,23 @@ void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, con
     hipLaunchKernelGGL((k_descriptor<kDescSmallR, false>), dim3(g28), dim3(kThreads), 0, s, d_oct,
                        d_params, d_cand, d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap,
                        d_kps, d_desc, nullptr, nullptr, d_mid_count, d_mid_list, q ? d_queues : nullptr);
+    if (max_radius <= kDescSmallR) return;
     hipLaunchKernelGGL((k_descriptor<kDescMaxR, true>), dim3(g31), dim3(kThreads), 0, s, d_oct,
                        d_params, d_cand, d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap,
                        d_kps, d_desc, d_mid_count, d_mid_list, d_wide_count, d_wide_list,
                        q ? d_queues + kNumXcd : nullptr);
-    hipLaunchKernelGGL(k_descriptor_wide, dim3(256), dim3(kThreads), 0, s, d_oct, d_params, d_cand,
-                       d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap, d_kps, d_desc,
-                       d_wide_count, d_wide_list);
+    if (max_radius > kDescMaxR)
+        hipLaunchKernelGGL(k_descriptor_wide, dim3(256), dim3(kThreads), 0, s, d_oct, d_params, d_cand,
+                           d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap, d_kps, d_desc,
+                           d_wide_count, d_wide_list);
 }
 
-void launch_finalize(const unsigned* d_slot_offsets, const int* d_img_slot_begin, int nimg,
-                     const unsigned* d_koff, const unsigned* d_total, int cap, unsigned* d_summary,
-                     unsigned* d_out_offsets, hipStream_t s) {
-    hipLaunchKernelGGL(k_finalize, dim3((nimg + 1 + 255) / 256), dim3(256), 0, s, d_slot_offsets,
-                       d_img_slot_begin, nimg, d_koff, d_total, cap, d_summary, d_out_offsets);
+// A keypoint's octave sigma is sigma * 2^(l / S) with l, its refined layer, below
+// S + 0.5 (the refinement keeps layers 1 .. S and offsets below 0.5), and its
+// descriptor radius the ceiling of 12 sqrt(1/2) of that; 1e-4 for the roundings.
+int descriptor_max_radius(float sigma, int intervals) {
+    const double so = (double)sigma * exp2(1.0 + 0.5 / intervals);
+    return (int)ceil(std::min(so * 6.0 * sqrt(2.0) * 1.0001, 1e9));
 }
 
 void launch_desc_u8(const float* d_desc, const unsigned* d_count, int kcap, uint8_t* d_out,

@@ -152,18 +152,26 @@ void launch_luma(const LumaJob* d_jobs, int njobs, int total_tiles, hipStream_t 
 void launch_blur_v_generic(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
 
 void launch_extrema(const OctaveDesc* d_oct, int noct, int total_rows, const ImageParams* d_params,
-                    unsigned long long* d_bits, unsigned* d_counts, int nslots, hipStream_t s);
+                    unsigned long long* d_bits, unsigned* d_counts, int nslots, bool zeroed, hipStream_t s);
 // Tiled extremum scan (64x16 tiles) for S in [1, 6]: zeroes the row-slot
-// counts, then one workgroup per tile; OctaveDesc.row_begin holds the tile prefix.
+// counts (and the kCountExtra after them) unless they are zeroed already, then one
+// workgroup per tile; OctaveDesc.row_begin holds the tile prefix.
 bool extrema_tile_supported(int S);
 void launch_extrema_tile(int S, int strip_rows, const OctaveDesc* d_oct, int noct, int total_tiles,
                          const ImageParams* d_params, unsigned long long* d_bits, unsigned* d_counts,
-                         int nslots, hipStream_t s);
-void launch_scan_dev(const unsigned* d_in, int n_max, const unsigned* n_dev, unsigned* d_out,
-                     unsigned* d_tmp, hipStream_t s);
+                         int nslots, bool zeroed, hipStream_t s);
+// Candidates from the bitmask: the slots' offsets (nslots + 1 entries, the last the
+// total) and the compaction. d_tmp: ceil(nslots / 4096) + 1 entries.
 void launch_compact(const OctaveDesc* d_oct, int noct, int nslots, const unsigned long long* d_bits,
-                    const unsigned* d_counts, const unsigned* d_offsets, Cand* d_cand, int cap,
+                    const unsigned* d_counts, unsigned* d_offsets, unsigned* d_tmp, Cand* d_cand, int cap,
                     hipStream_t s);
+// Keypoint offsets (exclusive sums of the candidates' peak counts) and the
+// summary: summary[0] = candidates, summary[1] = keypoints, summary[2..2+nimg] =
+// per-image keypoint offsets (nimg+1 entries), the offsets also to
+// d_out_offsets when it is not null. d_tmp: ceil(cap / 4096) + 1 entries.
+void launch_keypoint_offsets(const unsigned* d_npeaks, int cap, const unsigned* d_total, unsigned* d_koff,
+                             unsigned* d_tmp, const unsigned* d_slot_offsets, const int* d_img_slot_begin,
+                             int nimg, unsigned* d_summary, unsigned* d_out_offsets, hipStream_t s);
 void launch_refine(const OctaveDesc* d_oct, const ImageParams* d_params, const Cand* d_cand,
                    const unsigned* d_total, int cap, Keypoint* d_ref, int* d_valid,
                    float* d_cand_resp, hipStream_t s);
@@ -178,13 +186,10 @@ void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, con
                        const unsigned* d_npeaks, const float* d_angles, const unsigned* d_koff,
                        int kcap, Keypoint* d_kps, float* d_desc, unsigned* d_wide_count,
                        int* d_wide_list, unsigned* d_mid_count, int* d_mid_list, unsigned* d_queues,
-                       hipStream_t s);
-// Writes summary[0] = candidates, summary[1] = keypoints, summary[2..2+nimg] =
-// per-image keypoint offsets (nimg+1 entries), the offsets also to
-// d_out_offsets when it is not null.
-void launch_finalize(const unsigned* d_slot_offsets, const int* d_img_slot_begin, int nimg,
-                     const unsigned* d_koff, const unsigned* d_total, int cap,
-                     unsigned* d_summary, unsigned* d_out_offsets, hipStream_t s);
+                       int max_radius, hipStream_t s);
+// An upper bound of the descriptor radius of any keypoint with these parameters
+// (launch_descriptor's max_radius: instantiations for larger windows are left out).
+int descriptor_max_radius(float sigma, int intervals);
 // u8 descriptors of the WebGPU backends: out = trunc(clamp(d * 512, 0, 255)) for
 // the first min(*d_count, kcap) descriptors.
 void launch_desc_u8(const float* d_desc, const unsigned* d_count, int kcap, uint8_t* d_out,
@@ -201,6 +206,10 @@ constexpr int kSmallMaxRows = 128;
 // 11.2 KB + 50 KB of LDS, within 64 KB whatever jobs share a launch.
 constexpr int kSmallMaxRows8 = 800;
 constexpr int kScanTileElems = 4096;
+// Slots up to which the compaction makes its own scan, and up to which the
+// counters come zeroed with the job blob (64 KB of zeros at most, about 1 us of
+// its copy, instead of a fill kernel's launch).
+constexpr int kCompactScanMax = 16384;
 // Counters after the extremum row-slot counts, zeroed with them: the
 // descriptor's two lists, then the work-queue counters (kNumXcd each) of
 // k_orient and of the two descriptor instantiations.
