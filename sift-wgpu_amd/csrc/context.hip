@@ -359,7 +359,7 @@ struct LaunchRec {
     int kind;        // KernelId
     size_t job_off;  // offset in the job blob
     int njobs, tiles, max_pad;
-    int variant;     // k_blur_h: outputs per lane; k_blur_v_narrow: staged rows
+    int variant;     // k_blur_h: outputs per lane; k_blur_v_narrow: staged rows; k_blur_deep: LDS bytes
     double bytes;    // algorithmic HBM bytes of the launch
     double ops;      // f32 operations the reference's arithmetic prescribes (profile ops)
 };
@@ -369,7 +369,7 @@ enum KernelId {
     K_COMPACT, K_REFINE, K_ORIENT, K_DESCRIPTOR, K_BLUR_V_NARROW, K_BLUR_V_GENERIC,
     K_BLUR_H2, K_BLUR_H_SMALL, K_BLUR_V_SMALL, K_LUMA, K_DESC_U8, K_RESIZE_TALL, K_BLUR_V_SMALL8,
     K_BLUR_H16, K_BLUR_V8, K_BLUR_HV, K_BLUR_HV_LONG, K_BLUR_HV_SMALL, K_RESIZE_SMALL,
-    K_COUNT
+    K_BLUR_DEEP, K_COUNT
 };
 // Names as rocprofv3 reports the kernels (template arguments included).
 const char* const kKernelNames[K_COUNT] = {
@@ -378,10 +378,13 @@ const char* const kKernelNames[K_COUNT] = {
     "k_blur_v_narrow", "k_blur_v_generic", "k_blur_h<2>", "k_blur_h_small",
     "k_blur_v_small", "k_luma", "k_desc_u8", "k_resize_tall", "k_blur_v_small8", "k_blur_h<16>",
     "k_blur_v<8>", "k_blur_hv<false>", "k_blur_hv<true>", "k_blur_hv_small",
-    "k_resize_small"};
+    "k_resize_small", "k_blur_deep"};
 
 bool is_resize_both(int kind) { return kind == K_RESIZE_TALL || kind == K_RESIZE_SMALL; }
-bool is_blur_hv(int kind) { return kind == K_BLUR_HV || kind == K_BLUR_HV_LONG || kind == K_BLUR_HV_SMALL; }
+// a blur kernel that makes both passes
+bool is_blur_hv(int kind) {
+    return kind == K_BLUR_HV || kind == K_BLUR_HV_LONG || kind == K_BLUR_HV_SMALL || kind == K_BLUR_DEEP;
+}
 
 
 double blur_job_bytes(const BlurJob& j, int kind) {
@@ -527,6 +530,18 @@ void blur_hv_tiles(BlurJob& J, bool large) {
     const int tw = large ? kHvTileW : kHvSmallW, th = large ? kHvTileH : kHvSmallH;
     J.tiles_x = (J.w + tw - 1) / tw;
     J.tiles = J.tiles_x * ((J.h + th - 1) / th);
+}
+
+// A step's blurs of more taps go to k_blur_deep while its tiles hold at most this
+// many products together (64 levels of 80 x 60, 101 taps, 62 M: 16.0 against 22.1 us
+// of the best pair; one of 960 x 540, 41 taps, 54 M: 17.0 against 16.7; 64 of
+// 120 x 67, 199 taps, 205 M: 36.5 against 33.7) and each one at most this many
+// (240 x 135, 199 taps, 0.43 M: 18.8 against 19.6; 120 x 67, 395 taps, 0.42 M: 22.6
+// against 21.4).
+constexpr double kDeepStepWork = 60e6, kDeepTileWork = 0.4e6;
+bool blur_deep_valid(int h, int ntaps) {
+    return ntaps > kHvMaxTaps && deep_tile_work(h, ntaps) <= kDeepTileWork &&
+           deep_lds_bytes(h, ntaps) <= (size_t)kDeepMaxLds;
 }
 
 // Tile counts of a job in a form.
@@ -799,11 +814,11 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         maxO = std::max(maxO, (int)shapes[i].size());
         Lmax = std::max(Lmax, (int)B.params[i].num_intervals + 3);
     }
-    // per blur step up to 15 blur launches (three fused, five H forms, six V forms,
-    // the copy) and 3 Lanczos3 launches; at most 1 + maxO * Lmax steps. One image
-    // has at most three octaves in a step, with two launches each (the server's
-    // frame_device_bytes counts 15 per frame).
-    const size_t max_launches = (size_t)(1 + maxO * Lmax) * (n == 1 ? 15 : 18) + (size_t)maxO * 3 + 8;
+    // per blur step up to 16 blur launches (four of both passes, five H forms, six V
+    // forms, the copy) and 3 Lanczos3 launches; at most 1 + maxO * Lmax steps. One
+    // image has at most three octaves in a step, with two launches each (the
+    // server's frame_device_bytes counts 15 per frame).
+    const size_t max_launches = (size_t)(1 + maxO * Lmax) * (n == 1 ? 15 : 19) + (size_t)maxO * 3 + 8;
     const size_t max_jobs = (size_t)n * ((1 + (size_t)maxO * Lmax) * 2 + (size_t)maxO * 2);
     const size_t blob_bound = max_launches * 256 + max_jobs * std::max(sizeof(BlurJob), sizeof(ResizeJob)) +
                               octs.size() * sizeof(OctaveDesc) + (size_t)n * sizeof(ImageParams) +
@@ -831,6 +846,12 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     auto AP = [&](size_t off) { return A + off; };
 
     std::vector<BlurJob> hj, hj2, hj16, hgj, hsj, vj, v8j, vnj, vgj, vsj, vs8j, cj, hvj;
+    struct DeepJob {
+        BlurJob job;
+        uint8_t* tmp;
+        int tmp_pitch;
+    };
+    std::vector<DeepJob> dpj;
     const std::pair<int, int> forced = blur_forced();
     int vn_rows = 0, hs_taps4 = 0, vs_taps4 = 0, vs_rows = 0, vs8_taps4 = 0, vs8_rows = 0;
 
@@ -860,6 +881,54 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         size_t off = blob_take(jobs.size() * sizeof(jobs[0]));
         memcpy(blob.data() + off, jobs.data(), jobs.size() * sizeof(jobs[0]));
         launches.push_back({kind, off, (int)jobs.size(), tiles, max_pad, variant, bytes, ops});
+    };
+
+    // the two one-pass jobs of a blur through tmp; V: the whole blur but its source
+    auto push_two_pass = [&](const uint8_t* src, int src_pitch, uint8_t* tmp, int tmp_pitch, BlurJob V) {
+        const std::pair<int, int> form =
+            blur_choice(V.w, V.h, V.ntaps, V.ntaps_pad, n >= kTuneManyJobs, forced);
+        const int n4 = (V.ntaps + 3) & ~3, r = V.ntaps / 2;
+        BlurJob H = V;
+        H.dog = nullptr;
+        H.prev = nullptr;
+        H.dog_pitch = 0;
+        H.src = src;
+        H.src_pitch = src_pitch;
+        H.dst = tmp;
+        H.dst_pitch = tmp_pitch;
+        blur_h_tiles(H, form.first);
+        switch (form.first) {
+            case BH_W8: hj.push_back(H); break;
+            case BH_W16: hj16.push_back(H); break;
+            case BH_W2: hj2.push_back(H); break;
+            case BH_SMALL:
+                hsj.push_back(H);
+                hs_taps4 = std::max(hs_taps4, n4);
+                break;
+            default: hgj.push_back(H); break;
+        }
+        V.src = tmp;
+        V.src_pitch = tmp_pitch;
+        blur_v_tiles(V, form.second);
+        switch (form.second) {
+            case BV_WIDE: vj.push_back(V); break;
+            case BV_WIDE8: v8j.push_back(V); break;
+            case BV_NARROW:
+                vnj.push_back(V);
+                vn_rows = std::max(vn_rows, std::min(V.h, 16 + 2 * r));
+                break;
+            case BV_SMALL:
+                vsj.push_back(V);
+                vs_taps4 = std::max(vs_taps4, n4);
+                vs_rows = std::max(vs_rows, std::min(V.h, 4 + 2 * r));
+                break;
+            case BV_SMALL8:
+                vs8j.push_back(V);
+                vs8_taps4 = std::max(vs8_taps4, n4);
+                vs8_rows = std::max(vs8_rows, std::min(V.h, 4 + 2 * r));
+                break;
+            default: vgj.push_back(V); break;
+        }
     };
 
     auto make_blur_pair = [&](const uint8_t* src, int src_pitch, uint8_t* tmp, int tmp_pitch,
@@ -892,59 +961,27 @@ int Context::run(const Batch& B, RunOutputs* outs) {
             hvj.push_back(J);  // its tiles: flush_blur
             return;
         }
-        const std::pair<int, int> form = blur_choice(w, h, R.ntaps, R.npad, n >= kTuneManyJobs, forced);
-        const int n4 = (R.ntaps + 3) & ~3, r = R.ntaps / 2;
-        BlurJob H = J;
-        H.src = src;
-        H.src_pitch = src_pitch;
-        H.dst = tmp;
-        H.dst_pitch = tmp_pitch;
-        blur_h_tiles(H, form.first);
-        switch (form.first) {
-            case BH_W8: hj.push_back(H); break;
-            case BH_W16: hj16.push_back(H); break;
-            case BH_W2: hj2.push_back(H); break;
-            case BH_SMALL:
-                hsj.push_back(H);
-                hs_taps4 = std::max(hs_taps4, n4);
-                break;
-            default: hgj.push_back(H); break;
+        if (!dog && forced.first < 0 && forced.second < 0 && blur_deep_valid(h, R.ntaps)) {
+            J.src = src;
+            J.src_pitch = src_pitch;
+            J.dst = dst;
+            J.dst_pitch = dst_pitch;
+            J.tiles_x = (w + kDeepW - 1) / kDeepW;
+            J.tiles = J.tiles_x * deep_tiles_y(h, R.ntaps);
+            dpj.push_back({J, tmp, tmp_pitch});  // deep or two passes: flush_blur
+            return;
         }
         BlurJob V = J;
-        V.src = tmp;
-        V.src_pitch = tmp_pitch;
         V.dst = dst;
         V.dst_pitch = dst_pitch;
         V.dog = dog;
         V.prev = prev;
         V.dog_pitch = dog_pitch;
-        blur_v_tiles(V, form.second);
-        switch (form.second) {
-            case BV_WIDE: vj.push_back(V); break;
-            case BV_WIDE8: v8j.push_back(V); break;
-            case BV_NARROW:
-                vnj.push_back(V);
-                vn_rows = std::max(vn_rows, std::min(h, 16 + 2 * r));
-                break;
-            case BV_SMALL:
-                vsj.push_back(V);
-                vs_taps4 = std::max(vs_taps4, n4);
-                vs_rows = std::max(vs_rows, std::min(h, 4 + 2 * r));
-                break;
-            case BV_SMALL8:
-                vs8j.push_back(V);
-                vs8_taps4 = std::max(vs8_taps4, n4);
-                vs8_rows = std::max(vs8_rows, std::min(h, 4 + 2 * r));
-                break;
-            default: vgj.push_back(V); break;
-        }
+        push_two_pass(src, src_pitch, tmp, tmp_pitch, V);
     };
 
     auto flush_blur = [&]() {
         int maxpad = 0, maxpad2 = 0, maxpad16 = 0;
-        for (auto& j : hj) maxpad = std::max(maxpad, j.ntaps_pad);
-        for (auto& j : hj2) maxpad2 = std::max(maxpad2, j.ntaps_pad);
-        for (auto& j : hj16) maxpad16 = std::max(maxpad16, j.ntaps_pad);
         std::vector<BlurJob> hv[3];  // large tiles with short and long tap counts, small tiles
         double step_px = 0.0;
         for (const BlurJob& j : hvj) step_px += (double)j.w * j.h;
@@ -956,6 +993,23 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         push_launch(K_BLUR_HV, hv[0], 0, 0);
         push_launch(K_BLUR_HV_LONG, hv[1], 0, 0);
         push_launch(K_BLUR_HV_SMALL, hv[2], 0, 0);
+        std::vector<BlurJob> deep;
+        double deep_work = 0.0;
+        int deep_lds = 0;
+        for (const DeepJob& d : dpj) deep_work += d.job.tiles * deep_tile_work(d.job.h, d.job.ntaps);
+        for (const DeepJob& d : dpj) {
+            if (deep_work <= kDeepStepWork) {
+                deep.push_back(d.job);
+                deep_lds = std::max(deep_lds, (int)deep_lds_bytes(d.job.h, d.job.ntaps));
+            } else {
+                push_two_pass(d.job.src, d.job.src_pitch, d.tmp, d.tmp_pitch, d.job);
+            }
+        }
+        dpj.clear();
+        push_launch(K_BLUR_DEEP, deep, 0, deep_lds);
+        for (auto& j : hj) maxpad = std::max(maxpad, j.ntaps_pad);
+        for (auto& j : hj2) maxpad2 = std::max(maxpad2, j.ntaps_pad);
+        for (auto& j : hj16) maxpad16 = std::max(maxpad16, j.ntaps_pad);
         push_launch(K_BLUR_H16, hj16, maxpad16, 16);
         push_launch(K_BLUR_H, hj, maxpad, 8);
         push_launch(K_BLUR_H2, hj2, maxpad2, 2);
@@ -1215,6 +1269,9 @@ int Context::run(const Batch& B, RunOutputs* outs) {
                     break;
                 case K_BLUR_V: launch_blur_v((const BlurJob*)(D + L.job_off), L.njobs, L.tiles, 0, st); break;
                 case K_BLUR_V8: launch_blur_v8((const BlurJob*)(D + L.job_off), L.njobs, L.tiles, st); break;
+                case K_BLUR_DEEP:
+                    launch_blur_deep((const BlurJob*)(D + L.job_off), L.njobs, L.tiles, L.variant, st);
+                    break;
                 case K_BLUR_HV:
                 case K_BLUR_HV_LONG:
                     launch_blur_hv((const BlurJob*)(D + L.job_off), L.njobs, L.tiles, L.kind == K_BLUR_HV_LONG, st);

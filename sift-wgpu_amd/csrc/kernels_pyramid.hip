@@ -10,6 +10,8 @@
 // in tap order with separate multiply and add (no FMA; the file is compiled with
 // -ffp-contract=off and uses __fmul_rn/__fadd_rn), then truncates to u8 -- the
 // reference's arithmetic, so the levels are bit-identical to it.
+#include <algorithm>
+
 #include "sift_hip.h"
 #include "sift_internal.h"
 
@@ -856,6 +858,76 @@ __global__ __launch_bounds__(kThreads) void k_blur_v_small8(const BlurJob* __res
     blur_v_small_tile<uint8_t>(jobs, njobs, max_taps4, sm8);
 }
 
+// ---------------------------------------------------------------------------
+// Both passes of a long blur on a small level in one kernel (the deep octaves of
+// single frames and small batches: a few thousand pixels, dozens to hundreds of
+// taps). A work-group of 1024 threads makes a tile of kDeepW columns and up to
+// kDeepH rows (the level cut evenly). Its source rows, at most the level's, and
+// the replicated columns its windows need are staged as f32; the horizontal sums
+// of those rows go to LDS, the rows past the image are copies of the first and the
+// last, and the vertical sums read them: both are the same loop of one tap value
+// for all lanes, one input, a multiply and an add, without a bound in it.
+// Bound: latency (a wave alone on its SIMD issues every 8 cycles, four waves share
+// 2.5), so one output per lane and narrow tiles, whose extra horizontal rows cost
+// nothing while CUs are idle. Per level, with about 6 us of launch and event (two
+// of them in a pair of launches): 160 x 120, 51 taps 13.0 -> 8.8 us; 80 x 60, 101 taps
+// 15.6 -> 8.5; 40 x 30, 199 taps 15.4 -> 9.6; 240 x 135, 101 taps 15.5 -> 12.4. The
+// host keeps the one-pass forms where the tiles fill the GPU (64 levels of
+// 240 x 135, 51 taps: 53 against 37 us) or one tile is long (120 x 67, 395 taps: 22.6
+// against 21.4 us).
+// ---------------------------------------------------------------------------
+// Sum of the taps (padded with zeros to n4, a multiple of 4) over in[k * step].
+__device__ __forceinline__ float deep_sum(const float* in, int step, const float* tp, int n4) {
+    float acc = 0.0f;
+#pragma unroll 4
+    for (int k = 0; k < n4; k += 4) {
+        const float4 t4 = *reinterpret_cast<const float4*>(tp + k);
+        acc = mul_add_exact(acc, in[k * step], t4.x);
+        acc = mul_add_exact(acc, in[(k + 1) * step], t4.y);
+        acc = mul_add_exact(acc, in[(k + 2) * step], t4.z);
+        acc = mul_add_exact(acc, in[(k + 3) * step], t4.w);
+    }
+    return acc;
+}
+
+__global__ __launch_bounds__(kDeepThreads) void k_blur_deep(const BlurJob* __restrict__ jobs, int njobs) {
+    extern __shared__ __align__(16) float dsm[];
+    const int tile = xcd_remap(blockIdx.x, gridDim.x);
+    const BlurJob& J = jobs[find_job(jobs, njobs, tile)];
+    const int t = tile - J.tile_begin, tid = threadIdx.x;
+    const int w = J.w, h = J.h, n = J.ntaps, r = n >> 1, n4 = (n + 3) & ~3;
+    const int tiles_y = J.tiles / J.tiles_x, th = (h + tiles_y - 1) / tiles_y;
+    const int x0 = (t % J.tiles_x) * kDeepW, y0 = (t / J.tiles_x) * th;
+    const int rows = min(th, h - y0);
+    if (rows <= 0) return;
+    const int rlo = max(y0 - r, 0), nr = min(y0 + rows + r, h) - rlo;
+    const int segw = kDeepW + n4, stride = deep_stride(n4);
+    float* const tp = dsm;
+    float* const seg = dsm + n4;             // source rows rlo.., columns x0 - r.. (clamped)
+    float* const ext = seg + nr * stride;    // horizontal sums of rows y0 - r.. (clamped), kDeepW wide
+    for (int i = tid; i < n4; i += kDeepThreads) tp[i] = i < n ? J.taps[i] : 0.0f;
+    const float inv = 1.0f / (float)segw;
+    for (int i = tid; i < nr * segw; i += kDeepThreads) {
+        const int rr = (int)(((float)i + 0.5f) * inv), c = i - rr * segw;
+        seg[rr * stride + c] = (float)J.src[(size_t)(rlo + rr) * J.src_pitch + min(max(x0 - r + c, 0), w - 1)];
+    }
+    __syncthreads();
+    const int col = tid % kDeepW, first = rlo - (y0 - r);  // row rlo's place in ext
+    for (int rr = tid / kDeepW; rr < nr; rr += kDeepThreads / kDeepW)
+        ext[(first + rr) * kDeepW + col] = (float)u8_trunc(deep_sum(seg + rr * stride + col, 1, tp, n4));
+    __syncthreads();
+    for (int i = tid; i < (rows + n4) * kDeepW; i += kDeepThreads) {  // the rows past the image's
+        const int e = i / kDeepW;
+        if (e < first) ext[i] = ext[first * kDeepW + col];
+        else if (e >= first + nr) ext[i] = ext[(first + nr - 1) * kDeepW + col];
+    }
+    __syncthreads();
+    for (int y = tid / kDeepW; y < rows; y += kDeepThreads / kDeepW)
+        if (x0 + col < w)
+            J.dst[(size_t)(y0 + y) * J.dst_pitch + x0 + col] =
+                (uint8_t)u8_trunc(deep_sum(ext + y * kDeepW + col, kDeepW, tp, n4));
+}
+
 // Exact thread-per-pixel passes for kernels too wide for the LDS row tile.
 __global__ __launch_bounds__(kThreads) void k_blur_h_generic(const BlurJob* __restrict__ jobs,
                                                              int njobs) {
@@ -1289,6 +1361,33 @@ void launch_blur_hv(const BlurJob* d_jobs, int njobs, int total_tiles, bool long
 void launch_blur_hv_small(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s) {
     if (total_tiles <= 0) return;
     hipLaunchKernelGGL(k_blur_hv_small, dim3(total_tiles), dim3(kThreads), 0, s, d_jobs, njobs);
+}
+
+int deep_tiles_y(int h, int ntaps) {
+    const int r = ntaps / 2, least = (h + kDeepH - 1) / kDeepH;
+    constexpr int pass = kDeepThreads / kDeepW;  // rows of one horizontal pass
+    for (int ty = least; (h + ty - 1) / ty >= 32; ty++)
+        if (std::min(h, (h + ty - 1) / ty + 2 * r) <= pass) return ty;
+    return least;
+}
+
+size_t deep_lds_bytes(int h, int ntaps) {
+    const int ty = deep_tiles_y(h, ntaps), th = (h + ty - 1) / ty;
+    const size_t n4 = (size_t)((ntaps + 3) & ~3), nr = (size_t)std::min(h, th + 2 * (ntaps / 2));
+    return 4 * (n4 + nr * (size_t)deep_stride((int)n4) + (th + n4) * kDeepW);
+}
+
+double deep_tile_work(int h, int ntaps) {
+    const int ty = deep_tiles_y(h, ntaps), th = (h + ty - 1) / ty;
+    return (double)(std::min(h, th + 2 * (ntaps / 2)) + th) * kDeepW * ntaps;
+}
+
+void launch_blur_deep(const BlurJob* d_jobs, int njobs, int total_tiles, int lds, hipStream_t s) {
+    if (total_tiles <= 0) return;
+    // past the 64 KB a launch may ask for by default
+    if (lds > 65536)
+        (void)hipFuncSetAttribute((const void*)k_blur_deep, hipFuncAttributeMaxDynamicSharedMemorySize, kDeepMaxLds);
+    hipLaunchKernelGGL(k_blur_deep, dim3(total_tiles), dim3(kDeepThreads), lds, s, d_jobs, njobs);
 }
 
 void launch_blur_h_small(const BlurJob* d_jobs, int njobs, int total_tiles, int max_taps4,

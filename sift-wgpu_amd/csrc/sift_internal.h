@@ -126,6 +126,15 @@ void launch_blur_v8(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream
 // kHvSmallW x kHvSmallH tiles of any of them.
 void launch_blur_hv(const BlurJob* d_jobs, int njobs, int total_tiles, bool longer, hipStream_t s);
 void launch_blur_hv_small(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
+// Both passes in one kernel for long tap counts on small levels, without the DoG
+// epilogue: tiles of kDeepW columns x 1/deep_tiles_y of the level's rows (cut to
+// need one horizontal pass where tiles of 32 rows or more do), lds = the largest
+// deep_lds_bytes of the launch's jobs (at most kDeepMaxLds); deep_tile_work: the
+// products of a tile.
+int deep_tiles_y(int h, int ntaps);
+size_t deep_lds_bytes(int h, int ntaps);
+double deep_tile_work(int h, int ntaps);
+void launch_blur_deep(const BlurJob* d_jobs, int njobs, int total_tiles, int lds, hipStream_t s);
 void launch_resize_v(const ResizeJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
 // Both Lanczos3 passes in one kernel, the f32 intermediate kept in LDS, in tiles
 // of kResizeTallW x kResizeTallH or kResizeSmallW x kResizeSmallH outputs: at most
@@ -197,6 +206,11 @@ void launch_desc_u8(const float* d_desc, const unsigned* d_count, int kcap, uint
 // The fused blur: its tap counts and tiles.
 constexpr int kHvMinTaps = 5, kHvShortTaps = 15, kHvMaxTaps = 33;
 constexpr int kHvTileW = 256, kHvTileH = 64, kHvSmallW = 64, kHvSmallH = 16;
+// The fused blur of deep levels: tile, threads, dynamic LDS limit. Its staged rows are
+// deep_stride(n4) floats apart: 8 modulo 64, so that the 8 rows x 8 columns a wave
+// reads at one tap fall in distinct banks.
+constexpr int kDeepW = 8, kDeepH = 128, kDeepThreads = 1024, kDeepMaxLds = 160 * 1024;
+__host__ __device__ constexpr int deep_stride(int n4) { return (kDeepW + n4 + 55) / 64 * 64 + 8; }
 // Max padded tap count handled by the LDS row-tile horizontal pass.
 constexpr int kMaxHPad = 3576;
 // Small-level kernels: taps (rounded up to 4) and staged rows they accept.
