@@ -1738,11 +1738,23 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
 // ---------------------------------------------------------------------------
 // k_descriptor_wide: keypoints whose window exceeds the LDS patch
 // (R > 31, sigma_octave > 3.65; none with the default sigma and 3 intervals).
-// Direct per-sample path with global reads and the reference's f32 arithmetic;
-// 256 contiguous chunks of the (2R+1)^2 window as in k_descriptor. The fixed-point
-// scale drops below 2^20 when a copy would see more than kMaxCopySamples samples,
-// and is raised by the gain of the largest |gx|, |gy| of the window's samples.
+// The reference's f32 arithmetic per sample; 256 contiguous chunks of the (2R+1)^2
+// window as in k_descriptor. The fixed-point scale drops below 2^20 when a copy
+// would see more than kMaxCopySamples samples, and is raised by the gain of the
+// largest |gx|, |gy| of the window's samples.
+// Every sample takes four bilinear values, and the samples' points lie on one grid
+// (x_o + i, y_o + j), so the values of windows up to R = kWideGridR are made once
+// into LDS, from column and row tables, and a gradient is four reads instead of 16
+// gathers and 12 lerps, in the pass over the gradients' maximum and in every peak.
+// x_s + 1 and x_s - 1 are f32 sums of their own: where one is not the grid's
+// column (past a power of two the column's fraction loses a bit the sum kept),
+// the column is marked and that value formed directly. Two frames of 1023 x 767 at
+// sigma 2.0 (2.4 thousand wide windows): 811 -> 233 us.
 // ---------------------------------------------------------------------------
+constexpr int kWideGridR = 47;
+constexpr int kWideGS = 2 * kWideGridR + 3;
+constexpr int kWideGroups = 2048;  // of which three fit a CU at once; each takes few windows
+
 __global__ __launch_bounds__(kThreads) void k_descriptor_wide(
     const OctaveDesc* __restrict__ oct, const ImageParams* __restrict__ params,
     const Cand* __restrict__ cand, const unsigned* __restrict__ total, int cap,
@@ -1753,6 +1765,13 @@ __global__ __launch_bounds__(kThreads) void k_descriptor_wide(
     __shared__ float q[256];
     __shared__ __align__(16) unsigned hist[kHistCopies * kHistWords];
     __shared__ float wave_gmax[kThreads / 64];
+    __shared__ float grid[kWideGS * kWideGS];
+    // per grid column / row: the two clamped texel positions and the fraction
+    __shared__ int c0[kWideGS], c1[kWideGS], r0[kWideGS], r1[kWideGS];
+    __shared__ float cd[kWideGS], rd[kWideGS];
+    // sample column / row t - 1: bit 0, its -1 neighbour is not grid t - 1; bit 1, its
+    // +1 neighbour is not grid t + 1
+    __shared__ unsigned char cmark[kWideGS], rmark[kWideGS];
     fill_q(q);
     __syncthreads();
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -1762,25 +1781,69 @@ __global__ __launch_bounds__(kThreads) void k_descriptor_wide(
     for (int i = blockIdx.x; i < nw; i += gridDim.x) {
         const int c = wide_list[i];
         const DescGeom G = desc_geom(c, oct, params, cand, ref, npeaks, koff);
-        const int R = G.R, side = G.side, nsamp = side * side;
+        const int R = G.R, side = G.side, nsamp = side * side, gside = side + 2;
         const float wm1 = (float)(G.w - 1), hm1 = (float)(G.h - 1);
         const int per = (nsamp + kThreads - 1) / kThreads;
         const int i0 = (lane * 4 + wave) * per;
         const int iend = min(i0 + per, nsamp);
+        const bool on_grid = R <= kWideGridR;
+        if (on_grid) {
+            if (tid < gside || (tid >= 128 && tid < 128 + gside)) {
+                const bool is_row = tid >= 128;
+                const int t = is_row ? tid - 128 : tid;
+                const float o = is_row ? G.yo : G.xo;
+                const int last = (is_row ? G.h : G.w) - 1;
+                const float x = o + (float)(t - 1 - R), xf = floorf(x);
+                (is_row ? r0 : c0)[t] = min(max(f2i_sat(xf), 0), last);
+                (is_row ? r1 : c1)[t] = min(max(f2i_sat(xf + 1.0f), 0), last);
+                (is_row ? rd : cd)[t] = x - xf;
+                (is_row ? rmark : cmark)[t] = (unsigned char)((x - 1.0f != o + (float)(t - 2 - R) ? 1 : 0) |
+                                                              (x + 1.0f != o + (float)(t - R) ? 2 : 0));
+            }
+            __syncthreads();
+            const float inv = 1.0f / (float)gside;
+            for (int k = tid; k < gside * gside; k += kThreads) {
+                const int gy = (int)(((float)k + 0.5f) * inv), gx = k - gy * gside;
+                const float dx = cd[gx], dy = rd[gy];
+                const uint8_t* const g0 = G.g + (size_t)r0[gy] * G.pitch;
+                const uint8_t* const g1 = G.g + (size_t)r1[gy] * G.pitch;
+                const float q11 = q[g0[c0[gx]]], q21 = q[g0[c1[gx]]];
+                const float q12 = q[g1[c0[gx]]], q22 = q[g1[c1[gx]]];
+                grid[gy * kWideGS + gx] = q11 * (1.0f - dx) * (1.0f - dy) + q21 * dx * (1.0f - dy) +
+                                          q12 * (1.0f - dx) * dy + q22 * dx * dy;
+            }
+            __syncthreads();
+        }
+        // the gradient of sample (cx, cy) at (xs, ys)
+        auto gradient = [&](int cx, int cy, float xs, float ys, float& gx, float& gy) {
+            if (on_grid && (cmark[cx + 1] | rmark[cy + 1]) == 0) {
+                const float* p = grid + cy * kWideGS + cx;
+                gx = p[kWideGS + 2] - p[kWideGS];
+                gy = p[2 * kWideGS + 1] - p[1];
+            } else {
+                gx = bilinear(G.g, G.pitch, G.w, G.h, xs + 1.0f, ys, q) -
+                     bilinear(G.g, G.pitch, G.w, G.h, xs - 1.0f, ys, q);
+                gy = bilinear(G.g, G.pitch, G.w, G.h, xs, ys + 1.0f, q) -
+                     bilinear(G.g, G.pitch, G.w, G.h, xs, ys - 1.0f, q);
+            }
+        };
         {
             // the largest |gx|, |gy| of the in-image samples sets the keypoint's
             // fixed-point gain (written per wave, read after the first barrier of
             // the peak loop)
             float gm = 0.0f;
-            for (int i = i0; i < iend && G.np > 0; i++) {
-                const int cy = i / side, cx = i - cy * side;
+            int cy = i0 / side, cx = i0 - cy * side;
+            for (int k = i0; k < iend && G.np > 0; k++) {
                 const float xs = G.xo + (float)(cx - R), ys = G.yo + (float)(cy - R);
-                if (xs < 0.0f || xs >= wm1 || ys < 0.0f || ys >= hm1) continue;
-                const float gx = bilinear(G.g, G.pitch, G.w, G.h, xs + 1.0f, ys, q) -
-                                 bilinear(G.g, G.pitch, G.w, G.h, xs - 1.0f, ys, q);
-                const float gy = bilinear(G.g, G.pitch, G.w, G.h, xs, ys + 1.0f, q) -
-                                 bilinear(G.g, G.pitch, G.w, G.h, xs, ys - 1.0f, q);
-                gm = fmaxf(gm, fmaxf(fabsf(gx), fabsf(gy)));
+                if (!(xs < 0.0f || xs >= wm1 || ys < 0.0f || ys >= hm1)) {
+                    float gx, gy;
+                    gradient(cx, cy, xs, ys, gx, gy);
+                    gm = fmaxf(gm, fmaxf(fabsf(gx), fabsf(gy)));
+                }
+                if (++cx == side) {
+                    cx = 0;
+                    cy++;
+                }
             }
             gm = wave_max(gm);
             if (lane == 0) wave_gmax[wave] = gm;
@@ -1795,8 +1858,12 @@ __global__ __launch_bounds__(kThreads) void k_descriptor_wide(
             const float gmax = fmaxf(fmaxf(wave_gmax[0], wave_gmax[1]), fmaxf(wave_gmax[2], wave_gmax[3]));
             const float fix = kDescFix * fminf(1.0f, (float)kMaxCopySamples / (float)(128 * per)) *
                               desc_fix_gain(gmax, 1.0f);
-            for (int i = i0; i < iend; i++) {
-                const int cy = i / side, cx = i - cy * side;
+            int cy = i0 / side, cx = i0 - cy * side - 1;
+            for (int k = i0; k < iend; k++) {
+                if (++cx == side) {
+                    cx = 0;
+                    cy++;
+                }
                 const float py = (float)(cy - R), px = (float)(cx - R);
                 const float rx = ca * px + sa * py;
                 const float ry = -sa * px + ca * py;
@@ -1805,14 +1872,15 @@ __global__ __launch_bounds__(kThreads) void k_descriptor_wide(
                 if (!(xb > -1.0f && xb < 4.0f && yb > -1.0f && yb < 4.0f)) continue;
                 const float xs = G.xo + px, ys = G.yo + py;
                 if (xs < 0.0f || xs >= wm1 || ys < 0.0f || ys >= hm1) continue;
-                const float gx = bilinear(G.g, G.pitch, G.w, G.h, xs + 1.0f, ys, q) -
-                                 bilinear(G.g, G.pitch, G.w, G.h, xs - 1.0f, ys, q);
-                const float gy = bilinear(G.g, G.pitch, G.w, G.h, xs, ys + 1.0f, q) -
-                                 bilinear(G.g, G.pitch, G.w, G.h, xs, ys - 1.0f, q);
+                float gx, gy;
+                gradient(cx, cy, xs, ys, gx, gy);
                 const float wt = expf(-(px * px + py * py) / G.denom);
                 const float mag = sqrtf(gx * gx + gy * gy);
-                const float pa = atan2f(gy, gx);
-                const float ar = rem_euclid(pa - angle, kTwoPi);
+                // rem_euclid(d, 2 pi): |d| <= 2 pi, so its remainder is d itself, or a
+                // zero of its sign at the ends
+                const float d = atan2f(gy, gx) - angle;
+                const float m = fabsf(d) < kTwoPi ? d : copysignf(0.0f, d);
+                const float ar = m < 0.0f ? m + kTwoPi : m;
                 desc_scatter(hw, xb, yb, ar * 8.0f / kTwoPi, mag * wt * fix);
             }
             __syncthreads();
@@ -1999,7 +2067,7 @@ void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, con
                            d_kps, d_desc, nullptr, nullptr, d_wide_count, d_wide_list,
                            q ? d_queues + kNumXcd : nullptr);
         if (max_radius > kDescMaxR)
-            hipLaunchKernelGGL(k_descriptor_wide, dim3(256), dim3(kThreads), 0, s, d_oct, d_params, d_cand,
+            hipLaunchKernelGGL(k_descriptor_wide, dim3(kWideGroups), dim3(kThreads), 0, s, d_oct, d_params, d_cand,
                                d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap, d_kps, d_desc,
                                d_wide_count, d_wide_list);
         return;
@@ -2017,7 +2085,7 @@ void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, con
                        d_kps, d_desc, d_mid_count, d_mid_list, d_wide_count, d_wide_list,
                        q ? d_queues + kNumXcd : nullptr);
     if (max_radius > kDescMaxR)
-        hipLaunchKernelGGL(k_descriptor_wide, dim3(256), dim3(kThreads), 0, s, d_oct, d_params, d_cand,
+        hipLaunchKernelGGL(k_descriptor_wide, dim3(kWideGroups), dim3(kThreads), 0, s, d_oct, d_params, d_cand,
                            d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap, d_kps, d_desc,
                            d_wide_count, d_wide_list);
 }
