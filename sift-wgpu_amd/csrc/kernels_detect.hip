@@ -46,6 +46,9 @@ __device__ __forceinline__ float rem_euclid(float x, float m) {
 }
 
 __device__ __forceinline__ float pow2f(int o) { return ldexpf(1.0f, o); }
+// x / 2^o, exactly the IEEE division by that power (x is 0 or far from the
+// denormals), in one instruction instead of about ten
+__device__ __forceinline__ float over_pow2(float x, int o) { return __builtin_amdgcn_ldexpf(x, -o); }
 
 // atan2 for the gradient angles: octant reduction a = min(|x|,|y|)/max(|x|,|y|),
 // atan(a) = a * P(a^2) with P a degree-8 least-squares (Lawson-reweighted)
@@ -1230,26 +1233,28 @@ constexpr int kMaxCopySamples = 2048;           // per-copy sample bound that ke
 // below 2^32 (at most kMaxCopySamples samples of at most sqrt(2) * fix + 1/2
 // each), so the low word never carries into the high word.
 //
-// desc_bins: the bin pair address of one sample (its spatial neighbour 0), its
-// four spatial weights t_k and its angle fraction da; ab, the angle in bins, may
-// be anywhere in (-8, 8): its integer part is taken mod 8.
-__device__ __forceinline__ unsigned long long* desc_bins(unsigned* hcopy, float xb, float yb,
-                                                         float ab, float m, float (&tt)[4],
-                                                         float& da) {
+// desc_bins: the bin pair address of one sample (its spatial neighbour 0), as a byte
+// offset, its four spatial weights t_k and its angle fraction da; ab, the angle in
+// bins, may be anywhere in (-8, 8): its integer part is taken mod 8. hbytes: the
+// byte offset of the copy's cell (0, 0), as f32 (whole numbers below 2^24, exact).
+// The pair of bin a lies at byte 4 a + 36 (a & 1) of its cell: one v_perm picks that
+// from eight bytes.
+__device__ __forceinline__ unsigned desc_bins(float hbytes, float xb, float yb, float ab, float m,
+                                              float (&tt)[4], float& da) {
     const float xf = floorf(xb), yf = floorf(yb), af = floorf(ab);
     const unsigned ai = ((unsigned)(int)af) & 7u;
     const float dx = xb - xf, dy = yb - yf;
     da = ab - af;
-    // cell (xf, yf) of the padded 6 x 6 grid: 7 * kCellWords + the offset below
-    const unsigned cw =
-        (unsigned)(int)__builtin_fmaf(yf, 6.0f * kCellWords, xf * (float)kCellWords);
+    static_assert(kOddBase == 9 && kCellWords == 18, "the bytes below");
+    const unsigned pair = __builtin_amdgcn_perm(0x40183810u, 0x30082800u, ai);  // 0, 40, 8, 48, 16, 56, 24, 64
+    const unsigned cell = (unsigned)(int)__builtin_fmaf(
+        yf, 6.0f * 4.0f * kCellWords, __builtin_fmaf(xf, 4.0f * kCellWords, hbytes));
     const float t0 = m * (1.0f - dx), t1 = m * dx;
     tt[0] = t0 * (1.0f - dy);
     tt[1] = t1 * (1.0f - dy);
     tt[2] = t0 * dy;
     tt[3] = t1 * dy;
-    return reinterpret_cast<unsigned long long*>(hcopy + 7 * kCellWords +
-                                                 (cw + ai + __umul24(ai & 1u, (unsigned)kOddBase)));
+    return cell + pair;
 }
 
 // Adds four pairs of fixed-point sums (a[2k], a[2k+1]) at the spatial
@@ -1268,7 +1273,8 @@ __device__ __forceinline__ void desc_add_pairs(unsigned long long* base, const f
 __device__ __forceinline__ void desc_scatter(unsigned* hcopy, float xb, float yb, float ab,
                                              float m) {
     float tt[4], da;
-    unsigned long long* const base = desc_bins(hcopy, xb, yb, ab, m, tt, da);
+    unsigned long long* const base = reinterpret_cast<unsigned long long*>(
+        reinterpret_cast<char*>(hcopy) + desc_bins(7.0f * 4.0f * kCellWords, xb, yb, ab, m, tt, da));
     const float a[8] = {tt[0] * (1.0f - da), tt[0] * da, tt[1] * (1.0f - da), tt[1] * da,
                         tt[2] * (1.0f - da), tt[2] * da, tt[3] * (1.0f - da), tt[3] * da};
     desc_add_pairs(base, a);
@@ -1297,11 +1303,13 @@ __device__ __forceinline__ void desc_row_interval(float c, float d, float B, int
 // get_gauss_pixel_bilinear, src/sift.rs:238-266, as one lerp). The two texels
 // come from aligned words: a byte-aligned 16-bit LDS read would be an
 // unaligned access.
-__device__ __forceinline__ float desc_grid_row(const unsigned* pu, int a, float dx) {
-    const unsigned* wp = pu + ((unsigned)a >> 2);
-    const unsigned r = __builtin_amdgcn_alignbyte(wp[1], wp[0], (unsigned)a & 3u);
+__device__ __forceinline__ float desc_lerp(const unsigned* wp, unsigned shift, float dx) {
+    const unsigned r = __builtin_amdgcn_alignbyte(wp[1], wp[0], shift);
     const float p1 = (float)(r & 255u), p2 = (float)((r >> 8) & 255u);
     return __builtin_fmaf(p2 - p1, dx, p1);
+}
+__device__ __forceinline__ float desc_grid_row(const unsigned* pu, int a, float dx) {
+    return desc_lerp(pu + ((unsigned)a >> 2), (unsigned)a & 3u, dx);
 }
 
 // Per-keypoint geometry of compute (src/sift.rs:940-960).
@@ -1330,10 +1338,9 @@ __device__ __forceinline__ DescGeom desc_geom(int c, const OctaveDesc* __restric
     G.w = O.w;
     G.h = O.h;
     G.pitch = O.pitch;
-    const float scale = pow2f(G.base.octave);
-    G.xo = G.base.x / scale;
-    G.yo = G.base.y / scale;
-    G.so = G.base.size / scale;
+    G.xo = over_pow2(G.base.x, G.base.octave);
+    G.yo = over_pow2(G.base.y, G.base.octave);
+    G.so = over_pow2(G.base.size, G.base.octave);
     G.bw = 3.0f * G.so;
     const float win = G.bw * 4.0f;
     const float wsig = 0.5f * win;
@@ -1353,6 +1360,10 @@ __device__ __forceinline__ void desc_bounds(const DescGeom& G, int& bx0, int& bx
     bx1 = G.side - 1;
     by0 = 0;
     by1 = G.side - 1;
+    // most windows lie inside the image: their ends decide all four (the sums grow
+    // with ix and iy)
+    const float r = (float)G.R;
+    if (G.xo - r >= 0.0f && G.xo + r < wm1 && G.yo - r >= 0.0f && G.yo + r < hm1) return;
     while (bx0 <= bx1 && G.xo + (float)(bx0 - G.R) < 0.0f) bx0++;
     while (bx1 >= bx0 && G.xo + (float)(bx1 - G.R) >= wm1) bx1--;
     while (by0 <= by1 && G.yo + (float)(by0 - G.R) < 0.0f) by0++;
@@ -1460,10 +1471,16 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
     __shared__ int seg_len;
     // per wave: (max << 8) | (255 - min) of the patch texels it staged
     __shared__ unsigned wrange[kThreads / 64];
+    // whether a grid row's texel row is not the one after its predecessor's (by the wave
+    // that made the rows' terms)
+    __shared__ int row_skips[2];
     __shared__ float2 terms_own[kTermsInPatch ? 1 : 2 * kGS];
     __shared__ float pang[kMaxPeaks], pcos[kMaxPeaks], psin[kMaxPeaks];
     uint8_t* const patch = reinterpret_cast<uint8_t*>(pu);
     unsigned* const hist = pu;
+    auto pairs = [&](unsigned byte) {
+        return reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(pu) + byte);
+    };
     // grid columns / rows: texel offset, fraction
     float2* const gcol = kTermsInPatch ? reinterpret_cast<float2*>(patch + kPatchBytes) : terms_own;
     float2* const grw = gcol + kGS;
@@ -1489,6 +1506,9 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
         }
         const int R = G.R, side = G.side, gside = 2 * R + 3;
         const float xo = G.xo, yo = G.yo, bw = G.bw, denom = G.denom;
+        // Before the first barrier each wave also has a table of its own to make: wave 0
+        // the peaks' angles, wave 1 the grid's columns, wave 2 its rows, wave 3 the
+        // Gaussian factors.
         if (tid < G.np) {  // the peaks' angles and their cos / sin, once per keypoint
             const float a = angles[(size_t)c * kMaxPeaks + tid];
             pang[tid] = a;
@@ -1497,7 +1517,7 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
         }
         {
             const int pside = 2 * R + 6;
-            const int px0 = f2i_sat(floorf(xo)) - R - 2, py0 = f2i_sat(floorf(yo)) - R - 2;
+            const int px0 = (int)floorf(xo) - R - 2, py0 = (int)floorf(yo) - R - 2;
             const int px0a = px0 & ~3, poff = px0 - px0a;
             unsigned tmax = 0u, tmin = 255u;
             const int nw = (poff + pside + 3) >> 2;  // aligned words of a row, <= kPS / 4
@@ -1505,38 +1525,48 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
                 // interior: the words [px0a, round_up(px0 + pside, 4)) of each row lie
                 // within the image. (Ending within the row's pitch is not enough: the
                 // bytes past the width are whatever the memory held, and the texel
-                // range below would take them in.)
-                const int tot = nw * pside;              // <= 18 * 68 < 5 * 256
-                const float inv_nw = 1.0f / (float)nw;
-                const uint8_t* rowp = G.g + (size_t)py0 * G.pitch + px0a;
-                unsigned wv[5];
+                // range below would take them in.) 16 words of 16 rows per pass, so a
+                // pass is a fixed step in memory and in LDS; the one or two words past
+                // the 16th of windows with R >= 26, one row per thread.
+                constexpr int kPasses = (kPatchRows + 15) / 16;
+                const int row = tid >> 4, wd = tid & 15;
+                const uint8_t* const rowp = G.g + (size_t)py0 * G.pitch + px0a;
+                const unsigned off = (unsigned)row * (unsigned)G.pitch + 4u * (unsigned)wd;
+                unsigned wv[kPasses], we[2] = {0u, 0u};
 #pragma unroll
-                for (int k = 0; k < 5; k++) {
-                    const int i = tid + k * kThreads;
+                for (int k = 0; k < kPasses; k++) {
                     wv[k] = 0u;  // defined on every path: nothing carried across keypoints
-                    if (i < tot) {
-                        const int v = (int)(((float)i + 0.5f) * inv_nw);
-                        const int wd = i - v * nw;
-                        wv[k] = *reinterpret_cast<const unsigned*>(rowp + (size_t)v * G.pitch + 4 * wd);
-                    }
+                    if (row + 16 * k < pside && wd < nw)
+                        wv[k] = *reinterpret_cast<const unsigned*>(rowp + (off + 16u * k * (unsigned)G.pitch));
+                }
+                const bool more = nw > 16 && tid < pside;
+                const unsigned offe = (unsigned)tid * (unsigned)G.pitch + 64u;
+                if (more) {
+                    we[0] = *reinterpret_cast<const unsigned*>(rowp + offe);
+                    if (nw > 17) we[1] = *reinterpret_cast<const unsigned*>(rowp + offe + 4u);
                 }
                 // texel range of the staged words (a few texels left and right of
                 // the patch included: a wider range is still a bound)
+                auto range = [&](unsigned w) {
+                    const unsigned b0 = w & 255u, b1 = (w >> 8) & 255u;
+                    const unsigned b2 = (w >> 16) & 255u, b3 = w >> 24;
+                    tmax = max(max(tmax, max(b0, b1)), max(b2, b3));
+                    tmin = min(min(tmin, min(b0, b1)), min(b2, b3));
+                };
+                unsigned* const pw = pu + row * (kPS / 4) + wd;
 #pragma unroll
-                for (int k = 0; k < 5; k++) {
-                    if (tid + k * kThreads < tot) {
-                        const unsigned b0 = wv[k] & 255u, b1 = (wv[k] >> 8) & 255u;
-                        const unsigned b2 = (wv[k] >> 16) & 255u, b3 = wv[k] >> 24;
-                        tmax = max(max(tmax, max(b0, b1)), max(b2, b3));
-                        tmin = min(min(tmin, min(b0, b1)), min(b2, b3));
+                for (int k = 0; k < kPasses; k++) {
+                    if (row + 16 * k < pside && wd < nw) {
+                        range(wv[k]);
+                        pw[16 * k * (kPS / 4)] = wv[k];
                     }
                 }
-#pragma unroll
-                for (int k = 0; k < 5; k++) {
-                    const int i = tid + k * kThreads;
-                    if (i < tot) {
-                        const int v = (int)(((float)i + 0.5f) * inv_nw);
-                        pu[v * (kPS / 4) + (i - v * nw)] = wv[k];
+                if (more) {
+                    range(we[0]);
+                    pu[tid * (kPS / 4) + 16] = we[0];
+                    if (nw > 17) {
+                        range(we[1]);
+                        pu[tid * (kPS / 4) + 17] = we[1];
                     }
                 }
             } else {
@@ -1559,16 +1589,30 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
             // the grid's column and row terms: x = x_o + i (and y = y_o + j) are the
             // same f32 sums for every point of a column (row), so their texel offset
             // and fraction are formed once
-            if (tid < gside) {
-                const float x = xo + (float)(tid - R - 1);
+            bool skips = false;
+            if (tid >= 64 && tid < 64 + gside) {
+                const int t = tid - 64;
+                const float x = xo + (float)(t - R - 1);
                 const float xf = floorf(x);
-                gcol[tid] = make_float2(__int_as_float(min(max(f2i_sat(xf) - px0, 0), pside - 2)), x - xf);
-            } else if (tid >= 128 && tid < 128 + gside) {
-                const int gy = tid - 128;
-                const float y = yo + (float)(gy - R - 1);
+                gcol[t] = make_float2(__int_as_float(min(max((int)xf - px0, 0), pside - 2)), x - xf);
+            }
+            if (tid >= 128 && tid < 128 + gside) {
+                const int t = tid - 128;
+                const float y = yo + (float)(t - R - 1);
                 const float yf = floorf(y);
-                const int v0 = min(max(f2i_sat(yf) - py0, 0), pside - 2);
-                grw[gy] = make_float2(__int_as_float(v0 * kPS + poff), y - yf);
+                const int v0 = min(max((int)yf - py0, 0), pside - 2);
+                const int first = min(max((int)floorf(yo - (float)(R + 1)) - py0, 0), pside - 2);
+                skips = v0 != first + t;
+                grw[t] = make_float2(__int_as_float(v0 * kPS + poff), y - yf);
+            }
+            if (wave >= 2) {
+                const unsigned long long m = ballot64(skips);
+                if (lane == 0) row_skips[wave - 2] = m != 0ull;
+            }
+            // Gaussian weight exp(-(px^2+py^2)/denom) as exp(-px^2/denom) * exp(-py^2/denom)
+            if (tid >= 192 && tid < 192 + side) {
+                const int d = tid - 192 - R;
+                exs[tid - 192] = expf(-(float)(d * d) / denom);
             }
             __syncthreads();
             {
@@ -1577,44 +1621,65 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
                 // ("top", "bot") and then along y; the next grid row's v0 is
                 // v0 + 1 except where the clamp to the patch (or the f32 sum
                 // y_o + j) makes it otherwise, so its "top" is this row's "bot"
-                // and each patch row is interpolated once per band.
-                const float inv_gs = 1.0f / (float)gside;
-                const int nb = kThreads / gside;  // bands: >= 3 (gside <= 65)
+                // and each patch row is interpolated once per band. Where no row
+                // skips, the walk is a fixed step of the patch: every LDS address
+                // is the last one plus a constant.
+                const float inv_gs = __builtin_amdgcn_rcpf((float)gside);  // quotients of small integers, + 1/2
+                const int nb = (int)(((float)kThreads + 0.5f) * inv_gs);   // bands: >= 3 (gside <= 65)
                 const int band = (int)(((float)tid + 0.5f) * inv_gs), gx = tid - band * gside;
                 if (band < nb) {
-                    const int rows = (gside + nb - 1) / nb;
-                    const int gy1 = min((band + 1) * rows, gside);
+                    const int rows = (int)(((float)(gside + nb - 1) + 0.5f) * __builtin_amdgcn_rcpf((float)nb));
+                    const int gy0 = band * rows, gy1 = min(gy0 + rows, gside);
                     const float2 cxd = gcol[gx];
                     const int cxo = __float_as_int(cxd.x);
                     const float dx = cxd.y;
-                    float top = 0.0f;
-                    // patch offset of the previous row's v0; offsets are >= 0, so
-                    // the first row of the band never matches it
-                    int prev = -(1 << 30);
-                    for (int gy = band * rows; gy < gy1; gy++) {
-                        const float2 ryd = grw[gy];
-                        const int ro = __float_as_int(ryd.x);
-                        if (ro != prev + kPS) top = desc_grid_row(pu, ro + cxo, dx);
-                        const float bot = desc_grid_row(pu, ro + kPS + cxo, dx);
-                        grid[gy * kGS + gx] = __builtin_fmaf(bot - top, ryd.y, top);
-                        top = bot;
-                        prev = ro;
+                    if (!(row_skips[0] | row_skips[1])) {
+                        if (gy0 < gy1) {
+                            const int at = __float_as_int(grw[gy0].x) + cxo;
+                            const unsigned* wp = pu + ((unsigned)at >> 2);
+                            const unsigned sh = (unsigned)at & 3u;
+                            float top = desc_lerp(wp, sh, dx);
+                            float* gp = grid + gy0 * kGS + gx;
+                            const float2* rp = grw + gy0;
+                            const int n = gy1 - gy0;
+#pragma unroll 3
+                            for (int k = 0; k < n; k++) {
+                                const float bot = desc_lerp(wp + (k + 1) * (kPS / 4), sh, dx);
+                                gp[k * kGS] = __builtin_fmaf(bot - top, rp[k].y, top);
+                                top = bot;
+                            }
+                        }
+                    } else {
+                        float top = 0.0f;
+                        // patch offset of the previous row's v0; offsets are >= 0, so
+                        // the first row of the band never matches it
+                        int prev = -(1 << 30);
+                        for (int gy = gy0; gy < gy1; gy++) {
+                            const float2 ryd = grw[gy];
+                            const int ro = __float_as_int(ryd.x);
+                            if (ro != prev + kPS) top = desc_grid_row(pu, ro + cxo, dx);
+                            const float bot = desc_grid_row(pu, ro + kPS + cxo, dx);
+                            grid[gy * kGS + gx] = __builtin_fmaf(bot - top, ryd.y, top);
+                            top = bot;
+                            prev = ro;
+                        }
                     }
                 }
             }
-            // Gaussian weight exp(-(px^2+py^2)/denom) as exp(-px^2/denom) * exp(-py^2/denom)
-            for (int i = tid; i < side; i += kThreads) exs[i] = expf(-(float)((i - R) * (i - R)) / denom);
         }
         __syncthreads();  // patch reads done before the histograms reuse its storage
         int bx0, bx1, by0, by1;
         desc_bounds(G, bx0, bx1, by0, by1);
         const int nrows = G.so > 0.0f ? max(by1 - by0 + 1, 0) : 0;  // <= 63
+        // one division per keypoint: the empty asm keeps the compiler from repeating it
+        // in each place of use
+        float inv_bw = 1.0f / bw;
+        asm volatile("" : "+v"(inv_bw));
         for (int pk = 0; pk < G.np; pk++) {
             const float angle = uniform_f(pang[pk]);
             for (int i = tid; i < kHistCopies * kHistWords / 4; i += kThreads)
                 reinterpret_cast<uint4*>(hist)[i] = make_uint4(0u, 0u, 0u, 0u);
             const float ca = uniform_f(pcos[pk]), sa = uniform_f(psin[pk]);
-            const float inv_bw = uniform_f(1.0f / bw);
             const float msa = -sa;  // -sin * px is computed as (-sin) * px, the same value
             const float abin = uniform_f(angle * (4.0f / kPi));  // the peak angle in bins
             if (tid < 64) {
@@ -1639,11 +1704,16 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
                 // gives at most 256 segments (per <= 16: a row holds at most 63
                 // samples, so per = 16 gives at most 4 * 63 segments).
                 const int T = __builtin_amdgcn_readlane(wave_incl_scan(cnt), 63);
+                // (quotients of integers below 80 by at most 16, + 1/2 in the dividend: a
+                // product with the reciprocal, truncated, is exact)
                 int per = max((T + kThreads - 1) / kThreads, 1);
-                int segs = wave_incl_scan((cnt + per - 1) / per);
+                auto segments = [&]() {
+                    return (int)(((float)(cnt + per - 1) + 0.5f) * __builtin_amdgcn_rcpf((float)per));
+                };
+                int segs = wave_incl_scan(segments());
                 while (__builtin_amdgcn_readlane(segs, 63) > kThreads) {
                     per++;
-                    segs = wave_incl_scan((cnt + per - 1) / per);
+                    segs = wave_incl_scan(segments());
                 }
                 rpre[tid + 1] = segs;  // segment prefix over the rows
                 // the fixed-point scale 2^(20 + fe), passed with the segment length
@@ -1657,7 +1727,6 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
             const int per = seg_len & 0xffff, fe = seg_len >> 16;
             const int sg = lane * 4 + wave;  // lanes of a wave take segments far apart
             if (sg < rpre[nrows]) {
-                unsigned* hw = hist + (lane & 1) * kHistWords;  // neighbouring lanes: different copies
                 int r0 = 0, r1 = nrows;  // rpre[r0] <= sg < rpre[r1]: row r0 holds the segment
                 while (r1 - r0 > 1) {
                     const int mid = (r0 + r1) >> 1;
@@ -1685,7 +1754,12 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
                 // per run. The sums are defined from the start (each run resets them
                 // anyway): left undefined, they were carried through the keypoint
                 // loop and spilled to scratch once per keypoint.
-                unsigned long long* acc_base = nullptr;
+                // A run's bin pair is held as its byte offset in the histograms. The first
+                // one is a cell by lane, where the sums of no run (0.5, truncated) add
+                // zero: no step has to ask whether there is a run.
+                const int copy = (lane & 1) * kHistWords * 4;  // neighbouring lanes: different copies
+                const float hbytes = (float)(copy + 7 * 4 * kCellWords);
+                unsigned acc_base = (unsigned)(copy + (lane >> 1) % 28 * (4 * kCellWords));
                 float acc[8] = {0.5f, 0.5f, 0.5f, 0.5f, 0.5f, 0.5f, 0.5f, 0.5f};
                 float u = __builtin_fmaf(cai, (float)(cx - R), rz);
                 float v = __builtin_fmaf(msai, (float)(cx - R), rw);
@@ -1702,9 +1776,9 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
                     // integer floor) and the fraction ab - floor(ab) needs no wrap
                     const float ab = atan2_bins(gyv, gx) - abin;
                     float tt[4], da;
-                    unsigned long long* const base = desc_bins(hw, u + 1.5f, v + 1.5f, ab, m, tt, da);
+                    const unsigned base = desc_bins(hbytes, u + 1.5f, v + 1.5f, ab, m, tt, da);
                     if (base != acc_base) {  // a new bin pair: add the finished sums
-                        if (acc_base) desc_add_pairs<1>(acc_base, acc);
+                        desc_add_pairs<1>(pairs(acc_base), acc);
                         acc_base = base;
 #pragma unroll
                         for (int q8 = 0; q8 < 8; q8++) acc[q8] = 0.5f;
@@ -1716,7 +1790,7 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
                         acc[2 * q4 + 1] = __builtin_fmaf(tt[q4], da, acc[2 * q4 + 1]);
                     }
                 }
-                if (acc_base) desc_add_pairs<1>(acc_base, acc);
+                desc_add_pairs<1>(pairs(acc_base), acc);
             }
             __syncthreads();
             if (tid < 64) {
