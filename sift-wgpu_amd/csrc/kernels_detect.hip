@@ -1469,6 +1469,7 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
     __shared__ int rspan[64];  // per row: first and last column of its samples (16 bits each)
     __shared__ int rpre[65];
     __shared__ int seg_len;
+    __shared__ unsigned char seg_row[kThreads];  // the row of each segment
     // per wave: (max << 8) | (255 - min) of the patch texels it staged
     __shared__ unsigned wrange[kThreads / 64];
     // whether a grid row's texel row is not the one after its predecessor's (by the wave
@@ -1716,6 +1717,11 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
                     segs = wave_incl_scan(segments());
                 }
                 rpre[tid + 1] = segs;  // segment prefix over the rows
+                // each segment's row, one segment of every row at a time
+                const int mine = segments();
+                unsigned char* const sr = seg_row + (segs - mine);
+                for (int k = 0; ballot64(k < mine) != 0ull; k++)
+                    if (k < mine) sr[k] = (unsigned char)tid;
                 // the fixed-point scale 2^(20 + fe), passed with the segment length
                 const int fe = desc_range_exp(wrange);
                 if (tid == 0) {
@@ -1727,12 +1733,7 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
             const int per = seg_len & 0xffff, fe = seg_len >> 16;
             const int sg = lane * 4 + wave;  // lanes of a wave take segments far apart
             if (sg < rpre[nrows]) {
-                int r0 = 0, r1 = nrows;  // rpre[r0] <= sg < rpre[r1]: row r0 holds the segment
-                while (r1 - r0 > 1) {
-                    const int mid = (r0 + r1) >> 1;
-                    if (rpre[mid] <= sg) r0 = mid;
-                    else r1 = mid;
-                }
+                const int r0 = seg_row[sg];
                 const int span = rspan[r0];
                 int cx = (span & 0xffff) + (sg - rpre[r0]) * per;
                 const int len = min(per, (span >> 16) - cx + 1);
