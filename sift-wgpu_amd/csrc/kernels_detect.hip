@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 
 #include "sift_internal.h"
 
@@ -50,18 +51,43 @@ __device__ __forceinline__ float pow2f(int o) { return ldexpf(1.0f, o); }
 // denormals), in one instruction instead of about ten
 __device__ __forceinline__ float over_pow2(float x, int o) { return __builtin_amdgcn_ldexpf(x, -o); }
 
-// atan2 for the gradient angles: octant reduction a = min(|x|,|y|)/max(|x|,|y|),
+// Three-operand maximum / minimum of values that are never NaN. (fmaxf and fminf
+// first quiet each operand the compiler cannot prove is no signalling NaN: one
+// more instruction for every value read from LDS.)
+__device__ __forceinline__ float max3f(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float min3f(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float max2f(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float min2f(float a, float b) {
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Gradient angle in [0, 2 pi]: octant reduction a = min(|x|,|y|)/max(|x|,|y|),
 // atan(a) = a * P(a^2) with P a degree-8 least-squares (Lawson-reweighted)
 // fit to atan(a)/a on [0,1], evaluated with FMA (max error 1.0e-7 rad on [0,1];
 // about 2e-7 rad after the quadrant corrections, comparable to a 1-2 ulp
-// atan2f). Gradients here are differences of non-negative values, never -0.
-__device__ __forceinline__ float atan2_grad(float y, float x) {
+// atan2f). Gradients here are differences of non-negative values, never -0, and
+// 0 or far above 1e-30: x = y = 0 gives a = 0 without a test of its own.
+__device__ __forceinline__ float grad_angle(float y, float x) {
     const float ax = fabsf(x), ay = fabsf(y);
     // selects rather than fmaxf / fminf: the operands are never NaN, and one
     // comparison serves both and the octant test below
     const bool steep = ay > ax;
     const float mx = steep ? ay : ax, mn = steep ? ax : ay;
-    const float a = mx > 0.0f ? mn * __builtin_amdgcn_rcpf(mx) : 0.0f;
+    const float a = mn * __builtin_amdgcn_rcpf(max2f(mx, 1e-30f));
     const float s = a * a;
     float p = 0.002456706715747714f;
     p = __builtin_fmaf(p, s, -0.014401290565729141f);
@@ -75,7 +101,7 @@ __device__ __forceinline__ float atan2_grad(float y, float x) {
     float r = a * p;
     if (steep) r = 1.57079637050628662109f - r;
     if (x < 0.0f) r = 3.14159274101257324219f - r;
-    return copysignf(r, y);
+    return y < 0.0f ? kTwoPi - r : r;
 }
 
 // Gradient angle in descriptor bin units (pi/4 per bin, result in (-4, 4]):
@@ -107,6 +133,22 @@ __device__ __forceinline__ float div_two_pi(float x) {
     constexpr float rc = 1.0f / kTwoPi;
     const float y = x * rc;
     return __builtin_fmaf(__builtin_fmaf(-y, kTwoPi, x), rc, y);
+}
+
+// Bin of a gradient angle in [0, 2 pi] (36 bins; 36 stands for bin 0): (an * 36) /
+// 2pi with the reference's two roundings, as gradients along the axes land exactly
+// on bin edges, where the rounding decides the bin.
+__device__ __forceinline__ unsigned angle_bin(float an) {
+    return (unsigned)div_two_pi(an * 36.0f);
+}
+
+// x / 3 for x = 0 or x > 2^-60: one FMA correction of the product with RN(1/3).
+// Equal to the IEEE division for every f32 mantissa (checked exhaustively over two
+// binades; the operations scale with the exponent).
+__device__ __forceinline__ float over_3(float x) {
+    constexpr float rc = 1.0f / 3.0f;
+    const float y = x * rc;
+    return __builtin_fmaf(__builtin_fmaf(-y, 3.0f, x), rc, y);
 }
 
 // A wave-uniform f32 value moved to a scalar register (the compiler cannot prove
@@ -261,6 +303,7 @@ constexpr int kExtRW = kTileW + 8;                // staged D row: columns [x0-4
 static_assert(kExtItems <= kThreads, "one item per thread");
 typedef __attribute__((address_space(1))) const uint8_t gbyte_t;
 typedef __attribute__((address_space(1))) const unsigned long long gu64_t;
+typedef __attribute__((address_space(1))) const unsigned gu32_t;
 
 // The NG level words of this thread's item of the band starting at row y0 (rows
 // y0-1 .. y0+16, clamped): the aligned 8-byte word at the item's columns, or the
@@ -326,30 +369,6 @@ __device__ __forceinline__ void ext_stage(const unsigned long long (&u)[NG],
             for (int b = 0; b < 4; b++) qlo[b] = qhi[b];
         }
     }
-}
-
-// Three-operand maximum / minimum of values that are never NaN. (fmaxf and fminf
-// first quiet each operand the compiler cannot prove is no signalling NaN: one
-// more instruction for every value read from LDS.)
-__device__ __forceinline__ float max3f(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ float min3f(float a, float b, float c) {
-    float r;
-    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-__device__ __forceinline__ float max2f(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-__device__ __forceinline__ float min2f(float a, float b) {
-    float r;
-    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
 }
 
 // Occupancy target: the LDS bound (6 work-groups per CU for S <= 3).
@@ -869,20 +888,6 @@ __global__ __launch_bounds__(kThreads) void k_refine(const OctaveDesc* __restric
 }
 
 // ---------------------------------------------------------------------------
-// k_orient: one wave (workgroup of 64) per refined keypoint, grid-stride
-// (src/sift.rs:605-726). For R <= 16 the window's rows and columns of the
-// Gaussian level (every pixel the gradient of a sample can touch) are staged
-// in LDS as bytes; a sample reads q = v/255 of its 4 gradient texels from an
-// LDS table filled with the exact f32 q255f. Lane l takes one contiguous chunk of the
-// (2R+1)^2 window in raster order; each sample adds mag * exp(-(dx^2+dy^2)/denom)
-// to bin floor(theta * 36 / 2pi) of a u64 fixed-point (2^40) histogram, one of 4
-// copies by lane, with runs of same-bin samples summed in registers first
-// (integer adds: order-independent, deterministic, and as fine as the f32
-// contributions themselves). Lanes 0..35 then hold one bin
-// each for the two [1,1,1]/3 smoothing passes, the max and the peak test; a
-// ballot ranks the peaks in bin order.
-// ---------------------------------------------------------------------------
-// ---------------------------------------------------------------------------
 // Work queue of the keypoint kernels. With a queue, a launch has as many
 // work-groups as fit on the GPU at once, and each takes chunks of kChunk
 // consecutive keypoints until the count is reached. Work-group b uses counter
@@ -936,10 +941,58 @@ struct WorkQueue {
 constexpr int kOrientChunk = 8;
 constexpr int kDescChunk = 2;
 
-constexpr int kOriMaxR = 16;
-constexpr int kOriRows = 2 * kOriMaxR + 5;  // staged rows
-constexpr int kOS = 2 * kOriMaxR + 8;       // staged row stride (bytes): 4 * ceil((3 + rows + 3) / 4)
+// Maximum over the 64 lanes of a fully active wave with DPP:
+// shifts by 1, 2, 4, 8 inside each row of 16 lanes, then lane 15 of rows 0 and 2 to rows 1 and 3
+// and lane 31 to rows 2 and 3; returned to every lane.
+__device__ __forceinline__ unsigned wave_max_u32(unsigned x) {
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true));  // row_shr:1
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true));  // row_shr:2
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true));  // row_shr:4
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true));  // row_shr:8
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false)); // row_bcast:15
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false)); // row_bcast:31
+    return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
+}
 
+constexpr int kOriMaxR = 16;
+constexpr int kOriRows = 2 * kOriMaxR + 5;      // staged rows
+constexpr int kOS = 2 * kOriMaxR + 8;           // staged row stride (bytes): 4 * ceil((3 + rows + 3) / 4)
+constexpr int kOriHist = 37;                    // words of one histogram copy: 36 bins, and 36 for bin 0
+static_assert(2 * kOriMaxR + 1 <= 64, "one lane per row and column of the window");
+constexpr double kOriBias = 4503599627370496.0;  // 2^52
+
+// ---------------------------------------------------------------------------
+// k_orient: one wave (workgroup of 64) per refined keypoint
+// (src/sift.rs:605-726). Each sample of the (2R+1)^2 window adds
+// mag * exp(-(dx^2+dy^2)/denom) to bin floor(theta * 36 / 2pi) of a u64
+// fixed-point (2^40) histogram, one of 4 copies by lane (integer adds:
+// order-independent, deterministic, and as fine as the f32 contributions
+// themselves). Lanes 0..35 then hold one bin each for the two [1,1,1]/3 smoothing
+// passes, the max and the peak test; a ballot ranks the peaks in bin order.
+//
+// Windows with R <= 16 (all of the default schedule) are staged in LDS as
+// bytes, every texel a sample's gradient can touch. Lane l takes the samples
+// [l C, (l+1) C) in raster order, C = ceil(n / 64): lanes sit far apart in the
+// window, and a lane's consecutive samples are neighbours that often share a bin,
+// so they are summed in registers and added to LDS once per run. The sum is an f64
+// that starts at 2^52: the samples' fixed-point values are whole numbers, so its
+// low 52 bits hold the integer sum exactly (a window's total is below
+// 33^2 * sqrt(2) * 2^40 < 2^51) and are added as they are; what the biases leave in
+// the high 12 bits is masked off at the end.
+// The loop has the same count for every lane and no test per sample: a lane's C <=
+// 2R + 1 samples cross into the next row at most once, so the column table is
+// written twice over and the row is a choice of two; samples off the image or past
+// the window have weight 0 (they add 0 to some bin).
+//
+// Bound by vector instruction issue (about 100 instructions per sample step and 250
+// per keypoint), with LDS two thirds busy. 64 x 1920x1080: 940 us with a table of
+// v / 255 in LDS (10 LDS reads per sample, now 5), the u64 arithmetic on two words, a
+// test per sample, staging by a division and IEEE divisions by 3 and by powers of
+// two; 635 us so. Texels held as f32 instead of bytes (no conversion per sample):
+// 777-830 us, as LDS then holds 20 work-groups per CU instead of 32 and its reads
+// spread over more banks. 2 or 8 histogram copies, other row strides and an unaligned
+// word for the two horizontal texels were slower too (1150 us for the last).
+// ---------------------------------------------------------------------------
 __global__ __launch_bounds__(64) void k_orient(const OctaveDesc* __restrict__ oct,
                                                const ImageParams* __restrict__ params,
                                                const Cand* __restrict__ cand,
@@ -949,19 +1002,14 @@ __global__ __launch_bounds__(64) void k_orient(const OctaveDesc* __restrict__ oc
                                                unsigned* __restrict__ npeaks,
                                                float* __restrict__ angles,
                                                unsigned* __restrict__ queue) {
-    // 4 histogram copies (lane & 3), the staged window and the q table: 4.2 KB of
-    // LDS, so the 8 waves per SIMD that its 44 VGPRs allow fit (32 work-groups of one
-    // wave per CU; 21 with the window staged as f32)
-    __shared__ unsigned long long hist[4][36];
-    // v / 255 for every byte (q255f, exact): 4 LDS reads per sample instead of 12 VALU
-    // operations; written before the first keypoint's barrier, which orders it
-    __shared__ float qt[256];
-    for (int i = threadIdx.x; i < 256; i += 64) qt[i] = q255f((float)i);
+    __shared__ __align__(16) unsigned long long hist[4 * kOriHist];
     __shared__ __align__(16) uint8_t pq[kOriRows * kOS];
-    // per column / row of the window: (pixel offset as int bits, Gaussian factor)
-    __shared__ float2 ocx[2 * kOriMaxR + 1], ocy[2 * kOriMaxR + 1];
+    // per column (twice over) / row of the window: (byte offset in pq as int bits, Gaussian factor)
+    __shared__ float2 ocx[2 * (2 * kOriMaxR + 1)], ocy[64];
     const int lane = threadIdx.x;
     const int n = (int)min(*total, (unsigned)cap);
+    // the neighbour bins of the 36-bin circle, as ds_bpermute addresses
+    const int prev4 = 4 * (lane == 0 ? 35 : lane - 1), next4 = 4 * (lane == 35 ? 0 : min(lane + 1, 63));
     __shared__ int qslot[2];
     WorkQueue<kOrientChunk> Q{queue, 0, 0, 0};
     for (int c = Q.first(qslot); c < n; c = Q.next(qslot, c)) {
@@ -977,13 +1025,13 @@ __global__ __launch_bounds__(64) void k_orient(const OctaveDesc* __restrict__ oc
         const int gl = min(max(kp.layer, 0), S + 2);
         const uint8_t* g = O.levels + (long long)gl * O.level_stride;
         const int w = O.w, h = O.h, pitch = O.pitch;
-        const float scale = pow2f(kp.octave);
-        const float xo = kp.x / scale, yo = kp.y / scale, so = kp.size / scale;
+        const float xo = over_pow2(kp.x, kp.octave), yo = over_pow2(kp.y, kp.octave);
+        const float so = over_pow2(kp.size, kp.octave);
         if (!(so > 0.0f)) {
             if (lane == 0) npeaks[c] = 0;
             continue;
         }
-        const int R = f2i_sat(roundf(4.5f * so));
+        const int R = __builtin_amdgcn_readfirstlane(f2i_sat(roundf(4.5f * so)));
         const float ws = 1.5f * so;
         const float denom = 2.0f * ws * ws;
         const int side = 2 * R + 1, nsamp = side * side;
@@ -992,128 +1040,165 @@ __global__ __launch_bounds__(64) void k_orient(const OctaveDesc* __restrict__ oc
         const float kq = -1.44269504088896341f / denom;
         constexpr float lf = 40.0f;  // m = mag * weight * 2^40
         const bool lds = R <= kOriMaxR;
-        for (int i = lane; i < 4 * 36; i += 64) (&hist[0][0])[i] = 0ull;
-        // the samples' pixels (round(x_o + dx), round(y_o + dy)) and their 4-neighbours
-        // lie in columns px0 .. px0 + 2R + 4 and rows py0 .. py0 + 2R + 4
-        const int px0 = f2i_sat(roundf(xo)) - R - 2, py0 = f2i_sat(roundf(yo)) - R - 2;
-        const int px0a = px0 & ~3;
+        const float inv_side = __builtin_amdgcn_rcpf((float)side);
+        reinterpret_cast<uint4*>(hist)[lane] = make_uint4(0u, 0u, 0u, 0u);
+        if (lane < 2 * kOriHist - 64)
+            reinterpret_cast<uint4*>(hist)[64 + lane] = make_uint4(0u, 0u, 0u, 0u);
         if (lds) {
-            const int pside = 2 * R + 5;
-            const int nw = (px0 - px0a + pside + 3) >> 2;  // <= kOS / 4
-            const float inv_nw = 1.0f / (float)nw;
-            for (int i = lane; i < nw * pside; i += 64) {
-                const int v = (int)(((float)i + 0.5f) * inv_nw), wd = i - v * nw;
-                const int yy = py0 + v, xw = px0a + 4 * wd;
-                unsigned u = 0;
-                if (yy >= 0 && yy < h) {
-                    const uint8_t* row = g + (size_t)yy * pitch;
-                    if (xw >= 0 && xw + 4 <= pitch) {
-                        u = *reinterpret_cast<const unsigned*>(row + xw);
-                    } else {
+            // the samples' pixels (round(x_o + dx), round(y_o + dy)) and their 4-neighbours
+            // lie in columns px0 .. px0 + 2R + 4 and rows py0 .. py0 + 2R + 4
+            const int px0 = __builtin_amdgcn_readfirstlane((int)roundf(xo)) - R - 2;
+            const int py0 = __builtin_amdgcn_readfirstlane((int)roundf(yo)) - R - 2;
+            const int px0a = px0 & ~3;
+            // a lane stages one 4-texel word of every kPer-th row, all loads in flight
+            // at once; words and rows past the window are staged too where that saves
+            // a test. Eight words of a row hold R <= 12 (2 R + 5 texels and 3 before
+            // them), ten R <= 16.
+            gbyte_t* const g8 = (gbyte_t*)g;
+            auto stage = [&](auto words_tag, auto passes_tag) {
+                constexpr int kWords = decltype(words_tag)::value, kPasses = decltype(passes_tag)::value;
+                constexpr int kPer = 64 / kWords;
+                const int wd = lane % kWords, row = lane / kWords;
+                unsigned u[kPasses];
+                if (px0a >= 0 && px0a + 4 * kWords <= pitch && py0 >= 0 && py0 + kPer * kPasses <= h) {
+                    const unsigned off = __umul24(row, pitch) + 4 * wd;
+                    gbyte_t* base = g8 + ((size_t)py0 * pitch + px0a);
 #pragma unroll
-                        for (int b = 0; b < 4; b++)
-                            if (xw + b >= 0 && xw + b < w) u |= (unsigned)row[xw + b] << (8 * b);
+                    for (int k = 0; k < kPasses; k++, base += kPer * pitch) u[k] = *(gu32_t*)(base + off);
+                } else {
+                    // words off the image are taken from its nearest word: only samples of
+                    // weight 0 read them
+                    const unsigned xw = min(max(px0a + 4 * wd, 0), pitch - 4);
+#pragma unroll
+                    for (int k = 0; k < kPasses; k++) {
+                        const int yy = min(max(py0 + row + kPer * k, 0), h - 1);
+                        u[k] = *(gu32_t*)(g8 + (__umul24(yy, pitch) + xw));
                     }
                 }
-                *reinterpret_cast<unsigned*>(&pq[v * kOS + 4 * wd]) = u;
-            }
-            // per column and row of the window: the sample pixel's offset in the
-            // staged window, or -1 when it is outside [1, w-2] x [1, h-2], and the
-            // Gaussian weight's factor 2^(kq d^2 + 20) of that column / row offset
-            // d (the weight of sample (dx, dy) is the product of its column's and
-            // its row's factors: one multiply per sample instead of exp2)
-            if (lane < side) {
+                if (kWords > kOS / 4 && wd >= kOS / 4) return;
+                uint8_t* const dst = &pq[row * kOS + 4 * wd];
+#pragma unroll
+                for (int k = 0; k < kPasses; k++) {
+                    if (kPer * kPasses > kOriRows && row + kPer * k >= kOriRows) break;
+                    *reinterpret_cast<unsigned*>(dst + kPer * kOS * k) = u[k];
+                }
+            };
+            if (R <= 9) stage(std::integral_constant<int, 8>{}, std::integral_constant<int, 3>{});
+            else if (R <= 12) stage(std::integral_constant<int, 8>{}, std::integral_constant<int, 4>{});
+            else stage(std::integral_constant<int, 16>{}, std::integral_constant<int, 10>{});
+            // per column and row of the window: the offset in the staged window of the
+            // texel before the sample's, and the Gaussian weight's factor 2^(kq d^2 + 20)
+            // of that column / row offset d (the weight of sample (dx, dy) is the product
+            // of the two: one multiply per sample instead of exp2), 0 outside
+            // [1, w-2] x [1, h-2]
+            {
                 const float d = (float)(lane - R);
                 const float wf = __builtin_amdgcn_exp2f(__builtin_fmaf(kq, d * d, 0.5f * lf));
-                const int xi = f2i_sat(roundf(xo + d));
-                ocx[lane] = make_float2(__int_as_float((xi >= 1 && xi < w - 1) ? xi - px0a : -1), wf);
-                const int yi = f2i_sat(roundf(yo + d));
-                ocy[lane] = make_float2(__int_as_float((yi >= 1 && yi < h - 1) ? (yi - py0) * kOS : -1), wf);
+                const int xi = (int)roundf(xo + d), yi = (int)roundf(yo + d);
+                const bool row_in = lane < side && yi >= 1 && yi < h - 1;
+                ocy[lane] = make_float2(__int_as_float(row_in ? (yi - py0 - 1) * kOS : 0),
+                                        row_in ? wf : 0.0f);
+                if (lane < side) {
+                    const bool col_in = xi >= 1 && xi < w - 1;
+                    const float2 e = make_float2(__int_as_float(col_in ? (xi - px0a - 1) : 0),
+                                                 col_in ? wf : 0.0f);
+                    ocx[lane] = e;
+                    ocx[lane + side] = e;
+                }
             }
         }
         __syncthreads();
-        // lane l takes the samples [l C, (l+1) C) in raster order, C = ceil(n / 64):
-        // lanes sit far apart in the window, and a lane's consecutive samples are
-        // neighbours that often share a bin, so their fixed-point values are
-        // summed in registers (integer sums: the histogram is the same as with
-        // one add per sample) and added to LDS once per run
-        const int i0 = min(lane * iters, nsamp), i1 = min(i0 + iters, nsamp);
-        const int iy0 = (int)(((float)i0 + 0.5f) * (1.0f / (float)side));
-        int dy = iy0 - R, dx = i0 - iy0 * side - R;
-        unsigned long long run = 0;
-        int run_bin = -1;
-        unsigned long long* const hrow = hist[lane & 3];
-        for (int i = i0; i < i1; i++) {
-            float gx = 0.0f, gy = 0.0f, wgt = 0.0f;
-            bool in = true;
-            if (lds) {
-                const float2 cx = ocx[dx + R], cy = ocy[dy + R];
-                const int ox = __float_as_int(cx.x), oy = __float_as_int(cy.x);
-                wgt = cx.y * cy.y;
-                in = (ox | oy) >= 0;
-                if (in) {
-                    const uint8_t* pp = &pq[oy + ox];
-                    gx = qt[pp[1]] - qt[pp[-1]];
-                    gy = qt[pp[kOS]] - qt[pp[-kOS]];
+        unsigned long long* const hrow = hist + (lane & 3) * kOriHist;
+        unsigned run_bin = 0;
+        if (lds) {
+            const int i0 = lane * iters;
+            const int iy0 = (int)(((float)i0 + 0.5f) * inv_side);  // <= 63
+            const int ix0 = i0 - iy0 * side;
+            const int wrap = side - ix0;  // the first sample of the next row
+            const float2 row0 = ocy[iy0], row1 = ocy[min(iy0 + 1, 63)];
+            const float2* const cols = &ocx[ix0];
+            double run = kOriBias;
+            float gx, gy, wgt;
+            auto sample = [&](int k) {
+                const float2 cx = cols[k];
+                const bool second = k >= wrap;
+                const int off = __float_as_int(cx.x) + __float_as_int(second ? row1.x : row0.x);
+                const uint8_t* const pp = pq + off;
+                gx = q255f((float)pp[kOS + 2]) - q255f((float)pp[kOS]);
+                gy = q255f((float)pp[2 * kOS + 1]) - q255f((float)pp[1]);
+                wgt = cx.y * (second ? row1.y : row0.y);
+            };
+            sample(0);
+            for (int k = 0; k < iters; k++) {
+                const float sx = gx, sy = gy, sw = wgt;
+                sample(k + 1);
+                  // the next sample's reads overlap this one's arithmetic (the
+                                // last one's too: ix0 + iters < 2 side, a sample of some row)
+                const float m = __builtin_amdgcn_sqrtf(__builtin_fmaf(sx, sx, sy * sy)) * sw;
+                const unsigned bin = angle_bin(grad_angle(sy, sx));
+                if (bin != run_bin) {
+                    atomicAdd(&hrow[run_bin], (unsigned long long)__double_as_longlong(run));
+                    run = kOriBias;
+                    run_bin = bin;
                 }
-            } else {
+                run += (double)floorf(m);
+            }
+            atomicAdd(&hrow[run_bin], (unsigned long long)__double_as_longlong(run));
+        } else {
+            const int i0 = min(lane * iters, nsamp), i1 = min(i0 + iters, nsamp);
+            const int iy0 = i0 / side;
+            int dy = iy0 - R, dx = i0 - iy0 * side - R;
+            unsigned long long run = 0;
+            for (int i = i0; i < i1; i++) {
                 const int yi = f2i_sat(roundf(yo + (float)dy));
                 const int xi = f2i_sat(roundf(xo + (float)dx));
-                in = yi >= 1 && yi < h - 1 && xi >= 1 && xi < w - 1;
-                if (in) {
+                if (yi >= 1 && yi < h - 1 && xi >= 1 && xi < w - 1) {
                     const uint8_t* p = g + (size_t)yi * pitch + xi;
-                    gx = q255f((float)p[1]) - q255f((float)p[-1]);
-                    gy = q255f((float)p[pitch]) - q255f((float)p[-pitch]);
+                    const float gx = q255f((float)p[1]) - q255f((float)p[-1]);
+                    const float gy = q255f((float)p[pitch]) - q255f((float)p[-pitch]);
                     const float fdx = (float)dx, fdy = (float)dy;
-                    wgt = __builtin_amdgcn_exp2f(__builtin_fmaf(kq, __builtin_fmaf(fdx, fdx, fdy * fdy), lf));
+                    const float wgt =
+                        __builtin_amdgcn_exp2f(__builtin_fmaf(kq, __builtin_fmaf(fdx, fdx, fdy * fdy), lf));
+                    const float m = __builtin_amdgcn_sqrtf(__builtin_fmaf(gx, gx, gy * gy)) * wgt;
+                    const unsigned bin = angle_bin(grad_angle(gy, gx));
+                    if (bin != run_bin) {
+                        atomicAdd(&hrow[run_bin], run);
+                        run_bin = bin;
+                        run = 0;
+                    }
+                    run += (unsigned long long)m;
+                }
+                if (++dx > R) {
+                    dx = -R;
+                    dy++;
                 }
             }
-            if (in) {
-                const float m = __builtin_amdgcn_sqrtf(__builtin_fmaf(gx, gx, gy * gy)) * wgt;
-                const float ang = atan2_grad(gy, gx);
-                const float an = ang < 0.0f ? ang + kTwoPi : ang;
-                // (an * 36) / 2pi with the reference's two roundings: gradients along the
-                // axes land exactly on bin edges, where the rounding decides the bin
-                int bin = (int)floorf(div_two_pi(an * 36.0f));
-                bin = bin >= 36 ? bin - 36 : bin;
-                // m * 2^40 as a u64: the high word is exact (power-of-two scaling and
-                // floor), the remainder x - hi * 2^32 is exact (Sterbenz), both truncate
-                const float hi = floorf(m * 2.3283064365386963e-10f);
-                const float lo = __builtin_fmaf(-hi, 4294967296.0f, m);
-                const unsigned long long v = ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo;
-                if (bin != run_bin) {
-                    if (run_bin >= 0) atomicAdd(&hrow[run_bin], run);
-                    run_bin = bin;
-                    run = 0;
-                }
-                run += v;
-            }
-            if (++dx > R) {
-                dx = -R;
-                dy++;
-            }
+            atomicAdd(&hrow[run_bin], run);
         }
-        if (run_bin >= 0) atomicAdd(&hrow[run_bin], run);
         __syncthreads();
         float hv = 0.0f;
         if (lane < 36) {
             unsigned long long sum = 0;
 #pragma unroll
-            for (int k = 0; k < 4; k++) sum += hist[k][lane];
+            for (int k = 0; k < 4; k++) sum += hist[k * kOriHist + lane];
+            if (lane == 0) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) sum += hist[k * kOriHist + 36];
+            }
+            if (lds) sum &= (1ull << 52) - 1ull;
             hv = (float)((double)sum * (1.0 / 1099511627776.0));
         }
+        auto from_lane = [](int lane4, float v) {
+            return __int_as_float(__builtin_amdgcn_ds_bpermute(lane4, __float_as_int(v)));
+        };
         for (int it = 0; it < 2; it++) {
-            const float pv = __shfl(hv, lane < 36 ? (lane + 35) % 36 : lane, 64);
-            const float nv = __shfl(hv, lane < 36 ? (lane + 1) % 36 : lane, 64);
-            if (lane < 36) hv = (pv + hv + nv) / 3.0f;
+            const float pv = from_lane(prev4, hv), nv = from_lane(next4, hv);
+            if (lane < 36) hv = over_3(pv + hv + nv);
         }
-        float mx = lane < 36 ? hv : 0.0f;
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
-        mx = fmaxf(0.0f, mx);
+        // the values are not negative: their order is that of their bits
+        const float mx = __uint_as_float(wave_max_u32(__float_as_uint(hv)));
         const float thr = mx * 0.8f;
-        const float pv = __shfl(hv, lane < 36 ? (lane + 35) % 36 : lane, 64);
-        const float nv = __shfl(hv, lane < 36 ? (lane + 1) % 36 : lane, 64);
+        const float pv = from_lane(prev4, hv), nv = from_lane(next4, hv);
         const bool peak = lane < 36 && hv >= thr && hv > pv && hv > nv;
         const unsigned long long m = ballot64(peak);
         if (peak) {
@@ -1123,11 +1208,13 @@ __global__ __launch_bounds__(64) void k_orient(const OctaveDesc* __restrict__ oc
             const float step = kTwoPi / 36.0f;
             const float center = ((float)lane + 0.5f) * step;
             const float a = center + off * step;
-            float fa = rem_euclid(a, kTwoPi);
+            // rem_euclid: a itself but for the first and last bins' edges
+            float fa = a;
+            if (!(a >= 0.0f && a < kTwoPi)) fa = rem_euclid(a, kTwoPi);
             if (fa > kPi) fa = fa - kTwoPi;
             if (rank < kMaxPeaks) angles[(size_t)c * kMaxPeaks + rank] = fa;
         }
-        if (lane == 0) npeaks[c] = (unsigned)min(__popcll(m), kMaxPeaks);
+        if (lane == 0) npeaks[c] = min((unsigned)__popcll(m), (unsigned)kMaxPeaks);
         __syncthreads();
     }
 }
@@ -1182,18 +1269,6 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
     x = __float_as_int(__int_as_float(x) + __int_as_float(__builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false)));
     x = __float_as_int(__int_as_float(x) + __int_as_float(__builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false)));
     return __int_as_float(__builtin_amdgcn_readlane(x, 63));
-}
-
-// Maximum over the 64 lanes of a fully active wave (DPP, as wave_incl_scan),
-// returned to every lane.
-__device__ __forceinline__ unsigned wave_max_u32(unsigned x) {
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true));  // row_shr:1
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true));  // row_shr:2
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true));  // row_shr:4
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true));  // row_shr:8
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false)); // row_bcast:15
-    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false)); // row_bcast:31
-    return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
 }
 
 // Maximum over the 64 lanes of a fully active wave, returned to every lane.
