@@ -782,17 +782,12 @@ __global__ __launch_bounds__(kThreads) void k_compact(const OctaveDesc* __restri
 // ---------------------------------------------------------------------------
 // k_refine: one thread per candidate; the reference's arithmetic in the same
 // f32 operation order (compiled without FMA contraction).
+// Bound by the gathers: a step reads 3 rows of 4 Gaussian levels, most lines of the
+// pyramid in all. A word for the 3 texels of a row (12 loads a step instead of 38 of
+// single bytes): 64 x 1920x1080 190 -> 156 us.
 // ---------------------------------------------------------------------------
-struct DogView {
-    const uint8_t* levels;
-    long long stride;
-    int pitch, w, h;
-    __device__ __forceinline__ float at(int l, int x, int y) const {
-        x = min(max(x, 0), w - 1);
-        y = min(max(y, 0), h - 1);
-        const uint8_t* g0 = levels + (long long)l * stride + (size_t)y * pitch + x;
-        return q255f((float)g0[stride]) - q255f((float)g0[0]);
-    }
+struct __attribute__((packed)) UnalignedWord {
+    unsigned v;
 };
 
 __global__ __launch_bounds__(kThreads) void k_refine(const OctaveDesc* __restrict__ oct,
@@ -807,35 +802,51 @@ __global__ __launch_bounds__(kThreads) void k_refine(const OctaveDesc* __restric
         const Cand cd = cand[c];
         const OctaveDesc& O = oct[cd.job];
         const ImageParams& P = params[O.img];
-        DogView V{O.levels, O.level_stride, O.pitch, O.w, O.h};
         const int nd = P.num_intervals + 2;  // DoG layers per octave
         const float scale0 = pow2f(O.octave);
         // kp.x / 2^o of the candidate ((x + 0.5) * 2^o), `as i32` (src/sift.rs:309-313)
         const float xi = (((float)cd.x + 0.5f) * scale0) / scale0;
         const float yi = (((float)cd.y + 0.5f) * scale0) / scale0;
         int cx = f2i_sat(xi), cy = f2i_sat(yi), cl = cd.layer;
-        if (cand_resp) cand_resp[c] = V.at(cd.layer, cd.x, cd.y);
+        if (cand_resp) {
+            const uint8_t* g0 = O.levels + (long long)cd.layer * O.level_stride +
+                                ((size_t)cd.y * O.pitch + cd.x);
+            cand_resp[c] = q255f((float)g0[O.level_stride]) - q255f((float)g0[0]);
+        }
         int ok = 0;
         Keypoint r;
         for (int step = 0; step < 5; step++) {
             if (cl < 1 || cl >= nd - 1) break;
             if (cx < 1 || cx >= O.w - 1 || cy < 1 || cy >= O.h - 1) break;
-            const float pxp = V.at(cl, cx + 1, cy), pxm = V.at(cl, cx - 1, cy);
-            const float pyp = V.at(cl, cx, cy + 1), pym = V.at(cl, cx, cy - 1);
-            const float nxt = V.at(cl + 1, cx, cy), prv = V.at(cl - 1, cx, cy);
+            // the 3x3 texels around (cx, cy) of the four Gaussian levels cl - 1 .. cl + 2,
+            // a row by one word (columns cx - 1 .. cx + 2: cx + 2 <= w, and a byte past
+            // the last level's last row is still the arena's)
+            unsigned t[4][3];
+            const uint8_t* lv = O.levels + (long long)(cl - 1) * O.level_stride +
+                                ((size_t)(cy - 1) * O.pitch + (cx - 1));
+#pragma unroll
+            for (int l = 0; l < 4; l++, lv += O.level_stride)
+#pragma unroll
+                for (int r = 0; r < 3; r++)
+                    t[l][r] = reinterpret_cast<const UnalignedWord*>(lv + r * O.pitch)->v;
+            // DoG layer cl - 1 + l at row cy - 1 + r, column cx - 1 + x
+            auto dog = [&](int l, int r, int x) {
+                return q255f((float)((t[l + 1][r] >> (8 * x)) & 0xffu)) -
+                       q255f((float)((t[l][r] >> (8 * x)) & 0xffu));
+            };
+            const float pxp = dog(1, 1, 2), pxm = dog(1, 1, 0);
+            const float pyp = dog(1, 2, 1), pym = dog(1, 0, 1);
+            const float nxt = dog(2, 1, 1), prv = dog(0, 1, 1);
             const float dx = (pxp - pxm) / 2.0f;
             const float dy = (pyp - pym) / 2.0f;
             const float ds = (nxt - prv) / 2.0f;
-            const float cv = V.at(cl, cx, cy);
+            const float cv = dog(1, 1, 1);
             const float dxx = pxp + pxm - 2.0f * cv;
             const float dyy = pyp + pym - 2.0f * cv;
             const float dss = nxt + prv - 2.0f * cv;
-            const float dxy = (V.at(cl, cx + 1, cy + 1) - V.at(cl, cx - 1, cy + 1) -
-                               V.at(cl, cx + 1, cy - 1) + V.at(cl, cx - 1, cy - 1)) / 4.0f;
-            const float dxs = (V.at(cl + 1, cx + 1, cy) - V.at(cl + 1, cx - 1, cy) -
-                               (V.at(cl - 1, cx + 1, cy) - V.at(cl - 1, cx - 1, cy))) / 4.0f;
-            const float dys = (V.at(cl + 1, cx, cy + 1) - V.at(cl + 1, cx, cy - 1) -
-                               (V.at(cl - 1, cx, cy + 1) - V.at(cl - 1, cx, cy - 1))) / 4.0f;
+            const float dxy = (dog(1, 2, 2) - dog(1, 2, 0) - dog(1, 0, 2) + dog(1, 0, 0)) / 4.0f;
+            const float dxs = (dog(2, 1, 2) - dog(2, 1, 0) - (dog(0, 1, 2) - dog(0, 1, 0))) / 4.0f;
+            const float dys = (dog(2, 2, 1) - dog(2, 0, 1) - (dog(0, 2, 1) - dog(0, 0, 1))) / 4.0f;
             // solve_linear_system (src/sift.rs:478-503), b = -g
             const float a00 = dxx, a01 = dxy, a02 = dxs, a10 = dxy, a11 = dyy, a12 = dys,
                         a20 = dxs, a21 = dys, a22 = dss;
