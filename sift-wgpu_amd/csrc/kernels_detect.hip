@@ -790,7 +790,12 @@ struct __attribute__((packed)) UnalignedWord {
     unsigned v;
 };
 
-__global__ __launch_bounds__(kThreads) void k_refine(const OctaveDesc* __restrict__ oct,
+// Work-groups of one wave: the gathers of the few waves a single frame has are bound
+// by a CU's requests, so they are spread over all CUs (640x480: 17.5 us with groups of
+// four waves, 12.0 us; 1920x1080 19.1 and 13.4; 64 frames 157 and 151).
+constexpr int kRefineThreads = 64;
+
+__global__ __launch_bounds__(kRefineThreads) void k_refine(const OctaveDesc* __restrict__ oct,
                                                      const ImageParams* __restrict__ params,
                                                      const Cand* __restrict__ cand,
                                                      const unsigned* __restrict__ total, int cap,
@@ -798,7 +803,7 @@ __global__ __launch_bounds__(kThreads) void k_refine(const OctaveDesc* __restric
                                                      int* __restrict__ valid,
                                                      float* __restrict__ cand_resp) {
     const int n = (int)min(*total, (unsigned)cap);
-    for (int c = blockIdx.x * kThreads + threadIdx.x; c < n; c += gridDim.x * kThreads) {
+    for (int c = blockIdx.x * kRefineThreads + threadIdx.x; c < n; c += gridDim.x * kRefineThreads) {
         const Cand cd = cand[c];
         const OctaveDesc& O = oct[cd.job];
         const ImageParams& P = params[O.img];
@@ -2229,7 +2234,7 @@ static bool queue_enabled() {
 void launch_refine(const OctaveDesc* d_oct, const ImageParams* d_params, const Cand* d_cand,
                    const unsigned* d_total, int cap, Keypoint* d_ref, int* d_valid,
                    float* d_cand_resp, hipStream_t s) {
-    hipLaunchKernelGGL(k_refine, dim3(grid_for(cap, kThreads, 2048)), dim3(kThreads), 0, s, d_oct,
+    hipLaunchKernelGGL(k_refine, dim3(grid_for(cap, kRefineThreads, 8192)), dim3(kRefineThreads), 0, s, d_oct,
                        d_params, d_cand, d_total, cap, d_ref, d_valid, d_cand_resp);
 }
 
@@ -2238,10 +2243,14 @@ void launch_orient(const OctaveDesc* d_oct, const ImageParams* d_params, const C
                    unsigned* d_npeaks, float* d_angles, unsigned* d_queue, hipStream_t s) {
     // work queue: as many work-groups as fit, each taking keypoints until none
     // are left; or grid-stride over the candidates with many more work-groups
-    // than fit at once (each takes only a few keypoints, so the launch ends evenly)
+    // than fit at once (each takes only a few keypoints, so the launch ends evenly).
+    // Where the capacity says few candidates, half as many: the groups beyond the
+    // count only start and end (640x480 17.6 us with 65536, 11.0 with 32768;
+    // 1920x1080 22.5 and 19.5), while 64 frames take 648 us with 32768 and 630 with 65536.
+    const int most = cap <= kDescOneLaunchCap ? 32768 : 65536;
     const bool q = queue_enabled();
-    const int grid = q ? std::min(resident_groups((const void*)k_orient, 64), grid_for(cap, 1, 65536))
-                       : grid_for(cap, 1, 65536);
+    const int grid = q ? std::min(resident_groups((const void*)k_orient, 64), grid_for(cap, 1, most))
+                       : grid_for(cap, 1, most);
     // (d_queue: kNumXcd counters)
     hipLaunchKernelGGL(k_orient, dim3(grid), dim3(64), 0, s, d_oct, d_params, d_cand, d_total, cap,
                        d_ref, d_valid, d_npeaks, d_angles, q ? d_queue : nullptr);
