@@ -1342,12 +1342,12 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         prof_end(K_ORIENT, 0.0, ev);
         prof_begin(K_SCAN, 0.0, &ev);
         launch_keypoint_offsets(d_npk, cap, d_total, d_koff, (unsigned*)AP(scantmp2_off), d_offs,
-                                (const int*)(D + isb_blob), n, d_sum, B.ext ? B.ext->offsets : nullptr, st);
+                                (const int*)(D + isb_blob), n, d_sum, B.ext ? B.ext->offsets : nullptr, (int*)AP(mid_off), st);
         prof_end(K_SCAN, 0.0, ev);
         prof_begin(K_DESCRIPTOR, 0.0, &ev);
         launch_descriptor(d_oct, d_par, d_cand, d_total, cap, d_ref, d_npk, d_ang, d_koff, kcap, d_kps,
                           d_desc, d_counts + nslots, (int*)AP(wide_off), d_counts + nslots + 1,
-                          (int*)AP(mid_off), d_counts + nslots + 2 + kNumXcd, max_radius, st);
+                          (int*)AP(mid_off), d_counts + nslots + 2 + kNumXcd, d_sum + 1, max_radius, st);
         prof_end(K_DESCRIPTOR, 0.0, ev);
         if (B.desc_u8) {
             prof_begin(K_DESC_U8, 0.0, &ev);

@@ -566,10 +566,19 @@ __global__ __launch_bounds__(kThreads) void k_scan_tiles(unsigned* __restrict__ 
     }
 }
 
+// The candidate of every keypoint, for the descriptor's work-groups (owner may be null;
+// keypoints past its size are searched for): candidate c has the keypoints [k, e).
+__device__ __forceinline__ void mark_owner(int* __restrict__ owner, int size, int c, unsigned k,
+                                           unsigned e) {
+    for (; k < e; k++)
+        if (k < (unsigned)size) owner[k] = c;
+}
+
 __global__ __launch_bounds__(kThreads) void k_scan_down(const unsigned* __restrict__ in, int n_max,
                                                         const unsigned* n_dev,
                                                         const unsigned* __restrict__ tile_prefix,
-                                                        unsigned* __restrict__ out) {
+                                                        unsigned* __restrict__ out,
+                                                        int* __restrict__ owner) {
     __shared__ unsigned sh[8];
     const int n = scan_n(n_max, n_dev);
     const int base = blockIdx.x * kScanTile + threadIdx.x * 16;
@@ -581,6 +590,14 @@ __global__ __launch_bounds__(kThreads) void k_scan_down(const unsigned* __restri
     unsigned tot;
     unsigned ex = block_excl_scan(s, sh, tot);
     const unsigned end = scan_store16(out, base, n, v, tile_prefix[blockIdx.x] + ex);
+    if (owner) {
+        unsigned k = tile_prefix[blockIdx.x] + ex;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            mark_owner(owner, n_max, base + i, k, k + v[i]);
+            k += v[i];
+        }
+    }
     if (base < n && base + 16 >= n) out[n] = end;
     if (n == 0 && blockIdx.x == 0 && threadIdx.x == 0) out[0] = 0;
 }
@@ -624,7 +641,8 @@ constexpr int kScanSingleThreads = 1024;
 constexpr int kScanSingleMax = 1 << 16;
 __global__ __launch_bounds__(kScanSingleThreads) void k_scan_single(const unsigned* __restrict__ in,
                                                                    int n_max, const unsigned* n_dev,
-                                                                   unsigned* out, FinalizeArgs F) {
+                                                                   unsigned* out, FinalizeArgs F,
+                                                                   int* __restrict__ owner) {
     __shared__ unsigned sh[kScanSingleThreads / 64];
     const int n = scan_n(n_max, n_dev);
     unsigned carry = 0;
@@ -644,6 +662,22 @@ __global__ __launch_bounds__(kScanSingleThreads) void k_scan_single(const unsign
     if (F.summary) {
         __threadfence_block();
         __syncthreads();  // the offsets just written are read back
+        if (owner) {
+            // neighbouring lanes write neighbouring words, the offsets of four candidates
+            // of a lane loaded at once
+            constexpr int kU = 4;
+            for (int c = threadIdx.x; c < n; c += kScanSingleThreads * kU) {
+                unsigned k[kU], e[kU];
+#pragma unroll
+                for (int j = 0; j < kU; j++) {
+                    const int cj = c + j * kScanSingleThreads;
+                    k[j] = cj < n ? out[cj] : 0u;
+                    e[j] = cj < n ? out[cj + 1] : 0u;
+                }
+#pragma unroll
+                for (int j = 0; j < kU; j++) mark_owner(owner, n_max, c + j * kScanSingleThreads, k[j], e[j]);
+            }
+        }
         for (int i = threadIdx.x; i <= F.nimg; i += kScanSingleThreads) finalize_entry(F, i);
     }
 }
@@ -1580,7 +1614,25 @@ __device__ __forceinline__ void desc_finish(const unsigned* hist, float fix, dou
 // 2^20 times the largest power of two that keeps the patch's texel range times
 // it within 255 (desc_range_exp). Wave 0 sums the copies and normalises.
 // ---------------------------------------------------------------------------
-template <int MR, bool kFromList>
+// The candidate of keypoint k: from the list of the first `size` (mark_owner), or the
+// last one of the n whose offset is at most k.
+__device__ __forceinline__ int desc_owner(const int* __restrict__ owner, const unsigned* __restrict__ koff,
+                                          unsigned n, int size, int k) {
+    if (k < size) return owner[k];
+    unsigned lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const unsigned mid = (lo + hi + 1) >> 1;
+        if (koff[mid] <= (unsigned)k) lo = mid;
+        else hi = mid - 1;
+    }
+    return (int)lo;
+}
+
+// The items of a launch of k_descriptor: every candidate with all its peaks, the
+// candidates of a list, or single keypoints (a candidate's peaks apart).
+enum class DescItems { kAll, kList, kPeaks };
+
+template <int MR, DescItems kItems>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descriptor(
     const OctaveDesc* __restrict__ oct, const ImageParams* __restrict__ params,
@@ -1620,7 +1672,8 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
     float2* const gcol = kTermsInPatch ? reinterpret_cast<float2*>(patch + kPatchBytes) : terms_own;
     float2* const grw = gcol + kGS;
     // all candidates, or the ones an instantiation for smaller windows listed
-    const int n = (int)min(kFromList ? *in_count : *total, (unsigned)cap);
+    const int n = (int)min(kItems == DescItems::kAll ? *total : *in_count,
+                           (unsigned)(kItems == DescItems::kPeaks ? kcap : cap));
     __shared__ int qslot[2];
     WorkQueue<kDescChunk> Q{queue, 0, 0, 0};
     for (int idx = Q.first(qslot); idx < n; idx = Q.next(qslot, idx)) {
@@ -1632,11 +1685,15 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
         int tid = (int)threadIdx.x;
         asm volatile("" : "+v"(tid));
         const int wave = tid >> 6, lane = tid & 63;
-        const int c = kFromList ? in_list[idx] : idx;
+        const int c = kItems == DescItems::kList    ? in_list[idx]
+                      : kItems == DescItems::kPeaks ? desc_owner(in_list, koff, min(*total, (unsigned)cap), cap, idx)
+                                                    : idx;
         const DescGeom G = desc_geom(c, oct, params, cand, ref, npeaks, koff);
         if (G.np == 0) continue;
+        const int pk0 = kItems == DescItems::kPeaks ? idx - (int)G.k0 : 0;
+        const int pk1 = kItems == DescItems::kPeaks ? pk0 + 1 : G.np;
         if (G.R > MR) {  // wider windows: listed for the next instantiation
-            if (threadIdx.x == 0) out_list[atomicAdd(out_count, 1u)] = c;
+            if (threadIdx.x == 0 && pk0 == 0) out_list[atomicAdd(out_count, 1u)] = c;
             continue;
         }
         const int R = G.R, side = G.side, gside = 2 * R + 3;
@@ -1810,7 +1867,7 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
         // in each place of use
         float inv_bw = 1.0f / bw;
         asm volatile("" : "+v"(inv_bw));
-        for (int pk = 0; pk < G.np; pk++) {
+        for (int pk = pk0; pk < pk1; pk++) {
             const float angle = uniform_f(pang[pk]);
             for (int i = tid; i < kHistCopies * kHistWords / 4; i += kThreads)
                 reinterpret_cast<uint4*>(hist)[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -2154,17 +2211,17 @@ void launch_extrema_tile(int S, int strip_rows, const OctaveDesc* d_oct, int noc
 // n_dev may be null (then n_max is the count). out needs n_max+1 entries;
 // tmp needs ceil(n_max/4096)+1 entries. Returns whether fin (may be null) was done.
 static bool scan(const unsigned* d_in, int n_max, const unsigned* n_dev, unsigned* d_out,
-                 unsigned* d_tmp, const FinalizeArgs* fin, hipStream_t s) {
+                 unsigned* d_tmp, const FinalizeArgs* fin, int* d_owner, hipStream_t s) {
     if (n_max <= kScanSingleMax) {
         hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(kScanSingleThreads), 0, s, d_in, n_max, n_dev,
-                           d_out, fin ? *fin : FinalizeArgs{});
+                           d_out, fin ? *fin : FinalizeArgs{}, d_owner);
         return true;
     }
     const int tiles = n_max > 0 ? (n_max + kScanTile - 1) / kScanTile : 1;
     hipLaunchKernelGGL(k_scan_reduce, dim3(tiles), dim3(kThreads), 0, s, d_in, n_max, n_dev, d_tmp);
     hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kThreads), 0, s, d_tmp, tiles);
     hipLaunchKernelGGL(k_scan_down, dim3(tiles), dim3(kThreads), 0, s, d_in, n_max, n_dev, d_tmp,
-                       d_out);
+                       d_out, d_owner);
     return false;
 }
 
@@ -2180,7 +2237,7 @@ void launch_compact(const OctaveDesc* d_oct, int noct, int nslots, const unsigne
                            noct, nslots, d_bits, d_counts, d_offsets, d_cand, cap, spw);
         return;
     }
-    (void)scan(d_counts, nslots, nullptr, d_offsets, d_tmp, nullptr, s);
+    (void)scan(d_counts, nslots, nullptr, d_offsets, d_tmp, nullptr, nullptr, s);
     if (nslots <= 0) return;
     const int spw = nslots >= 65536 ? kCompactSlots : 1;  // slots per wave
     const int per = (kThreads / 64) * spw;                 // slots per work-group
@@ -2190,9 +2247,9 @@ void launch_compact(const OctaveDesc* d_oct, int noct, int nslots, const unsigne
 
 void launch_keypoint_offsets(const unsigned* d_npeaks, int cap, const unsigned* d_total, unsigned* d_koff,
                              unsigned* d_tmp, const unsigned* d_slot_offsets, const int* d_img_slot_begin,
-                             int nimg, unsigned* d_summary, unsigned* d_out_offsets, hipStream_t s) {
+                             int nimg, unsigned* d_summary, unsigned* d_out_offsets, int* d_owner, hipStream_t s) {
     const FinalizeArgs F{d_slot_offsets, d_img_slot_begin, nimg, d_koff, d_total, cap, d_summary, d_out_offsets};
-    if (!scan(d_npeaks, cap, d_total, d_koff, d_tmp, &F, s))
+    if (!scan(d_npeaks, cap, d_total, d_koff, d_tmp, &F, cap <= kDescOneLaunchCap ? d_owner : nullptr, s))
         hipLaunchKernelGGL(k_finalize, dim3((nimg + 1 + 255) / 256), dim3(256), 0, s, F);
 }
 
@@ -2261,23 +2318,29 @@ void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, con
                        const unsigned* d_npeaks, const float* d_angles, const unsigned* d_koff,
                        int kcap, Keypoint* d_kps, float* d_desc, unsigned* d_wide_count,
                        int* d_wide_list, unsigned* d_mid_count, int* d_mid_list, unsigned* d_queues,
-                       int max_radius, hipStream_t s) {
+                       const unsigned* d_count, int max_radius, hipStream_t s) {
     // as k_orient: a work queue, or few keypoints per work-group. Windows up to
     // kDescSmallR run at 8 work-groups per CU and list the few others for the
     // kDescMaxR instantiation (6 per CU), which lists still wider ones for
     // k_descriptor_wide. d_queues: the two instantiations' queue counters
-    // (kNumXcd each).
+    // (kNumXcd each). d_count: the number of keypoints.
     const bool q = queue_enabled();
     if (cap <= kDescOneLaunchCap) {
-        // few candidates (small frames): one launch of the wide instantiation
-        // over all of them; the GPU is far from full, so its lower occupancy
-        // costs less than the second launch's latency
-        const void* kall = (const void*)k_descriptor<kDescMaxR, false>;
-        const int g = q ? std::min(resident_groups(kall, kThreads), grid_for(cap, 1, 49152))
-                        : grid_for(cap, 1, 49152);
-        hipLaunchKernelGGL((k_descriptor<kDescMaxR, false>), dim3(g), dim3(kThreads), 0, s, d_oct,
+        // few candidates (single frames, small batches): one launch of the wide
+        // instantiation; the GPU is far from full, so its lower occupancy costs less
+        // than the second launch's latency. It takes keypoints rather than candidates
+        // (d_mid_list holds their candidates): the launch lasts as long as its
+        // longest group, and a candidate's two to four peaks one after the other
+        // were that (640x480: 59 us, 30 us so, and 1 us more in the offsets' scan;
+        // 1920x1080: 97 and 82, 4 more), while the patch and grid that the peaks then
+        // each make are work for idle CUs. Full launches keep the peaks together.
+        const void* kall = (const void*)k_descriptor<kDescMaxR, DescItems::kPeaks>;
+        const int most = 16384;  // 4096: 84 us at 1920x1080; 8192 to 49152: the same
+        const int g = q ? std::min(resident_groups(kall, kThreads), grid_for(kcap, 1, most))
+                        : grid_for(kcap, 1, most);
+        hipLaunchKernelGGL((k_descriptor<kDescMaxR, DescItems::kPeaks>), dim3(g), dim3(kThreads), 0, s, d_oct,
                            d_params, d_cand, d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap,
-                           d_kps, d_desc, nullptr, nullptr, d_wide_count, d_wide_list,
+                           d_kps, d_desc, d_count, d_mid_list, d_wide_count, d_wide_list,
                            q ? d_queues + kNumXcd : nullptr);
         if (max_radius > kDescMaxR)
             hipLaunchKernelGGL(k_descriptor_wide, dim3(kWideGroups), dim3(kThreads), 0, s, d_oct, d_params, d_cand,
@@ -2285,15 +2348,15 @@ void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, con
                                d_wide_count, d_wide_list);
         return;
     }
-    const void* k28 = (const void*)k_descriptor<kDescSmallR, false>;
-    const void* k31 = (const void*)k_descriptor<kDescMaxR, true>;
+    const void* k28 = (const void*)k_descriptor<kDescSmallR, DescItems::kAll>;
+    const void* k31 = (const void*)k_descriptor<kDescMaxR, DescItems::kList>;
     const int g28 = q ? std::min(resident_groups(k28, kThreads), grid_for(cap, 1, 49152)) : grid_for(cap, 1, 49152);
     const int g31 = q ? std::min(resident_groups(k31, kThreads), grid_for(cap, 1, 49152)) : grid_for(cap, 1, 49152);
-    hipLaunchKernelGGL((k_descriptor<kDescSmallR, false>), dim3(g28), dim3(kThreads), 0, s, d_oct,
+    hipLaunchKernelGGL((k_descriptor<kDescSmallR, DescItems::kAll>), dim3(g28), dim3(kThreads), 0, s, d_oct,
                        d_params, d_cand, d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap,
                        d_kps, d_desc, nullptr, nullptr, d_mid_count, d_mid_list, q ? d_queues : nullptr);
     if (max_radius <= kDescSmallR) return;
-    hipLaunchKernelGGL((k_descriptor<kDescMaxR, true>), dim3(g31), dim3(kThreads), 0, s, d_oct,
+    hipLaunchKernelGGL((k_descriptor<kDescMaxR, DescItems::kList>), dim3(g31), dim3(kThreads), 0, s, d_oct,
                        d_params, d_cand, d_total, cap, d_ref, d_npeaks, d_angles, d_koff, kcap,
                        d_kps, d_desc, d_mid_count, d_mid_list, d_wide_count, d_wide_list,
                        q ? d_queues + kNumXcd : nullptr);

@@ -177,10 +177,11 @@ void launch_compact(const OctaveDesc* d_oct, int noct, int nslots, const unsigne
 // Keypoint offsets (exclusive sums of the candidates' peak counts) and the
 // summary: summary[0] = candidates, summary[1] = keypoints, summary[2..2+nimg] =
 // per-image keypoint offsets (nimg+1 entries), the offsets also to
-// d_out_offsets when it is not null. d_tmp: ceil(cap / 4096) + 1 entries.
+// d_out_offsets when it is not null. d_tmp: ceil(cap / 4096) + 1 entries. d_owner: the
+// candidates of the first cap keypoints, where the descriptor takes them one by one.
 void launch_keypoint_offsets(const unsigned* d_npeaks, int cap, const unsigned* d_total, unsigned* d_koff,
                              unsigned* d_tmp, const unsigned* d_slot_offsets, const int* d_img_slot_begin,
-                             int nimg, unsigned* d_summary, unsigned* d_out_offsets, hipStream_t s);
+                             int nimg, unsigned* d_summary, unsigned* d_out_offsets, int* d_owner, hipStream_t s);
 void launch_refine(const OctaveDesc* d_oct, const ImageParams* d_params, const Cand* d_cand,
                    const unsigned* d_total, int cap, Keypoint* d_ref, int* d_valid,
                    float* d_cand_resp, hipStream_t s);
@@ -195,7 +196,7 @@ void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, con
                        const unsigned* d_npeaks, const float* d_angles, const unsigned* d_koff,
                        int kcap, Keypoint* d_kps, float* d_desc, unsigned* d_wide_count,
                        int* d_wide_list, unsigned* d_mid_count, int* d_mid_list, unsigned* d_queues,
-                       int max_radius, hipStream_t s);
+                       const unsigned* d_count, int max_radius, hipStream_t s);
 // An upper bound of the descriptor radius of any keypoint with these parameters
 // (launch_descriptor's max_radius: instantiations for larger windows are left out).
 int descriptor_max_radius(float sigma, int intervals);
