@@ -553,53 +553,12 @@ __global__ __launch_bounds__(kThreads) void k_scan_reduce(const unsigned* __rest
     if (threadIdx.x == 0) tile_sums[blockIdx.x] = tot;
 }
 
-__global__ __launch_bounds__(kThreads) void k_scan_tiles(unsigned* __restrict__ tile_sums, int ntiles) {
-    __shared__ unsigned sh[8];
-    unsigned carry = 0;
-    for (int b = 0; b < ntiles; b += kThreads) {
-        int k = b + threadIdx.x;
-        unsigned v = k < ntiles ? tile_sums[k] : 0u;
-        unsigned tot;
-        unsigned ex = block_excl_scan(v, sh, tot);
-        if (k < ntiles) tile_sums[k] = carry + ex;
-        carry += tot;
-    }
-}
-
 // The candidate of every keypoint, for the descriptor's work-groups (owner may be null;
 // keypoints past its size are searched for): candidate c has the keypoints [k, e).
 __device__ __forceinline__ void mark_owner(int* __restrict__ owner, int size, int c, unsigned k,
                                            unsigned e) {
     for (; k < e; k++)
         if (k < (unsigned)size) owner[k] = c;
-}
-
-__global__ __launch_bounds__(kThreads) void k_scan_down(const unsigned* __restrict__ in, int n_max,
-                                                        const unsigned* n_dev,
-                                                        const unsigned* __restrict__ tile_prefix,
-                                                        unsigned* __restrict__ out,
-                                                        int* __restrict__ owner) {
-    __shared__ unsigned sh[8];
-    const int n = scan_n(n_max, n_dev);
-    const int base = blockIdx.x * kScanTile + threadIdx.x * 16;
-    unsigned v[16];
-    unsigned s = 0;
-    scan_load16(in, base, n, v);
-#pragma unroll
-    for (int i = 0; i < 16; i++) s += v[i];
-    unsigned tot;
-    unsigned ex = block_excl_scan(s, sh, tot);
-    const unsigned end = scan_store16(out, base, n, v, tile_prefix[blockIdx.x] + ex);
-    if (owner) {
-        unsigned k = tile_prefix[blockIdx.x] + ex;
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            mark_owner(owner, n_max, base + i, k, k + v[i]);
-            k += v[i];
-        }
-    }
-    if (base < n && base + 16 >= n) out[n] = end;
-    if (n == 0 && blockIdx.x == 0 && threadIdx.x == 0) out[0] = 0;
 }
 
 // Per-image keypoint ranges: summary[2+i] = koff[first candidate of image i]
@@ -615,21 +574,64 @@ struct FinalizeArgs {
     unsigned* summary;
     unsigned* out_offsets;
 };
-__device__ __forceinline__ void finalize_entry(const FinalizeArgs& F, int i) {
+// Image i's range (i <= nimg; 0 writes the totals too), where owned(index) says that
+// the work-group has written the offset of that index.
+template <typename Owned>
+__device__ __forceinline__ void finalize_entry(const FinalizeArgs& F, int i, Owned owned) {
     const unsigned n = min(*F.total, (unsigned)F.cap);
     const unsigned cb = min(F.slot_offsets[F.img_slot_begin[i]], n);
-    const unsigned k = F.koff[cb];
-    F.summary[2 + i] = k;
-    if (F.out_offsets) F.out_offsets[i] = k;
-    if (i == 0) {
+    if (owned(cb)) {
+        const unsigned k = F.koff[cb];
+        F.summary[2 + i] = k;
+        if (F.out_offsets) F.out_offsets[i] = k;
+    }
+    if (i == 0 && owned(n)) {
         F.summary[0] = *F.total;
         F.summary[1] = F.koff[n];
     }
 }
 
-__global__ void k_finalize(FinalizeArgs F) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i <= F.nimg) finalize_entry(F, i);
+// The second launch of a scan: every work-group adds the sums of the tiles before its
+// own (the offsets' 4 M of 64 frames are 1012 tiles, four loads of a thread), which
+// saves a launch between, and the keypoint offsets' scan (F.summary set) writes the
+// image ranges that begin in the tile, which saves one after it (4 to 5 us each).
+__global__ __launch_bounds__(kThreads) void k_scan_down(const unsigned* __restrict__ in, int n_max,
+                                                        const unsigned* n_dev,
+                                                        const unsigned* __restrict__ tile_sums,
+                                                        unsigned* out, FinalizeArgs F,
+                                                        int* __restrict__ owner) {
+    __shared__ unsigned sh[8];
+    const int n = scan_n(n_max, n_dev);
+    const int first = blockIdx.x * kScanTile, base = first + threadIdx.x * 16;
+    if (first > 0 && first >= n) return;
+    unsigned v[16];
+    unsigned s = 0, before = 0, prefix, tot;
+    scan_load16(in, base, n, v);
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += kThreads) before += tile_sums[i];
+#pragma unroll
+    for (int i = 0; i < 16; i++) s += v[i];
+    block_excl_scan(before, sh, prefix);
+    unsigned k = prefix + block_excl_scan(s, sh, tot);
+    const unsigned end = scan_store16(out, base, n, v, k);
+    if (base < n && base + 16 >= n) out[n] = end;
+    if (n == 0 && threadIdx.x == 0) out[0] = 0;
+    if (owner) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            mark_owner(owner, n_max, base + i, k, k + v[i]);
+            k += v[i];
+        }
+    }
+    if (F.summary) {
+        __threadfence_block();
+        __syncthreads();  // the offsets just written are read back
+        const unsigned last = min(first + kScanTile, n) - 1u;  // ~0u if n = 0
+        auto owned = [&](unsigned i) {
+            return (i >= (unsigned)first && i < (unsigned)n && i - (unsigned)first < (unsigned)kScanTile) ||
+                   (i == (unsigned)n && last + 1u == (unsigned)n);
+        };
+        for (int i = threadIdx.x; i <= F.nimg; i += kThreads) finalize_entry(F, i, owned);
+    }
 }
 
 // The same scan in one work-group of 1024 threads, for few elements (single
@@ -678,7 +680,7 @@ __global__ __launch_bounds__(kScanSingleThreads) void k_scan_single(const unsign
                 for (int j = 0; j < kU; j++) mark_owner(owner, n_max, c + j * kScanSingleThreads, k[j], e[j]);
             }
         }
-        for (int i = threadIdx.x; i <= F.nimg; i += kScanSingleThreads) finalize_entry(F, i);
+        for (int i = threadIdx.x; i <= F.nimg; i += kScanSingleThreads) finalize_entry(F, i, [](unsigned) { return true; });
     }
 }
 
@@ -692,10 +694,13 @@ __global__ __launch_bounds__(kScanSingleThreads) void k_scan_single(const unsign
 // their loads overlap. For each slot the set bits are ranked with popcounts and
 // a wave prefix sum and the candidates written at offsets[slot] + rank, i.e. in
 // the reference's order. Rows of more than 64 words take a chunked loop.
-// kScan: the work-group sums the counts of all slots before its own itself and
-// writes its slots' offsets (and the total), which saves the scan its launch: a
+// The work-group sums the counts of all slots before its own itself (with many
+// slots, from the sums of 4096-slot tiles and the counts of its own tile) and writes
+// its slots' offsets (and the total), which saves the scan's other launches: a
 // single frame's few thousand counts lie in L2 (1920 x 1080: 25 KB, 13 KB per
-// work-group on average), where the scan in one work-group took 5 to 10 us.
+// work-group on average), where the scan in one work-group took 5 to 10 us; with the
+// tiles' sums one launch goes before where two or three did (16 frames of 640 x 480
+// 36 -> 25 us).
 // ---------------------------------------------------------------------------
 constexpr int kCompactSlots = 8;
 
@@ -727,53 +732,48 @@ __device__ __forceinline__ void compact_word(unsigned long long m, int wi, int j
     base += tot;
 }
 
-template <bool kScan>
 __global__ __launch_bounds__(kThreads) void k_compact(const OctaveDesc* __restrict__ oct, int noct,
                                                       int nslots,
                                                       const unsigned long long* __restrict__ bits,
                                                       const unsigned* __restrict__ counts,
+                                                      const unsigned* __restrict__ tile_sums,
                                                       unsigned* __restrict__ offsets,
                                                       Cand* __restrict__ cand, int cap, int spw) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int s0 = (blockIdx.x * (kThreads / 64) + wave) * spw;
     const int ns = min(spw, nslots - s0);
-    unsigned cnt_l, off_l;
-    if constexpr (kScan) {
-        __shared__ unsigned wsum[kThreads / 64];
-        const int per = (kThreads / 64) * spw, first = blockIdx.x * per;  // slots of the work-group, <= 64
-        unsigned p = 0;
-        for (int i = threadIdx.x * 4; i < first; i += kThreads * 4) {  // first is a multiple of 4
-            const uint4 v = *reinterpret_cast<const uint4*>(counts + i);
-            p += (v.x + v.y) + (v.z + v.w);
-        }
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) p += __shfl_xor(p, d, 64);
-        if (lane == 0) wsum[wave] = p;
-        const int slot = first + lane;
-        const bool mine = lane < per && slot < nslots;
-        const unsigned c = mine ? counts[slot] : 0u;
-        unsigned x = c;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const unsigned t = __shfl_up(x, d, 64);
-            if (lane >= d) x += t;
-        }
-        __syncthreads();
-        x += (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
-        if (wave == 0 && mine) {
-            offsets[slot] = x - c;
-            if (slot == nslots - 1) offsets[nslots] = x;
-        }
-        const int at = wave * spw + lane;
-        cnt_l = __shfl(c, at & 63, 64);
-        off_l = __shfl(x - c, at & 63, 64);
-        if (lane >= ns) cnt_l = 0u;
-        if (s0 >= nslots) return;
-    } else {
-        if (s0 >= nslots) return;
-        cnt_l = lane < ns ? counts[s0 + lane] : 0u;
-        off_l = lane < ns ? offsets[s0 + lane] : 0u;
+    __shared__ unsigned wsum[kThreads / 64];
+    const int per = (kThreads / 64) * spw, first = blockIdx.x * per;  // slots of the work-group, <= 64
+    const int tile = tile_sums ? first / kScanTile : 0;
+    unsigned p = 0;
+    for (int i = threadIdx.x; i < tile; i += kThreads) p += tile_sums[i];
+    for (int i = tile * kScanTile + threadIdx.x * 4; i < first; i += kThreads * 4) {  // first is a multiple of 4
+        const uint4 v = *reinterpret_cast<const uint4*>(counts + i);
+        p += (v.x + v.y) + (v.z + v.w);
     }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) p += __shfl_xor(p, d, 64);
+    if (lane == 0) wsum[wave] = p;
+    const int slot = first + lane;
+    const bool mine = lane < per && slot < nslots;
+    const unsigned c = mine ? counts[slot] : 0u;
+    unsigned x = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const unsigned t = __shfl_up(x, d, 64);
+        if (lane >= d) x += t;
+    }
+    __syncthreads();
+    x += (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+    if (wave == 0 && mine) {
+        offsets[slot] = x - c;
+        if (slot == nslots - 1) offsets[nslots] = x;
+    }
+    const int at = wave * spw + lane;
+    unsigned cnt_l = __shfl(c, at & 63, 64);
+    const unsigned off_l = __shfl(x - c, at & 63, 64);
+    if (lane >= ns) cnt_l = 0u;
+    if (s0 >= nslots) return;
     const unsigned long long any = ballot64(cnt_l != 0u);
     if (any == 0ull) return;
     // each slot's octave (the slots are ordered by octave)
@@ -2208,49 +2208,49 @@ void launch_extrema_tile(int S, int strip_rows, const OctaveDesc* d_oct, int noc
     }
 }
 
-// n_dev may be null (then n_max is the count). out needs n_max+1 entries;
-// tmp needs ceil(n_max/4096)+1 entries. Returns whether fin (may be null) was done.
-static bool scan(const unsigned* d_in, int n_max, const unsigned* n_dev, unsigned* d_out,
-                 unsigned* d_tmp, const FinalizeArgs* fin, int* d_owner, hipStream_t s) {
-    if (n_max <= kScanSingleMax) {
-        hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(kScanSingleThreads), 0, s, d_in, n_max, n_dev,
-                           d_out, fin ? *fin : FinalizeArgs{}, d_owner);
-        return true;
-    }
-    const int tiles = n_max > 0 ? (n_max + kScanTile - 1) / kScanTile : 1;
-    hipLaunchKernelGGL(k_scan_reduce, dim3(tiles), dim3(kThreads), 0, s, d_in, n_max, n_dev, d_tmp);
-    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(kThreads), 0, s, d_tmp, tiles);
-    hipLaunchKernelGGL(k_scan_down, dim3(tiles), dim3(kThreads), 0, s, d_in, n_max, n_dev, d_tmp,
-                       d_out, d_owner);
-    return false;
-}
-
 void launch_compact(const OctaveDesc* d_oct, int noct, int nslots, const unsigned long long* d_bits,
                     const unsigned* d_counts, unsigned* d_offsets, unsigned* d_tmp, Cand* d_cand, int cap,
                     hipStream_t s) {
-    if (nslots > 0 && nslots <= kCompactScanMax) {
-        // slots per wave: enough that the work-groups' reads of the counts before
-        // theirs stay a few MB in all (12756 slots of 3840 x 2160: 10 MB)
-        const int spw = nslots <= 2048 ? 1 : nslots <= 4096 ? 2 : nslots <= 8192 ? 4 : 8;
-        const int per = (kThreads / 64) * spw;
-        hipLaunchKernelGGL(k_compact<true>, dim3((nslots + per - 1) / per), dim3(kThreads), 0, s, d_oct,
-                           noct, nslots, d_bits, d_counts, d_offsets, d_cand, cap, spw);
+    if (nslots <= 0) {  // no octave: no candidates
+        hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(kScanSingleThreads), 0, s, d_counts, 0, nullptr,
+                           d_offsets, FinalizeArgs{}, nullptr);
         return;
     }
-    (void)scan(d_counts, nslots, nullptr, d_offsets, d_tmp, nullptr, nullptr, s);
-    if (nslots <= 0) return;
-    const int spw = nslots >= 65536 ? kCompactSlots : 1;  // slots per wave
-    const int per = (kThreads / 64) * spw;                 // slots per work-group
-    hipLaunchKernelGGL(k_compact<false>, dim3((nslots + per - 1) / per), dim3(kThreads), 0, s, d_oct, noct,
-                       nslots, d_bits, d_counts, d_offsets, d_cand, cap, spw);
+    // slots per wave: enough that the work-groups' reads of the counts before theirs
+    // stay a few MB in all (12756 slots of 3840 x 2160: 10 MB). With the sums of tiles
+    // only the counts of the group's own tile are read: 16 frames of 640 x 480 (45
+    // thousand slots) take 34 / 27 / 25 / 25 us with 1 / 2 / 4 / 8 slots a wave, 8 of
+    // 1280 x 720 30 / 25 / 22 / 25, 64 of 1920 x 1080 282 / 202 / 157 / 136.
+    const bool tiled = nslots > kCompactScanMax;
+    const int spw = nslots <= 2048                   ? 1
+                    : nslots <= 4096                 ? 2
+                    : nslots <= 8192                 ? 4
+                    : tiled && nslots < 65536        ? 4
+                                                     : kCompactSlots;
+    const int per = (kThreads / 64) * spw;  // slots per work-group
+    if (tiled)
+        hipLaunchKernelGGL(k_scan_reduce, dim3((nslots + kScanTile - 1) / kScanTile), dim3(kThreads), 0, s,
+                           d_counts, nslots, nullptr, d_tmp);
+    hipLaunchKernelGGL(k_compact, dim3((nslots + per - 1) / per), dim3(kThreads), 0, s, d_oct, noct, nslots,
+                       d_bits, d_counts, tiled ? d_tmp : nullptr, d_offsets, d_cand, cap, spw);
 }
 
+// The scan of the cap candidates' peak counts, of which d_total are there: d_koff has
+// cap + 1 entries, d_tmp ceil(cap / 4096) + 1.
 void launch_keypoint_offsets(const unsigned* d_npeaks, int cap, const unsigned* d_total, unsigned* d_koff,
                              unsigned* d_tmp, const unsigned* d_slot_offsets, const int* d_img_slot_begin,
                              int nimg, unsigned* d_summary, unsigned* d_out_offsets, int* d_owner, hipStream_t s) {
     const FinalizeArgs F{d_slot_offsets, d_img_slot_begin, nimg, d_koff, d_total, cap, d_summary, d_out_offsets};
-    if (!scan(d_npeaks, cap, d_total, d_koff, d_tmp, &F, cap <= kDescOneLaunchCap ? d_owner : nullptr, s))
-        hipLaunchKernelGGL(k_finalize, dim3((nimg + 1 + 255) / 256), dim3(256), 0, s, F);
+    if (cap > kDescOneLaunchCap) d_owner = nullptr;
+    if (cap <= kScanSingleMax) {
+        hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(kScanSingleThreads), 0, s, d_npeaks, cap, d_total,
+                           d_koff, F, d_owner);
+        return;
+    }
+    const int tiles = (cap + kScanTile - 1) / kScanTile;
+    hipLaunchKernelGGL(k_scan_reduce, dim3(tiles), dim3(kThreads), 0, s, d_npeaks, cap, d_total, d_tmp);
+    hipLaunchKernelGGL(k_scan_down, dim3(tiles), dim3(kThreads), 0, s, d_npeaks, cap, d_total, d_tmp, d_koff,
+                       F, d_owner);
 }
 
 static int grid_for(int cap, int per_block, int max_blocks) {
