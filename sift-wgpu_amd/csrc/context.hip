@@ -1332,13 +1332,17 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         launch_compact(d_oct, noct, nslots, (const unsigned long long*)AP(bits_off), d_counts, d_offs,
                        (unsigned*)AP(scantmp1_off), d_cand, cap, st);
         prof_end(K_COMPACT, 0.0, ev);
-        prof_begin(K_REFINE, 0.0, &ev);
-        launch_refine(d_oct, d_par, d_cand, d_total, cap, d_ref, d_valid,
-                      B.want_stages ? (float*)AP(candresp_off) : nullptr, st);
-        prof_end(K_REFINE, 0.0, ev);
+        // (the stages' candidate responses come from k_refine)
+        const bool refine_here = !B.want_stages && orient_refines(cap);
+        if (!refine_here) {
+            prof_begin(K_REFINE, 0.0, &ev);
+            launch_refine(d_oct, d_par, d_cand, d_total, cap, d_ref, d_valid,
+                          B.want_stages ? (float*)AP(candresp_off) : nullptr, st);
+            prof_end(K_REFINE, 0.0, ev);
+        }
         prof_begin(K_ORIENT, 0.0, &ev);
         launch_orient(d_oct, d_par, d_cand, d_total, cap, d_ref, d_valid, d_npk, d_ang,
-                      d_counts + nslots + 2, st);  // kNumXcd queue counters
+                      d_counts + nslots + 2, refine_here, st);  // kNumXcd queue counters
         prof_end(K_ORIENT, 0.0, ev);
         prof_begin(K_SCAN, 0.0, &ev);
         launch_keypoint_offsets(d_npk, cap, d_total, d_koff, (unsigned*)AP(scantmp2_off), d_offs,

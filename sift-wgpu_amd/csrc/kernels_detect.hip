@@ -829,6 +829,102 @@ struct __attribute__((packed)) UnalignedWord {
 // four waves, 12.0 us; 1920x1080 19.1 and 13.4; 64 frames 157 and 151).
 constexpr int kRefineThreads = 64;
 
+// The refinement of one candidate (refine_and_filter_extrema, src/sift.rs:299-474):
+// whether it is kept, and then its keypoint. kUniform: the whole wave has the same one.
+template <bool kUniform>
+__device__ __forceinline__ bool refine_candidate(const Cand& cd, const OctaveDesc& O,
+                                                 const ImageParams& P, Keypoint& r) {
+    const int nd = P.num_intervals + 2;  // DoG layers per octave
+    const float scale0 = pow2f(O.octave);
+    // kp.x / 2^o of the candidate ((x + 0.5) * 2^o), `as i32` (src/sift.rs:309-313)
+    const float xi = (((float)cd.x + 0.5f) * scale0) / scale0;
+    const float yi = (((float)cd.y + 0.5f) * scale0) / scale0;
+    int cx = f2i_sat(xi), cy = f2i_sat(yi), cl = cd.layer;
+    for (int step = 0; step < 5; step++) {
+        if (kUniform) {
+            cx = __builtin_amdgcn_readfirstlane(cx);
+            cy = __builtin_amdgcn_readfirstlane(cy);
+            cl = __builtin_amdgcn_readfirstlane(cl);
+        }
+        if (cl < 1 || cl >= nd - 1) return false;
+        if (cx < 1 || cx >= O.w - 1 || cy < 1 || cy >= O.h - 1) return false;
+        // the 3x3 texels around (cx, cy) of the four Gaussian levels cl - 1 .. cl + 2,
+        // a row by one word (columns cx - 1 .. cx + 2: cx + 2 <= w, and a byte past
+        // the last level's last row is still the arena's)
+        unsigned t[4][3];
+        const uint8_t* lv = O.levels + (long long)(cl - 1) * O.level_stride +
+                            ((size_t)(cy - 1) * O.pitch + (cx - 1));
+#pragma unroll
+        for (int l = 0; l < 4; l++, lv += O.level_stride)
+#pragma unroll
+            for (int r = 0; r < 3; r++)
+                t[l][r] = reinterpret_cast<const UnalignedWord*>(lv + r * O.pitch)->v;
+        // DoG layer cl - 1 + l at row cy - 1 + r, column cx - 1 + x
+        auto dog = [&](int l, int r, int x) {
+            return q255f((float)((t[l + 1][r] >> (8 * x)) & 0xffu)) -
+                   q255f((float)((t[l][r] >> (8 * x)) & 0xffu));
+        };
+        const float pxp = dog(1, 1, 2), pxm = dog(1, 1, 0);
+        const float pyp = dog(1, 2, 1), pym = dog(1, 0, 1);
+        const float nxt = dog(2, 1, 1), prv = dog(0, 1, 1);
+        const float dx = (pxp - pxm) / 2.0f;
+        const float dy = (pyp - pym) / 2.0f;
+        const float ds = (nxt - prv) / 2.0f;
+        const float cv = dog(1, 1, 1);
+        const float dxx = pxp + pxm - 2.0f * cv;
+        const float dyy = pyp + pym - 2.0f * cv;
+        const float dss = nxt + prv - 2.0f * cv;
+        const float dxy = (dog(1, 2, 2) - dog(1, 2, 0) - dog(1, 0, 2) + dog(1, 0, 0)) / 4.0f;
+        const float dxs = (dog(2, 1, 2) - dog(2, 1, 0) - (dog(0, 1, 2) - dog(0, 1, 0))) / 4.0f;
+        const float dys = (dog(2, 2, 1) - dog(2, 0, 1) - (dog(0, 2, 1) - dog(0, 0, 1))) / 4.0f;
+        // solve_linear_system (src/sift.rs:478-503), b = -g
+        const float a00 = dxx, a01 = dxy, a02 = dxs, a10 = dxy, a11 = dyy, a12 = dys,
+                    a20 = dxs, a21 = dys, a22 = dss;
+        const float b0 = -dx, b1 = -dy, b2 = -ds;
+        const float det_a = a00 * (a11 * a22 - a12 * a21) - a01 * (a10 * a22 - a12 * a20) +
+                            a02 * (a10 * a21 - a11 * a20);
+        if (fabsf(det_a) < 1e-10f) return false;
+        const float det_x = b0 * (a11 * a22 - a12 * a21) - a01 * (b1 * a22 - a12 * b2) +
+                            a02 * (b1 * a21 - a11 * b2);
+        const float det_y = a00 * (b1 * a22 - a12 * b2) - b0 * (a10 * a22 - a12 * a20) +
+                            a02 * (a10 * b2 - b1 * a20);
+        const float det_z = a00 * (a11 * b2 - b1 * a21) - a01 * (a10 * b2 - b1 * a20) +
+                            b0 * (a10 * a21 - a11 * a20);
+        const float ox = det_x / det_a, oy = det_y / det_a, os = det_z / det_a;
+        if (fabsf(ox) < 0.5f && fabsf(oy) < 0.5f && fabsf(os) < 0.5f) {
+            const float val = cv + 0.5f * (dx * ox + dy * oy + ds * os);
+            if (fabsf(val) < P.contrast_threshold) return false;
+            const float tr = dxx + dyy;
+            const float trace_sq = tr * tr;
+            const float det = dxx * dyy - dxy * dxy;
+            if (det <= 0.0f) return false;
+            const float ratio = trace_sq / det;
+            const float e1 = P.edge_threshold + 1.0f;
+            const float thr = e1 * e1 / P.edge_threshold;
+            if (ratio >= thr) return false;
+            const float scale = pow2f(O.octave);
+            const float fl = (float)cl + os;
+            const float e = (float)O.octave + fl / (float)P.num_intervals;
+            // 2.0_f32.powf(e): correctly rounded via double exp2
+            const float psig = P.sigma * (float)exp2((double)e);
+            r.x = ((float)cx + ox) * scale;
+            r.y = ((float)cy + oy) * scale;
+            r.size = psig;
+            r.angle = 0.0f;
+            r.response = val;
+            r.octave = O.octave;
+            r.layer = f2i_sat(roundf(fl));
+            return true;
+        } else {
+            cx = f2i_sat(roundf((float)cx + ox));
+            cy = f2i_sat(roundf((float)cy + oy));
+            cl = f2i_sat(roundf((float)cl + os));
+            if (cl < 0 || cl >= nd) return false;
+        }
+    }
+    return false;
+}
+
 __global__ __launch_bounds__(kRefineThreads) void k_refine(const OctaveDesc* __restrict__ oct,
                                                      const ImageParams* __restrict__ params,
                                                      const Cand* __restrict__ cand,
@@ -840,98 +936,13 @@ __global__ __launch_bounds__(kRefineThreads) void k_refine(const OctaveDesc* __r
     for (int c = blockIdx.x * kRefineThreads + threadIdx.x; c < n; c += gridDim.x * kRefineThreads) {
         const Cand cd = cand[c];
         const OctaveDesc& O = oct[cd.job];
-        const ImageParams& P = params[O.img];
-        const int nd = P.num_intervals + 2;  // DoG layers per octave
-        const float scale0 = pow2f(O.octave);
-        // kp.x / 2^o of the candidate ((x + 0.5) * 2^o), `as i32` (src/sift.rs:309-313)
-        const float xi = (((float)cd.x + 0.5f) * scale0) / scale0;
-        const float yi = (((float)cd.y + 0.5f) * scale0) / scale0;
-        int cx = f2i_sat(xi), cy = f2i_sat(yi), cl = cd.layer;
         if (cand_resp) {
             const uint8_t* g0 = O.levels + (long long)cd.layer * O.level_stride +
                                 ((size_t)cd.y * O.pitch + cd.x);
             cand_resp[c] = q255f((float)g0[O.level_stride]) - q255f((float)g0[0]);
         }
-        int ok = 0;
         Keypoint r;
-        for (int step = 0; step < 5; step++) {
-            if (cl < 1 || cl >= nd - 1) break;
-            if (cx < 1 || cx >= O.w - 1 || cy < 1 || cy >= O.h - 1) break;
-            // the 3x3 texels around (cx, cy) of the four Gaussian levels cl - 1 .. cl + 2,
-            // a row by one word (columns cx - 1 .. cx + 2: cx + 2 <= w, and a byte past
-            // the last level's last row is still the arena's)
-            unsigned t[4][3];
-            const uint8_t* lv = O.levels + (long long)(cl - 1) * O.level_stride +
-                                ((size_t)(cy - 1) * O.pitch + (cx - 1));
-#pragma unroll
-            for (int l = 0; l < 4; l++, lv += O.level_stride)
-#pragma unroll
-                for (int r = 0; r < 3; r++)
-                    t[l][r] = reinterpret_cast<const UnalignedWord*>(lv + r * O.pitch)->v;
-            // DoG layer cl - 1 + l at row cy - 1 + r, column cx - 1 + x
-            auto dog = [&](int l, int r, int x) {
-                return q255f((float)((t[l + 1][r] >> (8 * x)) & 0xffu)) -
-                       q255f((float)((t[l][r] >> (8 * x)) & 0xffu));
-            };
-            const float pxp = dog(1, 1, 2), pxm = dog(1, 1, 0);
-            const float pyp = dog(1, 2, 1), pym = dog(1, 0, 1);
-            const float nxt = dog(2, 1, 1), prv = dog(0, 1, 1);
-            const float dx = (pxp - pxm) / 2.0f;
-            const float dy = (pyp - pym) / 2.0f;
-            const float ds = (nxt - prv) / 2.0f;
-            const float cv = dog(1, 1, 1);
-            const float dxx = pxp + pxm - 2.0f * cv;
-            const float dyy = pyp + pym - 2.0f * cv;
-            const float dss = nxt + prv - 2.0f * cv;
-            const float dxy = (dog(1, 2, 2) - dog(1, 2, 0) - dog(1, 0, 2) + dog(1, 0, 0)) / 4.0f;
-            const float dxs = (dog(2, 1, 2) - dog(2, 1, 0) - (dog(0, 1, 2) - dog(0, 1, 0))) / 4.0f;
-            const float dys = (dog(2, 2, 1) - dog(2, 0, 1) - (dog(0, 2, 1) - dog(0, 0, 1))) / 4.0f;
-            // solve_linear_system (src/sift.rs:478-503), b = -g
-            const float a00 = dxx, a01 = dxy, a02 = dxs, a10 = dxy, a11 = dyy, a12 = dys,
-                        a20 = dxs, a21 = dys, a22 = dss;
-            const float b0 = -dx, b1 = -dy, b2 = -ds;
-            const float det_a = a00 * (a11 * a22 - a12 * a21) - a01 * (a10 * a22 - a12 * a20) +
-                                a02 * (a10 * a21 - a11 * a20);
-            if (fabsf(det_a) < 1e-10f) break;
-            const float det_x = b0 * (a11 * a22 - a12 * a21) - a01 * (b1 * a22 - a12 * b2) +
-                                a02 * (b1 * a21 - a11 * b2);
-            const float det_y = a00 * (b1 * a22 - a12 * b2) - b0 * (a10 * a22 - a12 * a20) +
-                                a02 * (a10 * b2 - b1 * a20);
-            const float det_z = a00 * (a11 * b2 - b1 * a21) - a01 * (a10 * b2 - b1 * a20) +
-                                b0 * (a10 * a21 - a11 * a20);
-            const float ox = det_x / det_a, oy = det_y / det_a, os = det_z / det_a;
-            if (fabsf(ox) < 0.5f && fabsf(oy) < 0.5f && fabsf(os) < 0.5f) {
-                const float val = cv + 0.5f * (dx * ox + dy * oy + ds * os);
-                if (fabsf(val) < P.contrast_threshold) break;
-                const float tr = dxx + dyy;
-                const float trace_sq = tr * tr;
-                const float det = dxx * dyy - dxy * dxy;
-                if (det <= 0.0f) break;
-                const float ratio = trace_sq / det;
-                const float e1 = P.edge_threshold + 1.0f;
-                const float thr = e1 * e1 / P.edge_threshold;
-                if (ratio >= thr) break;
-                const float scale = pow2f(O.octave);
-                const float fl = (float)cl + os;
-                const float e = (float)O.octave + fl / (float)P.num_intervals;
-                // 2.0_f32.powf(e): correctly rounded via double exp2
-                const float psig = P.sigma * (float)exp2((double)e);
-                r.x = ((float)cx + ox) * scale;
-                r.y = ((float)cy + oy) * scale;
-                r.size = psig;
-                r.angle = 0.0f;
-                r.response = val;
-                r.octave = O.octave;
-                r.layer = f2i_sat(roundf(fl));
-                ok = 1;
-                break;
-            } else {
-                cx = f2i_sat(roundf((float)cx + ox));
-                cy = f2i_sat(roundf((float)cy + oy));
-                cl = f2i_sat(roundf((float)cl + os));
-                if (cl < 0 || cl >= nd) break;
-            }
-        }
+        const bool ok = refine_candidate<false>(cd, O, params[O.img], r);
         valid[c] = ok;
         if (ok) out[c] = r;
     }
@@ -1012,8 +1023,8 @@ static_assert(2 * kOriMaxR + 1 <= 64, "one lane per row and column of the window
 constexpr double kOriBias = 4503599627370496.0;  // 2^52
 
 // ---------------------------------------------------------------------------
-// k_orient: one wave (workgroup of 64) per refined keypoint
-// (src/sift.rs:605-726). Each sample of the (2R+1)^2 window adds
+// k_orient: one wave (workgroup of 64) per refined keypoint, or (kRefine) per
+// candidate, which it refines first (src/sift.rs:605-726). Each sample of the (2R+1)^2 window adds
 // mag * exp(-(dx^2+dy^2)/denom) to bin floor(theta * 36 / 2pi) of a u64
 // fixed-point (2^40) histogram, one of 4 copies by lane (integer adds:
 // order-independent, deterministic, and as fine as the f32 contributions
@@ -1043,12 +1054,12 @@ constexpr double kOriBias = 4503599627370496.0;  // 2^52
 // spread over more banks. 2 or 8 histogram copies, other row strides and an unaligned
 // word for the two horizontal texels were slower too (1150 us for the last).
 // ---------------------------------------------------------------------------
+template <bool kRefine>
 __global__ __launch_bounds__(64) void k_orient(const OctaveDesc* __restrict__ oct,
                                                const ImageParams* __restrict__ params,
                                                const Cand* __restrict__ cand,
                                                const unsigned* __restrict__ total, int cap,
-                                               const Keypoint* __restrict__ ref,
-                                               const int* __restrict__ valid,
+                                               Keypoint* __restrict__ ref, int* __restrict__ valid,
                                                unsigned* __restrict__ npeaks,
                                                float* __restrict__ angles,
                                                unsigned* __restrict__ queue) {
@@ -1064,13 +1075,30 @@ __global__ __launch_bounds__(64) void k_orient(const OctaveDesc* __restrict__ oc
     WorkQueue<kOrientChunk> Q{queue, 0, 0, 0};
     for (int c = Q.first(qslot); c < n; c = Q.next(qslot, c)) {
         Q.prefetch(qslot);
-        if (!valid[c]) {
+        const Cand cd = cand[c];
+        const OctaveDesc& O = oct[cd.job];
+        const ImageParams& P = params[O.img];
+        Keypoint kp;
+        bool ok;
+        if (kRefine) {
+            ok = __builtin_amdgcn_readfirstlane((int)refine_candidate<true>(cd, O, P, kp)) != 0;
+            if (lane == 0) {
+                valid[c] = ok;
+                if (ok) ref[c] = kp;
+            }
+            kp.x = uniform_f(kp.x);
+            kp.y = uniform_f(kp.y);
+            kp.size = uniform_f(kp.size);
+            kp.octave = O.octave;
+            kp.layer = __builtin_amdgcn_readfirstlane(kp.layer);
+        } else {
+            ok = valid[c] != 0;
+            kp = ref[c];
+        }
+        if (!ok) {
             if (lane == 0) npeaks[c] = 0;
             continue;
         }
-        const Keypoint kp = ref[c];
-        const OctaveDesc& O = oct[cand[c].job];
-        const ImageParams& P = params[O.img];
         const int S = P.num_intervals;
         const int gl = min(max(kp.layer, 0), S + 2);
         const uint8_t* g = O.levels + (long long)gl * O.level_stride;
@@ -2288,6 +2316,12 @@ static bool queue_enabled() {
     return e && e[0] == '1';
 }
 
+// With few candidates each orientation wave refines its own: the whole wave does one
+// candidate's arithmetic, but a launch and the latency of its few waves go (k_refine and
+// k_orient 640x480 24 -> 14 us, 1280x720 29 -> 21, 1920x1080 32 -> 29; 8 x 640x480, whose
+// capacity is just above the limit, 45 -> 48).
+bool orient_refines(int cap) { return cap <= 65536; }
+
 void launch_refine(const OctaveDesc* d_oct, const ImageParams* d_params, const Cand* d_cand,
                    const unsigned* d_total, int cap, Keypoint* d_ref, int* d_valid,
                    float* d_cand_resp, hipStream_t s) {
@@ -2296,8 +2330,8 @@ void launch_refine(const OctaveDesc* d_oct, const ImageParams* d_params, const C
 }
 
 void launch_orient(const OctaveDesc* d_oct, const ImageParams* d_params, const Cand* d_cand,
-                   const unsigned* d_total, int cap, const Keypoint* d_ref, const int* d_valid,
-                   unsigned* d_npeaks, float* d_angles, unsigned* d_queue, hipStream_t s) {
+                   const unsigned* d_total, int cap, Keypoint* d_ref, int* d_valid, unsigned* d_npeaks,
+                   float* d_angles, unsigned* d_queue, bool refine, hipStream_t s) {
     // work queue: as many work-groups as fit, each taking keypoints until none
     // are left; or grid-stride over the candidates with many more work-groups
     // than fit at once (each takes only a few keypoints, so the launch ends evenly).
@@ -2306,11 +2340,15 @@ void launch_orient(const OctaveDesc* d_oct, const ImageParams* d_params, const C
     // 1920x1080 22.5 and 19.5), while 64 frames take 648 us with 32768 and 630 with 65536.
     const int most = cap <= kDescOneLaunchCap ? 32768 : 65536;
     const bool q = queue_enabled();
-    const int grid = q ? std::min(resident_groups((const void*)k_orient, 64), grid_for(cap, 1, most))
+    const int grid = q ? std::min(resident_groups((const void*)k_orient<false>, 64), grid_for(cap, 1, most))
                        : grid_for(cap, 1, most);
     // (d_queue: kNumXcd counters)
-    hipLaunchKernelGGL(k_orient, dim3(grid), dim3(64), 0, s, d_oct, d_params, d_cand, d_total, cap,
-                       d_ref, d_valid, d_npeaks, d_angles, q ? d_queue : nullptr);
+    if (refine)
+        hipLaunchKernelGGL(k_orient<true>, dim3(grid), dim3(64), 0, s, d_oct, d_params, d_cand, d_total, cap,
+                           d_ref, d_valid, d_npeaks, d_angles, q ? d_queue : nullptr);
+    else
+        hipLaunchKernelGGL(k_orient<false>, dim3(grid), dim3(64), 0, s, d_oct, d_params, d_cand, d_total, cap,
+                           d_ref, d_valid, d_npeaks, d_angles, q ? d_queue : nullptr);
 }
 
 void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, const Cand* d_cand,

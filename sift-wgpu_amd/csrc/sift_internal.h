@@ -182,6 +182,9 @@ void launch_compact(const OctaveDesc* d_oct, int noct, int nslots, const unsigne
 void launch_keypoint_offsets(const unsigned* d_npeaks, int cap, const unsigned* d_total, unsigned* d_koff,
                              unsigned* d_tmp, const unsigned* d_slot_offsets, const int* d_img_slot_begin,
                              int nimg, unsigned* d_summary, unsigned* d_out_offsets, int* d_owner, hipStream_t s);
+// Whether launch_orient is to refine the candidates itself (refine = true) in place of
+// launch_refine.
+bool orient_refines(int cap);
 void launch_refine(const OctaveDesc* d_oct, const ImageParams* d_params, const Cand* d_cand,
                    const unsigned* d_total, int cap, Keypoint* d_ref, int* d_valid,
                    float* d_cand_resp, hipStream_t s);
@@ -189,8 +192,8 @@ void launch_refine(const OctaveDesc* d_oct, const ImageParams* d_params, const C
 // for each of the descriptor's two instantiations), among the kCountExtra after
 // the row slots.
 void launch_orient(const OctaveDesc* d_oct, const ImageParams* d_params, const Cand* d_cand,
-                   const unsigned* d_total, int cap, const Keypoint* d_ref, const int* d_valid,
-                   unsigned* d_npeaks, float* d_angles, unsigned* d_queue, hipStream_t s);
+                   const unsigned* d_total, int cap, Keypoint* d_ref, int* d_valid, unsigned* d_npeaks,
+                   float* d_angles, unsigned* d_queue, bool refine, hipStream_t s);
 void launch_descriptor(const OctaveDesc* d_oct, const ImageParams* d_params, const Cand* d_cand,
                        const unsigned* d_total, int cap, const Keypoint* d_ref,
                        const unsigned* d_npeaks, const float* d_angles, const unsigned* d_koff,
