@@ -23,7 +23,9 @@ sys.path.insert(0, os.path.join(REPO, "sift-wgpu_amd"))
 
 METRIC = "1080p frames/s & MPix/s (batched); p50/p99 latency on mixed-size stream"
 HBM_PEAK_GBS = 8000.0
-VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12  # non-packed f32 lane operations per second (39.3 T)
+# non-packed f32 lane operations per second (78.6 T): 256 CUs x 4 SIMDs x 32 lanes a clock;
+# independent multiplies and adds measure 2.2 cycles a wave64 instruction
+VALU_PEAK_TOPS = 256 * 128 * 2.4e9 / 1e12
 
 
 def parse():
@@ -512,7 +514,7 @@ def main():
         ops = stats[dom][3]
         if ops > 0:
             # the exact arithmetic (a multiply and an add per tap, no FMA, no packed
-            # FP32) against the non-packed f32 VALU rate: 256 CUs x 64 lanes x 2.4 GHz
+            # FP32) against the non-packed f32 VALU rate: 256 CUs x 128 lanes x 2.4 GHz
             vach = ops / n / avg_s / 1e12
             out["roofline"]["valu_achieved"] = round(vach, 3)
             out["roofline"]["valu_peak"] = VALU_PEAK_TOPS
