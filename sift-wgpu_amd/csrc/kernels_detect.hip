@@ -1752,20 +1752,20 @@ __attribute__((amdgpu_waves_per_eu(MR <= kDescSmallR ? 8 : 6))) void k_descripto
                 // the 16th of windows with R >= 26, one row per thread.
                 constexpr int kPasses = (kPatchRows + 15) / 16;
                 const int row = tid >> 4, wd = tid & 15;
-                const uint8_t* const rowp = G.g + (size_t)py0 * G.pitch + px0a;
+                gbyte_t* const rowp = (gbyte_t*)G.g + ((size_t)py0 * G.pitch + px0a);
                 const unsigned off = (unsigned)row * (unsigned)G.pitch + 4u * (unsigned)wd;
                 unsigned wv[kPasses], we[2] = {0u, 0u};
 #pragma unroll
                 for (int k = 0; k < kPasses; k++) {
                     wv[k] = 0u;  // defined on every path: nothing carried across keypoints
                     if (row + 16 * k < pside && wd < nw)
-                        wv[k] = *reinterpret_cast<const unsigned*>(rowp + (off + 16u * k * (unsigned)G.pitch));
+                        wv[k] = *(gu32_t*)(rowp + (off + 16u * k * (unsigned)G.pitch));
                 }
                 const bool more = nw > 16 && tid < pside;
                 const unsigned offe = (unsigned)tid * (unsigned)G.pitch + 64u;
                 if (more) {
-                    we[0] = *reinterpret_cast<const unsigned*>(rowp + offe);
-                    if (nw > 17) we[1] = *reinterpret_cast<const unsigned*>(rowp + offe + 4u);
+                    we[0] = *(gu32_t*)(rowp + offe);
+                    if (nw > 17) we[1] = *(gu32_t*)(rowp + (offe + 4u));
                 }
                 // texel range of the staged words (a few texels left and right of
                 // the patch included: a wider range is still a bound)
