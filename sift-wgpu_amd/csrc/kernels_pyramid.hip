@@ -315,7 +315,9 @@ __device__ __forceinline__ void cvt4(unsigned v, float* o) {
     o[3] = (float)(v >> 24);
 }
 
-// v: four pixels of row y from column x, packed.
+// v: four pixels of row y from column x, packed; kDog: with the DoG row where the job
+// has one.
+template <bool kDog>
 __device__ __forceinline__ void store_row4(const BlurJob& J, int y, int x, unsigned v) {
     uint8_t* dst = J.dst + (size_t)y * J.dst_pitch + x;
     const int w = J.w;
@@ -326,7 +328,7 @@ __device__ __forceinline__ void store_row4(const BlurJob& J, int y, int x, unsig
         for (int c = 0; c < 4; c++)
             if (x + c < w) dst[c] = (uint8_t)(v >> (8 * c));
     }
-    if (J.dog) {
+    if (kDog && J.dog) {
         const uint8_t* prev = J.prev + (size_t)y * J.dst_pitch + x;
         float* dg = J.dog + (size_t)y * J.dog_pitch + x;
 #pragma unroll
@@ -473,7 +475,7 @@ __global__ __launch_bounds__(kThreads) void k_blur_v(const BlurJob* __restrict__
     for (int q = 0; q < RV; q++) {
         const int y = yb + q;
         if (y >= h) break;
-        store_row4(J, y, x, res[q]);
+        store_row4<true>(J, y, x, res[q]);
     }
 }
 
@@ -607,7 +609,7 @@ __device__ __forceinline__ void blur_hv_tile(const BlurJob& J, int x0, int y0, u
         trunc_rows(acc, res);
 #pragma unroll
         for (int q = 0; q < RV; q++)
-            if (yb + q < h && x < w) store_row4(J, yb + q, x, res[q]);
+            if (yb + q < h && x < w) store_row4<false>(J, yb + q, x, res[q]);
     }
 }
 
