@@ -852,13 +852,13 @@ __device__ __forceinline__ bool refine_candidate(const Cand& cd, const OctaveDes
         // a row by one word (columns cx - 1 .. cx + 2: cx + 2 <= w, and a byte past
         // the last level's last row is still the arena's)
         unsigned t[4][3];
-        const uint8_t* lv = O.levels + (long long)(cl - 1) * O.level_stride +
-                            ((size_t)(cy - 1) * O.pitch + (cx - 1));
+        gbyte_t* lv = (gbyte_t*)O.levels + ((long long)(cl - 1) * O.level_stride +
+                                            (long long)((size_t)(cy - 1) * O.pitch + (cx - 1)));
 #pragma unroll
         for (int l = 0; l < 4; l++, lv += O.level_stride)
 #pragma unroll
             for (int r = 0; r < 3; r++)
-                t[l][r] = reinterpret_cast<const UnalignedWord*>(lv + r * O.pitch)->v;
+                t[l][r] = ((const __attribute__((address_space(1))) UnalignedWord*)(lv + r * O.pitch))->v;
         // DoG layer cl - 1 + l at row cy - 1 + r, column cx - 1 + x
         auto dog = [&](int l, int r, int x) {
             return q255f((float)((t[l + 1][r] >> (8 * x)) & 0xffu)) -
