@@ -554,11 +554,11 @@ __global__ __launch_bounds__(kThreads) void k_scan_reduce(const unsigned* __rest
 }
 
 // The candidate of every keypoint, for the descriptor's work-groups (owner may be null;
-// keypoints past its size are searched for): candidate c has the keypoints [k, e).
+// keypoints past its size are searched for): candidate c has the keypoints [k, e), at
+// most kMaxPeaks.
 __device__ __forceinline__ void mark_owner(int* __restrict__ owner, int size, int c, unsigned k,
                                            unsigned e) {
-    for (; k < e; k++)
-        if (k < (unsigned)size) owner[k] = c;
+    for (e = min(e, min(k + (unsigned)kMaxPeaks, (unsigned)size)); k < e; k++) owner[k] = c;
 }
 
 // Per-image keypoint ranges: summary[2+i] = koff[first candidate of image i]
