@@ -539,9 +539,10 @@ void blur_hv_tiles(BlurJob& J, bool large) {
 // (240 x 135, 199 taps, 0.43 M: 18.8 against 19.6; 120 x 67, 395 taps, 0.42 M: 22.6
 // against 21.4).
 constexpr double kDeepStepWork = 60e6, kDeepTileWork = 0.4e6;
-bool blur_deep_valid(int h, int ntaps) {
+bool blur_deep_valid(int src_pitch, int h, int ntaps) {
     return ntaps > kHvMaxTaps && deep_tile_work(h, ntaps) <= kDeepTileWork &&
-           deep_lds_bytes(h, ntaps) <= (size_t)kDeepMaxLds;
+           deep_lds_bytes(h, ntaps) <= (size_t)kDeepMaxLds &&
+           (long long)deep_rows(h, ntaps) * src_pitch <= INT_MAX;
 }
 
 // Tile counts of a job in a form.
@@ -961,7 +962,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
             hvj.push_back(J);  // its tiles: flush_blur
             return;
         }
-        if (!dog && forced.first < 0 && forced.second < 0 && blur_deep_valid(h, R.ntaps)) {
+        if (!dog && forced.first < 0 && forced.second < 0 && blur_deep_valid(src_pitch, h, R.ntaps)) {
             J.src = src;
             J.src_pitch = src_pitch;
             J.dst = dst;

@@ -914,6 +914,8 @@ __global__ __launch_bounds__(kDeepThreads) void k_blur_deep(const BlurJob* __res
     // below, in contrast, was slower (99 us): four waves a SIMD hide those already.
     const float inv = __builtin_amdgcn_rcpf((float)segw);
     const int total = nr * segw;
+    // (32-bit offsets from the first staged row: the host keeps the staged rows'
+    // span within them, whatever stride the caller's frame has)
     gbyte_t* const src =
         (gbyte_t*)J.src + (size_t)rlo * J.src_pitch;
     for (int i0 = tid; i0 < total; i0 += 8 * kDeepThreads) {
@@ -1392,15 +1394,20 @@ int deep_tiles_y(int h, int ntaps) {
     return least;
 }
 
+int deep_rows(int h, int ntaps) {
+    const int ty = deep_tiles_y(h, ntaps), th = (h + ty - 1) / ty;
+    return std::min(h, th + 2 * (ntaps / 2));
+}
+
 size_t deep_lds_bytes(int h, int ntaps) {
     const int ty = deep_tiles_y(h, ntaps), th = (h + ty - 1) / ty;
-    const size_t n4 = (size_t)((ntaps + 3) & ~3), nr = (size_t)std::min(h, th + 2 * (ntaps / 2));
+    const size_t n4 = (size_t)((ntaps + 3) & ~3), nr = (size_t)deep_rows(h, ntaps);
     return 4 * (n4 + nr * (size_t)deep_stride((int)n4) + (th + n4) * kDeepW);
 }
 
 double deep_tile_work(int h, int ntaps) {
     const int ty = deep_tiles_y(h, ntaps), th = (h + ty - 1) / ty;
-    return (double)(std::min(h, th + 2 * (ntaps / 2)) + th) * kDeepW * ntaps;
+    return (double)(deep_rows(h, ntaps) + th) * kDeepW * ntaps;
 }
 
 void launch_blur_deep(const BlurJob* d_jobs, int njobs, int total_tiles, int lds, hipStream_t s) {

@@ -130,8 +130,10 @@ void launch_blur_hv_small(const BlurJob* d_jobs, int njobs, int total_tiles, hip
 // epilogue: tiles of kDeepW columns x 1/deep_tiles_y of the level's rows (cut to
 // need one horizontal pass where tiles of 32 rows or more do), lds = the largest
 // deep_lds_bytes of the launch's jobs (at most kDeepMaxLds); deep_tile_work: the
-// products of a tile.
+// products of a tile; deep_rows: the most source rows a tile stages, which must span
+// at most INT_MAX bytes (their texels are at 32-bit offsets).
 int deep_tiles_y(int h, int ntaps);
+int deep_rows(int h, int ntaps);
 size_t deep_lds_bytes(int h, int ntaps);
 double deep_tile_work(int h, int ntaps);
 void launch_blur_deep(const BlurJob* d_jobs, int njobs, int total_tiles, int lds, hipStream_t s);
