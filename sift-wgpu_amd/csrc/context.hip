@@ -510,7 +510,7 @@ bool resize_fits(const LanczosRef& LH, const LanczosRef& LV, int tw, int span) {
 }
 
 // Whether both passes of a blur go in one kernel (k_blur_hv / k_blur_hv_small).
-bool blur_hv_valid(const uint8_t* src, int src_pitch, int ntaps) {
+bool blur_hv_valid(const uint8_t* src, unsigned src_pitch, int ntaps) {
     return ntaps >= kHvMinTaps && ntaps <= kHvMaxTaps && (((uintptr_t)src | (uintptr_t)src_pitch) & 3) == 0;
 }
 // The fused blur's tiles for a job of a step whose fused jobs hold step_px pixels.
@@ -539,7 +539,7 @@ void blur_hv_tiles(BlurJob& J, bool large) {
 // (240 x 135, 199 taps, 0.43 M: 18.8 against 19.6; 120 x 67, 395 taps, 0.42 M: 22.6
 // against 21.4).
 constexpr double kDeepStepWork = 60e6, kDeepTileWork = 0.4e6;
-bool blur_deep_valid(int src_pitch, int h, int ntaps) {
+bool blur_deep_valid(unsigned src_pitch, int h, int ntaps) {
     return ntaps > kHvMaxTaps && deep_tile_work(h, ntaps) <= kDeepTileWork &&
            deep_lds_bytes(h, ntaps) <= (size_t)kDeepMaxLds &&
            (long long)deep_rows(h, ntaps) * src_pitch <= INT_MAX;
@@ -676,7 +676,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     if (B.ext) C.off = round_up(tables.host.size(), 256);  // the tables come first
     std::vector<size_t> in_off(n), rtmp_off(n);
     std::vector<std::vector<size_t>> lev_off(n), dog_off(n), htemp_off(n);
-    std::vector<int> in_pitch(n);
+    std::vector<unsigned> in_pitch(n);
     // colour inputs: raw pixels (host inputs are staged at color_off) and the
     // grey image k_luma writes at in_off
     std::vector<size_t> color_off(n, 0);
@@ -686,9 +686,9 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         const uint32_t fmt = B.format(i);
         int S = (int)B.params[i].num_intervals, L = S + 3;
         if (B.device_input && fmt == SIFT_PIXEL_GRAY8) {
-            in_pitch[i] = (int)(im.stride ? im.stride : im.width);
+            in_pitch[i] = im.stride ? im.stride : im.width;
         } else {
-            in_pitch[i] = (int)round_up(im.width, 64);
+            in_pitch[i] = (unsigned)round_up(im.width, 64);
             // a grey host input goes with the staged inputs below
             if (fmt != SIFT_PIXEL_GRAY8) in_off[i] = C.take((size_t)in_pitch[i] * im.height);
         }
@@ -885,7 +885,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     };
 
     // the two one-pass jobs of a blur through tmp; V: the whole blur but its source
-    auto push_two_pass = [&](const uint8_t* src, int src_pitch, uint8_t* tmp, int tmp_pitch, BlurJob V) {
+    auto push_two_pass = [&](const uint8_t* src, unsigned src_pitch, uint8_t* tmp, int tmp_pitch, BlurJob V) {
         const std::pair<int, int> form =
             blur_choice(V.w, V.h, V.ntaps, V.ntaps_pad, n >= kTuneManyJobs, forced);
         const int n4 = (V.ntaps + 3) & ~3, r = V.ntaps / 2;
@@ -932,7 +932,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         }
     };
 
-    auto make_blur_pair = [&](const uint8_t* src, int src_pitch, uint8_t* tmp, int tmp_pitch,
+    auto make_blur_pair = [&](const uint8_t* src, unsigned src_pitch, uint8_t* tmp, int tmp_pitch,
                               uint8_t* dst, int dst_pitch, int w, int h, const TapsRef& R,
                               float* dog, const uint8_t* prev, int dog_pitch) {
         if (w <= 0 || h <= 0) return;
@@ -1043,7 +1043,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
             J.src = B.device_input ? im.data : (const uint8_t*)AP(color_off[i]);
             J.src_pitch = color_pitch[i];
             J.dst = (uint8_t*)AP(in_off[i]);
-            J.dst_pitch = in_pitch[i];
+            J.dst_pitch = (int)in_pitch[i];
             J.w = (int)im.width;
             J.h = (int)im.height;
             J.format = (int)fmt;

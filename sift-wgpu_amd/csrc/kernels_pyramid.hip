@@ -505,7 +505,8 @@ __device__ __forceinline__ void blur_hv_tile(const BlurJob& J, int x0, int y0, u
     constexpr int R = NT / 2, kHalo = R <= 8 ? 8 : 16, NW = (PX + 2 * kHalo) / 4;
     constexpr int kLanes = TW / PX;               // lanes per row
     constexpr int kPassRows = kThreads / kLanes;  // rows of one pass of the work-group
-    const int w = J.w, h = J.h, pitch = J.src_pitch;
+    const int w = J.w, h = J.h;
+    const unsigned pitch = J.src_pitch;
     const ctap_t* taps = as_const_taps(J.taps);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

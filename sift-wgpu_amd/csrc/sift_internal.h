@@ -34,7 +34,8 @@ struct BlurJob {
     int ntaps;            // 2r+1
     int ntaps_pad;        // multiple of kTapBlock
     int w, h;
-    int src_pitch, dst_pitch, dog_pitch;
+    unsigned src_pitch;   // a caller's frame may have any 32-bit stride
+    int dst_pitch, dog_pitch;
     int tiles_x;          // tiles along x for this job
     int tile_begin;       // prefix over jobs in the launch
     int tiles;            // tiles of this job

@@ -1,6 +1,7 @@
 """Device frames whose rows lie far apart: a frame is described the same, bit for
 bit, whatever stride it is given with. Rows 64 MiB apart put a tile's rows more than
-4 GiB apart, past what 32-bit offsets from its first row reach."""
+4 GiB apart, past what 32-bit offsets from its first row reach; a stride of 2 GiB or
+more does not fit an int."""
 import numpy as np
 import pytest
 
@@ -24,16 +25,11 @@ def _upload(img, stride):
     return buf
 
 
-# base kernels of 7, 37, 49 and 81 taps: both passes in one kernel up to 33 taps and, on
-# small levels, beyond
-@pytest.mark.parametrize("sigma", [1.6, 9.0, 12.0, 20.0])
-@pytest.mark.parametrize("stride", [64 << 20, (64 << 20) + 1])
-def test_rows_far_apart(sigma, stride):
-    w, h = 96, 200
+def _compare(sigma, w, h, stride, least):
     img = _blocks(w, h)
     sift = sift_hip.Sift(sigma, 2, 3, 0.5, 0.0, 1000.0)
     want_k, want_d = sift.detect_and_compute(img)
-    assert len(want_k) > 10
+    assert len(want_k) >= least
     buf = _upload(img, stride)
     (n,), kp, de, _ = sift.detect_batch_device([(buf.addr, w, h, stride)])
     got_k, got_d = devmem.download(kp, n * want_k.itemsize), devmem.download(de, n * 512)
@@ -41,3 +37,17 @@ def test_rows_far_apart(sigma, stride):
     assert n == len(want_k)
     assert got_k.tobytes() == want_k.tobytes()
     assert got_d.tobytes() == want_d.tobytes()
+
+
+# base kernels of 7, 37, 49 and 81 taps: both passes in one kernel up to 33 taps and, on
+# small levels, beyond
+@pytest.mark.parametrize("sigma", [1.6, 9.0, 12.0, 20.0])
+@pytest.mark.parametrize("stride", [64 << 20, (64 << 20) + 1])
+def test_rows_far_apart(sigma, stride):
+    _compare(sigma, 96, 200, stride, 10)
+
+
+@pytest.mark.parametrize("sigma", [1.6, 9.0])
+@pytest.mark.parametrize("stride", [(2 << 30) + 4, (2 << 30) + 1])
+def test_strides_past_an_int(sigma, stride):
+    _compare(sigma, 120, 24, stride, 1)
