@@ -509,9 +509,11 @@ bool resize_fits(const LanczosRef& LH, const LanczosRef& LV, int tw, int span) {
     return true;
 }
 
-// Whether both passes of a blur go in one kernel (k_blur_hv / k_blur_hv_small).
-bool blur_hv_valid(const uint8_t* src, unsigned src_pitch, int ntaps) {
-    return ntaps >= kHvMinTaps && ntaps <= kHvMaxTaps && (((uintptr_t)src | (uintptr_t)src_pitch) & 3) == 0;
+// Whether both passes of a blur go in one kernel (k_blur_hv / k_blur_hv_small), which
+// reads whole words: a caller's rows of fewer than 4 pixels (w; not padded) hold none.
+bool blur_hv_valid(const uint8_t* src, unsigned src_pitch, int w, bool padded, int ntaps) {
+    return (padded || w >= 4) && ntaps >= kHvMinTaps && ntaps <= kHvMaxTaps &&
+           (((uintptr_t)src | (uintptr_t)src_pitch) & 3) == 0;
 }
 // The fused blur's tiles for a job of a step whose fused jobs hold step_px pixels.
 // The large tiles need 6 Mpixel to fill the GPU (16 levels of 640 x 480, 7 taps:
@@ -934,7 +936,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
 
     auto make_blur_pair = [&](const uint8_t* src, unsigned src_pitch, uint8_t* tmp, int tmp_pitch,
                               uint8_t* dst, int dst_pitch, int w, int h, const TapsRef& R,
-                              float* dog, const uint8_t* prev, int dog_pitch) {
+                              float* dog, const uint8_t* prev, int dog_pitch, bool padded = true) {
         if (w <= 0 || h <= 0) return;
         BlurJob J{};
         J.w = w;
@@ -954,7 +956,7 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         J.taps = (const float*)(T + R.off);
         J.ntaps = R.ntaps;
         J.ntaps_pad = R.npad;
-        if (!dog && forced.first < 0 && forced.second < 0 && blur_hv_valid(src, src_pitch, R.ntaps)) {
+        if (!dog && forced.first < 0 && forced.second < 0 && blur_hv_valid(src, src_pitch, w, padded, R.ntaps)) {
             J.src = src;
             J.src_pitch = src_pitch;
             J.dst = dst;
@@ -1057,12 +1059,11 @@ int Context::run(const Batch& B, RunOutputs* outs) {
     // initial blur into octave 0 level 0
     for (int i = 0; i < n; i++) {
         const OctShape& s = shapes[i][0];
-        const uint8_t* src = B.device_input && B.format(i) == SIFT_PIXEL_GRAY8
-                                 ? B.images[i].data
-                                 : (const uint8_t*)AP(in_off[i]);
+        const bool callers = B.device_input && B.format(i) == SIFT_PIXEL_GRAY8;
+        const uint8_t* src = callers ? B.images[i].data : (const uint8_t*)AP(in_off[i]);
         make_blur_pair(src, in_pitch[i], (uint8_t*)AP(htemp_off[i][0]), s.pitch,
                        (uint8_t*)AP(lev_off[i][0]), s.pitch, s.w, s.h, ptab[i]->initial, nullptr,
-                       nullptr, 0);
+                       nullptr, 0, !callers);
     }
     flush_blur();
     // The levels as a wavefront: level s >= 1 of octave o of image i is blurred in

@@ -820,10 +820,6 @@ __global__ __launch_bounds__(kThreads) void k_compact(const OctaveDesc* __restri
 // pyramid in all. A word for the 3 texels of a row (12 loads a step instead of 38 of
 // single bytes): 64 x 1920x1080 190 -> 156 us.
 // ---------------------------------------------------------------------------
-struct __attribute__((packed)) UnalignedWord {
-    unsigned v;
-};
-
 // Work-groups of one wave: the gathers of the few waves a single frame has are bound
 // by a CU's requests, so they are spread over all CUs (640x480: 17.5 us with groups of
 // four waves, 12.0 us; 1920x1080 19.1 and 13.4; 64 frames 157 and 151).

@@ -12,6 +12,7 @@
 // reference's arithmetic, so the levels are bit-identical to it.
 #include <algorithm>
 
+#include "edge_words.h"
 #include "sift_hip.h"
 #include "sift_internal.h"
 
@@ -489,8 +490,7 @@ __global__ __launch_bounds__(kThreads) void k_blur_v(const BlurJob* __restrict__
 // memory: a lane loads the aligned words of its PX + 2 kHalo window bytes (its
 // neighbours' loads hit L1) and needs no LDS or exchange. In tiles at the left or
 // right edge the word addresses are clamped and the bytes past the edge replaced
-// by one v_perm per word (a word past the image is never read: the last one read
-// holds the row's last pixel).
+// by one v_perm per word (edge_words.h: no byte past the row's last pixel is read).
 // Vertical: RV rows x 4 columns (256-column tiles) or x 1 column (64) per lane,
 // each staged row read and converted once, as in k_blur_v.
 // Bound: the exact multiply and add of every tap; the staged rows' 2r / TH extra
@@ -512,9 +512,7 @@ __device__ __forceinline__ void blur_hv_tile(const BlurJob& J, int x0, int y0, u
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int xl = (tid % kLanes) * PX;  // the lane's first column in the tile
     const bool inside = x0 >= kHalo && x0 + TW + kHalo <= w;
-    const int wl = (w - 1) & ~3, last = (w - 1) & 3;  // the row's last word and its last pixel's byte
-    const unsigned sel_end = last == 3 ? 0x03020100u : last == 2 ? 0x02020100u : last == 1 ? 0x01010100u : 0u;
-    const unsigned sel_past = (unsigned)last * 0x01010101u;
+    const EdgeRow edge = edge_row(w);
     float wk[NT];
 #pragma unroll
     for (int k = 0; k < NT; k++) wk[k] = taps[k];
@@ -532,13 +530,9 @@ __device__ __forceinline__ void blur_hv_tile(const BlurJob& J, int x0, int y0, u
         } else {
 #pragma unroll
             for (int k = 0; k < NW; k++)
-                u[k] = *(__attribute__((address_space(1))) const unsigned*)(src + min(max(xb + 4 * k, 0), wl));
+                u[k] = ((const __attribute__((address_space(1))) UnalignedWord*)(src + edge.at(xb + 4 * k)))->v;
 #pragma unroll
-            for (int k = 0; k < NW; k++) {
-                const int xw = xb + 4 * k;
-                const unsigned sel = xw < 0 ? 0u : xw < wl ? 0x03020100u : xw == wl ? sel_end : sel_past;
-                u[k] = __builtin_amdgcn_perm(u[k], u[k], sel);
-            }
+            for (int k = 0; k < NW; k++) u[k] = __builtin_amdgcn_perm(u[k], u[k], edge.sel(xb + 4 * k));
         }
         float win[PX + NT - 1];
 #pragma unroll

@@ -24,6 +24,11 @@ __device__ __forceinline__ int xcd_remap(int b, int n) {
     return x * q + min(x, r) + b / kNumXcd;
 }
 
+// A 32-bit word at any byte address.
+struct __attribute__((packed)) UnalignedWord {
+    unsigned v;
+};
+
 // One separable-blur pass over one image level (horizontal or vertical).
 struct BlurJob {
     const uint8_t* src;
@@ -122,7 +127,8 @@ void launch_blur_v(const BlurJob* d_jobs, int njobs, int total_tiles, int narrow
 // 8 rows per lane (256 x 32 tiles); only for 7, 9, 11, 13 or 15 taps.
 void launch_blur_v8(const BlurJob* d_jobs, int njobs, int total_tiles, hipStream_t s);
 // Both passes in one kernel, without the DoG epilogue (BlurJob src -> dst): odd
-// tap counts from 5 to kHvMaxTaps, the source and its pitch aligned to 4 bytes.
+// tap counts from 5 to kHvMaxTaps, the source and its pitch aligned to 4 bytes, rows
+// of at least 4 pixels or padded to them.
 // kHvTileW x kHvTileH tiles, tap counts up to kHvShortTaps or (longer) above; or
 // kHvSmallW x kHvSmallH tiles of any of them.
 void launch_blur_hv(const BlurJob* d_jobs, int njobs, int total_tiles, bool longer, hipStream_t s);

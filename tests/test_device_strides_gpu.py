@@ -51,3 +51,9 @@ def test_rows_far_apart(sigma, stride):
 @pytest.mark.parametrize("stride", [(2 << 30) + 4, (2 << 30) + 1])
 def test_strides_past_an_int(sigma, stride):
     _compare(sigma, 120, 24, stride, 1)
+
+
+@pytest.mark.parametrize("w", [33, 34, 35, 36, 61])
+def test_last_row_ends_the_buffer(w):
+    """Rows on word boundaries whose last word is not the frame's alone."""
+    _compare(1.6, w, 200, (w + 3) // 4 * 4, 1)
