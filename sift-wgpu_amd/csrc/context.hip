@@ -806,8 +806,9 @@ int Context::run(const Batch& B, RunOutputs* outs) {
 
     // --- job blob (host), uploaded to the end of the arena ---
     std::vector<char> blob;
+    constexpr size_t kBlobAlign = 128;  // a cache line
     auto blob_take = [&](size_t bytes) {
-        size_t off = round_up(blob.size(), 256);
+        size_t off = round_up(blob.size(), kBlobAlign);
         blob.resize(off + bytes);
         return off;
     };
@@ -818,12 +819,15 @@ int Context::run(const Batch& B, RunOutputs* outs) {
         Lmax = std::max(Lmax, (int)B.params[i].num_intervals + 3);
     }
     // per blur step up to 16 blur launches (four of both passes, five H forms, six V
-    // forms, the copy) and 3 Lanczos3 launches; at most 1 + maxO * Lmax steps. One
-    // image has at most three octaves in a step, with two launches each (the
-    // server's frame_device_bytes counts 15 per frame).
-    const size_t max_launches = (size_t)(1 + maxO * Lmax) * (n == 1 ? 15 : 19) + (size_t)maxO * 3 + 8;
+    // forms, the copy) and 3 Lanczos3 launches; at most 1 + maxO * Lmax steps. What
+    // their tables' padding may take decides which batches the fixed scratch accepts
+    // (and the server's frame_device_bytes counts it): a step has 15 x 256 bytes, more
+    // than 19 tables of a cache line's padding need, whatever n.
+    constexpr size_t kStepPadding = 15 * 256;
+    static_assert(19 * kBlobAlign <= kStepPadding, "the padding of a step's job tables");
+    const size_t padding = (size_t)(1 + maxO * Lmax) * kStepPadding + ((size_t)maxO * 3 + 8) * 256;
     const size_t max_jobs = (size_t)n * ((1 + (size_t)maxO * Lmax) * 2 + (size_t)maxO * 2);
-    const size_t blob_bound = max_launches * 256 + max_jobs * std::max(sizeof(BlurJob), sizeof(ResizeJob)) +
+    const size_t blob_bound = padding + max_jobs * std::max(sizeof(BlurJob), sizeof(ResizeJob)) +
                               octs.size() * sizeof(OctaveDesc) + (size_t)n * sizeof(ImageParams) +
                               (size_t)(n + 1) * sizeof(int) + 4096 +
                               (counts_in_blob ? counts_bytes : 0);
