@@ -4,12 +4,14 @@ replay of the reference's HIP backend arm.
 - oracle/_san/san_check: the oracle (test infrastructure) built with both
   sanitizers, over 1x1 to 333x45 images, every public function (CPU).
 - tests/c/arm_replay_asan: the library's host code and the replay program built
-  with both sanitizers (device code as usual). Without a GPU it runs the checks
-  that need none (parameter helpers, argument validation, drawing); with one it
+  with both sanitizers (device code as usual): the checks that need no GPU
+  (parameter helpers, argument validation, drawing), on any machine.
+- tests/c/arm_replay: the same program against the library as shipped (GPU). It
   makes the Rust arm's exact calls (sift_hip_detect_batch_color with n = 1,
   stride 0, the params struct the arm builds, for Luma8 / Rgb8 / Rgba8 / LumaA8
-  buffers) and compares each result with the grey path bit for bit.
-- tests/c/arm_replay: the same program against the library as shipped (GPU).
+  buffers) and compares each result with the grey path bit for bit. The
+  sanitizer build makes them only with SIFT_REPLAY_DEVICE=1: a run of it on a
+  GPU did not end.
 
 Leak checking is on; tests/c/lsan.supp names the ROCm runtime libraries, whose
 allocations live until the process ends.
@@ -54,7 +56,7 @@ def test_oracle_under_sanitizers():
 
 
 def test_abi_host_checks_under_sanitizers():
-    """On a machine without a GPU: the checks that need none; with one, all."""
+    """The checks that need no GPU; with one there, the program makes no others."""
     _need(REPLAY_ASAN, os.path.join(REPO, "sift-wgpu_amd"), "arm_replay")
     rc, out = _run(REPLAY_ASAN, 300)
     assert rc == 0, out[-2000:]
