@@ -60,39 +60,75 @@ __device__ __forceinline__ float mul_add_exact(float acc, float a, float b) {
     return __fadd_rn(acc, __fmul_rn(a, b));
 }
 
-// From here on v_cvt_pk_u8_f32 truncates: the wave's f32 rounding mode is set to
-// round toward zero. Every sum of `a` is complete before the switch and is read
-// only after it (volatile asm statements keep their order). No other f32
-// arithmetic may follow, but for round_even().
-template <int N>
-__device__ __forceinline__ void pin(float (&a)[N]) {
-#pragma unroll
-    for (int i = 0; i < N; i++) asm volatile("" : "+v"(a[i]));
+// Sums to bytes. v_cvt_pk_u8_f32 under round toward zero equals min((unsigned)x, 255)
+// for every f32 x >= 0 (checked for all of them up to 2^33) and places the byte, one
+// instruction where the conversion, the bound and the packing took three. The wave's
+// f32 rounding mode is switched for it and back within one asm statement: the compiler
+// does not know that other arithmetic depends on the mode, and can put none between.
+#define SH_TRUNCATE "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\ts_nop 1\n\t"
+#define SH_ROUND_EVEN "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\ts_nop 1"
+#define SH_BYTE0(d) "v_cvt_pk_u8_f32 %" #d ", %" #d ", 0, 0\n\t"
+#define SH_BYTE(d, s, k) "v_cvt_pk_u8_f32 %" #d ", %" #s ", " #k ", %" #d "\n\t"
+
+// Word k of v: the bytes of a[4 k] .. a[4 k + 3], none of them negative.
+__device__ __forceinline__ void pack_u8(const float (&a)[4], unsigned (&v)[1]) {
+    float w = a[0];
+    asm(SH_TRUNCATE SH_BYTE0(0) SH_BYTE(0, 1, 1) SH_BYTE(0, 2, 2) SH_BYTE(0, 3, 3) SH_ROUND_EVEN
+        : "+&v"(w) : "v"(a[1]), "v"(a[2]), "v"(a[3]));
+    v[0] = __float_as_uint(w);
 }
-template <int N>
-__device__ __forceinline__ void truncating(float (&a)[N]) {
-    pin(a);
-    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 3\n\ts_nop 1");
-    pin(a);
+__device__ __forceinline__ void pack_u8(const float (&a)[8], unsigned (&v)[2]) {
+    float w0 = a[0], w1 = a[4];
+    asm(SH_TRUNCATE SH_BYTE0(0) SH_BYTE0(1) SH_BYTE(0, 2, 1) SH_BYTE(1, 3, 1) SH_BYTE(0, 4, 2) SH_BYTE(1, 5, 2)
+            SH_BYTE(0, 6, 3) SH_BYTE(1, 7, 3) SH_ROUND_EVEN
+        : "+&v"(w0), "+&v"(w1) : "v"(a[1]), "v"(a[5]), "v"(a[2]), "v"(a[6]), "v"(a[3]), "v"(a[7]));
+    v[0] = __float_as_uint(w0);
+    v[1] = __float_as_uint(w1);
 }
-// Back to round to nearest even, once the conversions packed into v are done.
-template <int N>
-__device__ __forceinline__ void round_even(unsigned (&v)[N]) {
-#pragma unroll
-    for (int i = 0; i < N; i++) asm volatile("" : "+v"(v[i]));
-    asm volatile("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 0, 2), 0\n\ts_nop 1");
-#pragma unroll
-    for (int i = 0; i < N; i++) asm volatile("" : "+v"(v[i]));
+__device__ __forceinline__ void pack_u8(const float (&a)[16], unsigned (&v)[4]) {
+    float w0 = a[0], w1 = a[4], w2 = a[8], w3 = a[12];
+    asm(SH_TRUNCATE SH_BYTE0(0) SH_BYTE0(1) SH_BYTE0(2) SH_BYTE0(3)
+            SH_BYTE(0, 4, 1) SH_BYTE(1, 5, 1) SH_BYTE(2, 6, 1) SH_BYTE(3, 7, 1)
+            SH_BYTE(0, 8, 2) SH_BYTE(1, 9, 2) SH_BYTE(2, 10, 2) SH_BYTE(3, 11, 2)
+            SH_BYTE(0, 12, 3) SH_BYTE(1, 13, 3) SH_BYTE(2, 14, 3) SH_BYTE(3, 15, 3) SH_ROUND_EVEN
+        : "+&v"(w0), "+&v"(w1), "+&v"(w2), "+&v"(w3)
+        : "v"(a[1]), "v"(a[5]), "v"(a[9]), "v"(a[13]), "v"(a[2]), "v"(a[6]), "v"(a[10]), "v"(a[14]),
+          "v"(a[3]), "v"(a[7]), "v"(a[11]), "v"(a[15]));
+    v[0] = __float_as_uint(w0);
+    v[1] = __float_as_uint(w1);
+    v[2] = __float_as_uint(w2);
+    v[3] = __float_as_uint(w3);
 }
-// Four non-negative sums as bytes, after truncating(): v_cvt_pk_u8_f32 under
-// round toward zero equals min((unsigned)x, 255) for every f32 x >= 0 (checked for
-// all of them up to 2^33) and places the byte, one instruction where the
-// conversion, the bound and the packing took three.
-__device__ __forceinline__ unsigned pack_u8(float a, float b, float c, float d) {
-    unsigned v = __builtin_amdgcn_cvt_pk_u8_f32(a, 0u, 0u);
-    v = __builtin_amdgcn_cvt_pk_u8_f32(b, 1u, v);
-    v = __builtin_amdgcn_cvt_pk_u8_f32(c, 2u, v);
-    return __builtin_amdgcn_cvt_pk_u8_f32(d, 3u, v);
+// Byte 0 of v[k]: that of a[k].
+__device__ __forceinline__ void each_u8(const float (&a)[2], unsigned (&v)[2]) {
+    float w0 = a[0], w1 = a[1];
+    asm(SH_TRUNCATE SH_BYTE0(0) SH_BYTE0(1) SH_ROUND_EVEN : "+&v"(w0), "+&v"(w1));
+    v[0] = __float_as_uint(w0);
+    v[1] = __float_as_uint(w1);
+}
+__device__ __forceinline__ void each_u8(const float (&a)[4], unsigned (&v)[4]) {
+    float w0 = a[0], w1 = a[1], w2 = a[2], w3 = a[3];
+    asm(SH_TRUNCATE SH_BYTE0(0) SH_BYTE0(1) SH_BYTE0(2) SH_BYTE0(3) SH_ROUND_EVEN
+        : "+&v"(w0), "+&v"(w1), "+&v"(w2), "+&v"(w3));
+    v[0] = __float_as_uint(w0);
+    v[1] = __float_as_uint(w1);
+    v[2] = __float_as_uint(w2);
+    v[3] = __float_as_uint(w3);
+}
+// round(clamp(x, 0, 255)) of any sums, a byte each of one word (of a[0] alone): x + 0.5
+// and the conversion, both toward zero. The sum cannot reach an integer that the exact
+// one does not, and negative sums give 0 (checked for every f32 up to 2^15).
+#define SH_HALF(d) "v_add_f32 %" #d ", 0.5, %" #d "\n\t"
+__device__ __forceinline__ unsigned round_u8(const float (&a)[4]) {
+    float w = a[0], b = a[1], c = a[2], d = a[3];
+    asm(SH_TRUNCATE SH_HALF(0) SH_HALF(1) SH_HALF(2) SH_HALF(3) SH_BYTE0(0) SH_BYTE(0, 1, 1) SH_BYTE(0, 2, 2)
+            SH_BYTE(0, 3, 3) SH_ROUND_EVEN
+        : "+&v"(w), "+&v"(b), "+&v"(c), "+&v"(d));
+    return __float_as_uint(w);
+}
+__device__ __forceinline__ unsigned round_u8(float a) {
+    asm(SH_TRUNCATE SH_HALF(0) SH_BYTE0(0) SH_ROUND_EVEN : "+&v"(a));
+    return __float_as_uint(a);
 }
 
 __device__ __forceinline__ float q255(unsigned v) { return __fdiv_rn((float)v, 255.0f); }
@@ -281,11 +317,9 @@ __global__ __launch_bounds__(kThreads) void k_blur_h(const BlurJob* __restrict__
     const int x = x0 + base;
     if (x >= w) return;
     uint8_t* dst = J.dst + (size_t)y * J.dst_pitch + x;
-    truncating(acc);
     if constexpr (PX >= 8) {
         unsigned v[PX / 4];
-#pragma unroll
-        for (int k = 0; k < PX / 4; k++) v[k] = pack_u8(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]);
+        pack_u8(acc, v);
         if (x + PX <= w) {
             if constexpr (PX == 8) *(uint2*)dst = make_uint2(v[0], v[1]);
             else *(uint4*)dst = make_uint4(v[0], v[1], v[2], v[3]);
@@ -295,9 +329,11 @@ __global__ __launch_bounds__(kThreads) void k_blur_h(const BlurJob* __restrict__
         for (int q = 0; q < PX; q++)
             if (x + q < w) dst[q] = (uint8_t)(v[q / 4] >> (8 * (q & 3)));
     } else {
+        unsigned v[PX];
+        each_u8(acc, v);
 #pragma unroll
         for (int q = 0; q < PX; q++)
-            if (x + q < w) dst[q] = (uint8_t)__builtin_amdgcn_cvt_pk_u8_f32(acc[q], 0u, 0u);
+            if (x + q < w) dst[q] = (uint8_t)v[q];
     }
 }
 
@@ -338,18 +374,19 @@ __device__ __forceinline__ void store_row4(const BlurJob& J, int y, int x, unsig
     }
 }
 
-// RV rows of four sums as packed bytes; the rounding mode is as before after it
-// (the DoG epilogue divides).
+// RV rows of four sums as packed bytes, four rows at a time.
 template <int RV>
-__device__ __forceinline__ void trunc_rows(float (&acc)[RV][4], unsigned (&res)[RV]) {
+__device__ __forceinline__ void trunc_rows(const float (&acc)[RV][4], unsigned (&res)[RV]) {
 #pragma unroll
-    for (int q = 0; q < RV; q++) pin(acc[q]);
-    truncating(acc[0]);
+    for (int q = 0; q < RV; q += 4) {
+        float a[16];
+        unsigned v[4];
 #pragma unroll
-    for (int q = 1; q < RV; q++) pin(acc[q]);
+        for (int i = 0; i < 16; i++) a[i] = acc[q + i / 4][i & 3];
+        pack_u8(a, v);
 #pragma unroll
-    for (int q = 0; q < RV; q++) res[q] = pack_u8(acc[q][0], acc[q][1], acc[q][2], acc[q][3]);
-    round_even(res);
+        for (int i = 0; i < 4; i++) res[q + i] = v[i];
+    }
 }
 
 // Any tap count: a register window of RV input rows x 4 columns slides over the
@@ -547,11 +584,8 @@ __device__ __forceinline__ void blur_hv_tile(const BlurJob& J, int x0, int y0, u
         for (int k = 1; k < NT; k++)
 #pragma unroll
             for (int q = 0; q < PX; q++) acc[q] = mul_add_exact(acc[q], win[q + k], wk[k]);
-        truncating(acc);
         unsigned v[PX / 4];
-#pragma unroll
-        for (int k = 0; k < PX / 4; k++) v[k] = pack_u8(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]);
-        round_even(v);
+        pack_u8(acc, v);
         uint8_t* to = rows + row * TW + xl;
         if constexpr (PX == 16) *(uint4*)to = make_uint4(v[0], v[1], v[2], v[3]);
         else if constexpr (PX == 8) *(uint2*)to = make_uint2(v[0], v[1]);
@@ -574,11 +608,11 @@ __device__ __forceinline__ void blur_hv_tile(const BlurJob& J, int x0, int y0, u
                 acc[q] = k == 0 ? __fmul_rn(p, wk[0]) : mul_add_exact(acc[q], p, wk[k]);
             }
         }
-        truncating(acc);
+        unsigned v[RV];
+        each_u8(acc, v);
 #pragma unroll
         for (int q = 0; q < RV; q++)
-            if (yb + q < h)
-                J.dst[(size_t)(yb + q) * J.dst_pitch + x] = (uint8_t)__builtin_amdgcn_cvt_pk_u8_f32(acc[q], 0u, 0u);
+            if (yb + q < h) J.dst[(size_t)(yb + q) * J.dst_pitch + x] = (uint8_t)v[q];
         return;
     }
     const int x = x0 + 4 * lane;
@@ -1146,9 +1180,7 @@ __global__ __launch_bounds__(kThreads) void k_resize_h(const ResizeJob* __restri
 // Both passes of the octave step in one kernel: the vertical pass of a tile's
 // rows, over the input columns its horizontal windows need, goes to LDS as f32 (the
 // same t += p * w in window order as k_resize_v) and the horizontal pass reads it
-// there. The rounding is round(clamp(t, 0, 255)) as t + 0.5 and the conversion,
-// both under round toward zero: the sum cannot reach an integer that the exact one
-// does not, and negative sums give 0 (checked for every f32 up to 2^15).
+// there; round_u8 makes the bytes.
 // k_resize_tall: tiles of kResizeTallW x kResizeTallH outputs, four rows per wave. A
 // wave's lanes hold the tile's input column quads (120 outputs need at most 64) and
 // stream the rows its four windows share once, converting each texel once instead
@@ -1262,16 +1294,11 @@ __global__ __launch_bounds__(kThreads) void k_resize_tall(const ResizeJob* __res
 #pragma unroll
             for (int q = 0; q < 4; q++) h[q] = mul_add_exact(h[q], vt[wave][q][at + i], wv[i]);
         }
-        truncating(h);
-        unsigned v[1];
-#pragma unroll
-        for (int q = 0; q < 4; q++) h[q] = __fadd_rn(h[q], 0.5f);
-        v[0] = pack_u8(h[0], h[1], h[2], h[3]);
-        round_even(v);
+        const unsigned v = round_u8(h);
 #pragma unroll
         for (int q = 0; q < 4; q++)
             if (y0 + q < J.out_h)
-                J.dst[(size_t)(y0 + q) * J.dst_pitch + ox0 + c] = (uint8_t)(v[0] >> (8 * q));
+                J.dst[(size_t)(y0 + q) * J.dst_pitch + ox0 + c] = (uint8_t)(v >> (8 * q));
     }
 }
 
@@ -1327,14 +1354,12 @@ __global__ __launch_bounds__(kThreads) void k_resize_small(const ResizeJob* __re
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const float* row = &vt[wave][l - lo4];
-    float h[1] = {0.0f};
+    float h = 0.0f;
 #pragma unroll
     for (int i = 0; i < kResizeMaxTaps; i++)
-        if (i < hn) h[0] = mul_add_exact(h[0], row[i], wv[i]);
-    truncating(h);
-    h[0] = __fadd_rn(h[0], 0.5f);  // truncated, as the conversion is: rounds half up, exactly
-    if (ox < J.out_w)
-        J.dst[(size_t)oy * J.dst_pitch + ox] = (uint8_t)__builtin_amdgcn_cvt_pk_u8_f32(h[0], 0u, 0u);
+        if (i < hn) h = mul_add_exact(h, row[i], wv[i]);
+    const unsigned v = round_u8(h);
+    if (ox < J.out_w) J.dst[(size_t)oy * J.dst_pitch + ox] = (uint8_t)v;
 }
 
 }  // namespace
