@@ -494,9 +494,13 @@ std::pair<int, int> blur_heuristic(int w, int h, int ntaps, int npad) {
 }
 
 // A step whose octave steps read at least this many pixels takes k_resize_tall,
-// else k_resize_small (one level of 1920 x 1080: 11.7 against 12.7 us; two of
-// 1023 x 767, 1.6 Mpixel: 14.7 against 11.3 us).
-constexpr double kResizeTallPixels = 2.05e6;
+// else k_resize_small. Launches in a row, tall against small: one level of 1600 x 900
+// (1.44 Mpixel) 9.0 / 8.3 us, 1680 x 1050 (1.76) 9.0 / 10.0, 1792 x 1008 (1.81) 9.1 / 9.3,
+// 1920 x 1080 9.5 / 10.1, 2560 x 1440 9.9 / 15.7; two of 1023 x 767 (1.57) 12.3 / 9.0, two
+// of 1280 x 720 (1.84) 10.0 / 9.8; 5, 6 and 8 of 640 x 480 (1.54, 1.84, 2.46) 9.4 / 8.6,
+// 10.1 / 10.1, 10.1 / 11.7. Levels that fill either's tiles badly cross elsewhere (64 of
+// 160 x 120, 1.23: 9.2 / 10.2; 64 of 240 x 135, 2.07: 13.2 / 11.2).
+constexpr double kResizeTallPixels = 1.7e6;
 // Whether an octave step's windows fit a kernel of both passes with tiles of tw
 // output columns over `span` input columns.
 bool resize_fits(const LanczosRef& LH, const LanczosRef& LV, int tw, int span) {
@@ -535,11 +539,18 @@ void blur_hv_tiles(BlurJob& J, bool large) {
 }
 
 // A step's blurs of more taps go to k_blur_deep while its tiles hold at most this
-// many products together (64 levels of 80 x 60, 101 taps, 62 M: 16.0 against 22.1 us
-// of the best pair; one of 960 x 540, 41 taps, 54 M: 17.0 against 16.7; 64 of
-// 120 x 67, 199 taps, 205 M: 36.5 against 33.7) and each one at most this many
-// (240 x 135, 199 taps, 0.43 M: 18.8 against 19.6; 120 x 67, 395 taps, 0.42 M: 22.6
-// against 21.4).
+// many products together and each one at most that many. No such line parts the steps
+// of one shape cleanly. Launches in a row, deep against the best pair: while the tiles
+// fit the GPU at once (512, or 256 of more than 80 KB) deep wins at 31 M (one level of
+// 640 x 480, 41 taps: 8.5 / 9.3 us) as at 102 M (32 of 120 x 67, 199 taps: 17.7 / 18.7);
+// past that it wins at 62 M where tiles make no row twice (64 of 80 x 60, 101 taps:
+// 13.2 / 16.6) and loses at 54 M where they do (one of 960 x 540, 41 taps: 13.9 / 10.7);
+// at 205 M it loses (64 of 120 x 67, 199 taps: 30.7 / 27.6). Tiles cross at about 0.27 M
+// (240 x 135, 159 and 199 taps, 0.26 and 0.32 M: 12.7 / 13.5 and 15.2 / 14.7; 120 x 67, 255
+// and 395 taps, 0.27 and 0.42 M: 14.2 / 13.4 and 20.0 / 17.0). But the steps of frames of
+// many sizes are one deep launch, and a blur sent to the pair adds the launches of its
+// two forms: with limits by what fits at once, and tiles of 0.27 M, 12 frames of mixed
+// odd sizes took 1420 us instead of 1390, 20 served ones 3500 instead of 3400.
 constexpr double kDeepStepWork = 60e6, kDeepTileWork = 0.4e6;
 bool blur_deep_valid(unsigned src_pitch, int h, int ntaps) {
     return ntaps > kHvMaxTaps && deep_tile_work(h, ntaps) <= kDeepTileWork &&
