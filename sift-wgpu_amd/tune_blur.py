@@ -13,6 +13,11 @@ the entry names the built-in form, so the table never trades a measured loss
 for noise. Every form computes the same exact sums, so any choice gives the
 same pyramid (tests/test_tune_gpu.py checks each form against the oracle).
 
+The forms are those of the two separate passes. Detection blurs levels of 5 to 33
+taps, and small levels of more, with one launch for both passes, which no entry
+governs; for those levels the table serves sift_hip_pyramid with a DoG output and the
+first blur of device frames whose rows are not word aligned.
+
     python tune_blur.py [--out blur_tune.json] [--reps 15] [--margin 0.03]
 """
 import argparse
