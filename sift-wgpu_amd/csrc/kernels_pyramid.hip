@@ -115,16 +115,19 @@ __device__ __forceinline__ void each_u8(const float (&a)[4], unsigned (&v)[4]) {
     v[2] = __float_as_uint(w2);
     v[3] = __float_as_uint(w3);
 }
-// round(clamp(x, 0, 255)) of any sums, a byte each of one word (of a[0] alone): x + 0.5
-// and the conversion, both toward zero. The sum cannot reach an integer that the exact
-// one does not, and negative sums give 0 (checked for every f32 up to 2^15).
+// Byte 0 of v[k]: round(clamp(a[k], 0, 255)) of any sum, as a[k] + 0.5 and the
+// conversion, both toward zero. The sum cannot reach an integer that the exact one does
+// not, and negative sums give 0 (checked for every f32 up to 2^15).
 #define SH_HALF(d) "v_add_f32 %" #d ", 0.5, %" #d "\n\t"
-__device__ __forceinline__ unsigned round_u8(const float (&a)[4]) {
-    float w = a[0], b = a[1], c = a[2], d = a[3];
-    asm(SH_TRUNCATE SH_HALF(0) SH_HALF(1) SH_HALF(2) SH_HALF(3) SH_BYTE0(0) SH_BYTE(0, 1, 1) SH_BYTE(0, 2, 2)
-            SH_BYTE(0, 3, 3) SH_ROUND_EVEN
-        : "+&v"(w), "+&v"(b), "+&v"(c), "+&v"(d));
-    return __float_as_uint(w);
+__device__ __forceinline__ void round_u8(const float (&a)[4], unsigned (&v)[4]) {
+    float w0 = a[0], w1 = a[1], w2 = a[2], w3 = a[3];
+    asm(SH_TRUNCATE SH_HALF(0) SH_HALF(1) SH_HALF(2) SH_HALF(3) SH_BYTE0(0) SH_BYTE0(1) SH_BYTE0(2) SH_BYTE0(3)
+            SH_ROUND_EVEN
+        : "+&v"(w0), "+&v"(w1), "+&v"(w2), "+&v"(w3));
+    v[0] = __float_as_uint(w0);
+    v[1] = __float_as_uint(w1);
+    v[2] = __float_as_uint(w2);
+    v[3] = __float_as_uint(w3);
 }
 __device__ __forceinline__ unsigned round_u8(float a) {
     asm(SH_TRUNCATE SH_HALF(0) SH_BYTE0(0) SH_ROUND_EVEN : "+&v"(a));
@@ -1279,6 +1282,9 @@ __global__ __launch_bounds__(kThreads) void k_resize_tall(const ResizeJob* __res
 #pragma unroll
     for (int q = 0; q < 4; q++) *(float4*)&vt[wave][q][4 * lane] = make_float4(s[q][0], s[q][1], s[q][2], s[q][3]);
     __syncthreads();
+    // (read once: after a store the compiler would read them again, and wait for them)
+    uint8_t* const dst = J.dst + (size_t)y0 * J.dst_pitch + ox0;
+    const int dst_pitch = J.dst_pitch, rows = J.out_h - y0;
     for (int c0 = 0; c0 < cols; c0 += 60) {
         const int c = c0 + lane;
         if (lane >= 60 || c >= cols) continue;
@@ -1294,11 +1300,11 @@ __global__ __launch_bounds__(kThreads) void k_resize_tall(const ResizeJob* __res
 #pragma unroll
             for (int q = 0; q < 4; q++) h[q] = mul_add_exact(h[q], vt[wave][q][at + i], wv[i]);
         }
-        const unsigned v = round_u8(h);
+        unsigned v[4];
+        round_u8(h, v);
 #pragma unroll
         for (int q = 0; q < 4; q++)
-            if (y0 + q < J.out_h)
-                J.dst[(size_t)(y0 + q) * J.dst_pitch + ox0 + c] = (uint8_t)(v >> (8 * q));
+            if (q < rows) dst[(size_t)q * dst_pitch + c] = (uint8_t)v[q];
     }
 }
 
